@@ -25,6 +25,7 @@
 #include <cmath>
 #include <cstring>
 #include <random>
+#include <type_traits>
 
 #include "fopis_internal.hpp"
 
@@ -67,10 +68,11 @@ __device__ inline int xcd_block(int p, int n) {
 enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_PHI = 2 };
 
 struct ConvArgs {
-  const uint16_t* x;     // input [voxel][cin] (at half resolution when UP)
+  const uint16_t* x;     // input [voxel][cin] (at half resolution when up)
   const uint16_t* w;     // packed weights [nqp][cout][8]
   const float* bias;     // [cout]
   const uint16_t* add;   // [voxel][cout] added before the activation, or null
+  const uint16_t* gate;  // [voxel][cout]: the result is kept where this is > 0 (a ReLU's backward), or null
   uint16_t* y;           // EPI_BF16: [voxel][cout]
   float* y32;            // EPI_F32: channel 0, [voxel]
   double* phi;           // EPI_PHI: glue-layout potential
@@ -80,109 +82,239 @@ struct ConvArgs {
   int64_t gsx, gsy, goff;
   int vn0, vn1, vn2;     // EPI_PHI: voxels that map to interior nodes
   int n0, n1, n2;        // output grid
-  int cin, cout, nq, nqp;
+  int cin, cout;
+  int up;                // 1: x is at half resolution (nearest-neighbour upsampling on read)
+  int nbrick;            // output bricks
   int relu;
 };
 
-// Output bricks of kBI x kBJ x 16 voxels per workgroup: the brick's input
-// with a one-voxel halo (kBI+2, kBJ+2, 18) is staged once in LDS, channel rows
-// padded by 8 elements so that the 16 lanes of a fragment read hit distinct
-// banks; each of the 4 waves then owns kBI*kBJ/4 rows of 16 voxels (its M
-// tiles) and reads its A fragments from LDS, B fragments (weights) from
-// global memory through the caches.
+// Output bricks of kBI x kBJ x 16 voxels: the brick's input with a one-voxel
+// halo (kBI+2, kBJ+2, 18) is staged once in LDS, channel rows padded by 8
+// elements so that the 16 lanes of a fragment read hit distinct banks; each
+// of the 4 waves then owns kBI*kBJ/4 rows of 16 voxels (its M tiles) and reads
+// its A fragments from LDS, B fragments (weights) from global memory through
+// the caches.
 constexpr int kBI = 4, kBJ = 4, kBK = 16;
 constexpr int kHI = kBI + 2, kHJ = kBJ + 2, kHK = kBK + 2;
 constexpr int kHalo = kHI * kHJ * kHK;
 constexpr int kRowsPerWave = kBI * kBJ / 4;
+static_assert(kRowsPerWave == kBJ, "wave w owns the brick's plane w");
+static_assert(kHI + kHJ + kHK <= 32, "one bit per halo plane");
 
-inline size_t conv_lds_bytes(int cin) { return (size_t)kHalo * (cin + 8) * sizeof(uint16_t); }
+constexpr size_t conv_lds_bytes(int cin) { return (size_t)kHalo * (cin + 8) * sizeof(uint16_t); }
 
-template <int NT, int EPI, bool UP>
-__global__ __launch_bounds__(256) void k_conv(ConvArgs A) {
+// LDS element offset, from a row's own voxel, of the 8-channel chunk q of the
+// K axis (q = tap * cin / 8 + channel / 8); chunks past the last tap sit at 0.
+template <int CIN>
+constexpr int chunk_off(int q) {
+  constexpr int cpt = CIN / 8;
+  if (q >= 27 * cpt) return 0;
+  const int tap = q / cpt;
+  return ((tap / 9 * kHJ + (tap / 3) % 3) * kHK + tap % 3) * (CIN + 8) + (q % cpt) * 8;
+}
+
+template <int MASK>
+__device__ inline float quad_swap(float v) {  // the value of lane ^ MASK, MASK 1 or 2
+  constexpr int ctrl = MASK == 1 ? 0xB1 : 0x4E;
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, true));
+}
+
+// Two floats rounded to BF16 (nearest even), the first in the low half.
+__device__ inline uint32_t pack_bf16(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
+}
+
+// NT tiles of 16 output channels per workgroup, tiles blockIdx.y * NT on.
+// The input channel count is a template argument, so that the K loop unrolls
+// and every fragment's LDS address is a lane base plus an immediate: with the
+// count at run time a K step spent ~80 vector instructions (a division by
+// cin/8 among them) on the addresses of four 16-cycle MFMAs, and those
+// bounded the kernel. A workgroup walks a run of neighbouring bricks: each
+// thread's voxels sit at the same offsets from every brick's corner, computed
+// once, and one bit per halo plane tells which of them lie outside the grid;
+// the next brick's voxels are loaded while the current brick is multiplied;
+// with one tile the weights stay in registers (all of their loads are then in
+// flight before the first brick arrives, which is what a small grid waits
+// for). The result leaves through a 4x4 exchange between the four lanes that hold
+// neighbouring channels, so that a lane stores (and loads the addend and the
+// gate as) four channels of one voxel, 8 bytes, instead of four times 2 bytes.
+// Bound by LDS reads (one per product with 16 output channels) and the
+// latency of a brick's stage-multiply-store chain. 16 -> 16 channels at 128^3:
+// 115 -> 58 us (2.3 TB/s, 0.5 PFLOP/s), 32 -> 16 upsampled: 222 -> 117 us,
+// 64 -> 64 at 16^3: 38 -> 15 us.
+template <int CIN, int NT, int EPI>
+__global__ __launch_bounds__(256, CIN >= 56 || (NT == 1 && CIN >= 40) ? 1 : (CIN >= 48 || NT > 2 || (NT == 1 && CIN >= 24) ? 2 : 3)) void k_conv(ConvArgs A) {
   extern __shared__ __attribute__((aligned(16))) uint16_t xs[];
   constexpr int MT = kRowsPerWave;
+  constexpr int CPT = CIN / 8, NQ = 27 * CPT, NS = (NQ + 3) / 4, LS = CIN + 8;
+  constexpr bool kWReg = NT == 1;
+  const int cout = A.cout, ct0 = blockIdx.y * NT * 16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int row = lane & 15, grp = lane >> 4;
   const int nb1 = (A.n1 + kBJ - 1) / kBJ, nb2 = (A.n2 + kBK - 1) / kBK;
-  const int blk = xcd_block(blockIdx.x, gridDim.x);
-  const int b2 = blk % nb2, b1 = (blk / nb2) % nb1, b0 = blk / (nb2 * nb1);
-  const int i0 = b0 * kBI, j0 = b1 * kBJ, k0 = b2 * kBK;
-  const int cpt = A.cin >> 3;
-  const int ls = A.cin + 8;  // LDS elements per staged voxel
-  const int in1 = UP ? (A.n1 >> 1) : A.n1, in2 = UP ? (A.n2 >> 1) : A.n2;
+  const int in1 = A.n1 >> A.up, in2 = A.n2 >> A.up;
+  const int per = (A.nbrick + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int first = xcd_block(blockIdx.x, gridDim.x) * per, last = min(first + per, A.nbrick);
+  if (first >= last) return;
 
-  // stage the input brick with its halo (zeros outside the grid)
-  for (int e = threadIdx.x; e < kHalo * cpt; e += 256) {
-    const int ch = e % cpt, hv = e / cpt;
+  // the thread's units (16 bytes of one halo voxel): offset from the brick's
+  // corner in x, and one bit per halo plane along each axis
+  constexpr int kUnits = kHalo * CPT, IT = (kUnits + 255) / 256;
+  int rel[IT];
+  uint32_t planes[IT];
+#pragma unroll
+  for (int u = 0; u < IT; ++u) {
+    const int e = threadIdx.x + u * 256;
+    const int ch = e % CPT, hv = e / CPT;
     const int hk = hv % kHK, hj = (hv / kHK) % kHJ, hi = hv / (kHK * kHJ);
-    int gi = i0 - 1 + hi, gj = j0 - 1 + hj, gk = k0 - 1 + hk;
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (gi >= 0 && gi < A.n0 && gj >= 0 && gj < A.n1 && gk >= 0 && gk < A.n2) {
-      if (UP) {
-        gi >>= 1;
-        gj >>= 1;
-        gk >>= 1;
+    // (bricks start at even voxels, so the halving of a coordinate splits)
+    rel[u] = ((((hi - 1) >> A.up) * in1 + ((hj - 1) >> A.up)) * in2 + ((hk - 1) >> A.up)) * CIN + ch * 8;
+    planes[u] = e < kUnits ? (1u << hi) | (1u << (kHI + hj)) | (1u << (kHI + kHJ + hk)) : 0xffffffffu;
+  }
+  u32x4 v[IT];
+  auto fetch = [&](int blk) {
+    const int b2 = blk % nb2, b1 = (blk / nb2) % nb1, b0 = blk / (nb2 * nb1);
+    const int i0 = b0 * kBI, j0 = b1 * kBJ, k0 = b2 * kBK;
+    // halo planes outside the grid: below the first voxel, from the last one on
+    auto off = [](int o, int n, int h) -> uint32_t {
+      const int live = min(h, n - o + 1);  // planes 1 .. live - 1 (and 0 when o > 0) are inside
+      return (o > 0 ? 0u : 1u) | (((1u << h) - 1u) & ~((1u << live) - 1u));
+    };
+    const uint32_t out = off(i0, A.n0, kHI) | (off(j0, A.n1, kHJ) << kHI) | (off(k0, A.n2, kHK) << (kHI + kHJ));
+    const uint16_t* base = A.x + (((int64_t)(i0 >> A.up) * in1 + (j0 >> A.up)) * in2 + (k0 >> A.up)) * CIN;
+#pragma unroll
+    for (int u = 0; u < IT; ++u) {
+      v[u] = (u32x4){0u, 0u, 0u, 0u};
+      if (!(planes[u] & (out | (1u << 31)))) v[u] = *reinterpret_cast<const u32x4*>(base + rel[u]);
+    }
+  };
+  fetch(first);
+
+  bf16x8 wreg[kWReg ? NS : 1][NT];
+  if constexpr (kWReg) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)  // chunk 4s + grp, output channel ct0 + nt * 16 + row
+        wreg[s][nt] = load8(A.w + (int64_t)(s * 4 + grp) * cout * 8 + (ct0 + nt * 16 + row) * 8);
+  }
+  float bias[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) bias[nt] = A.bias[ct0 + nt * 16 + row];
+
+  for (int blk = first; blk < last; ++blk) {
+    const int b2 = blk % nb2, b1 = (blk / nb2) % nb1, b0 = blk / (nb2 * nb1);
+    const int i0 = b0 * kBI, j0 = b1 * kBJ, k0 = b2 * kBK;
+    if (blk != first) __syncthreads();  // the last brick's fragments have been read
+#pragma unroll
+    for (int u = 0; u < IT; ++u) {
+      const int e = threadIdx.x + u * 256;
+      if ((u + 1) * 256 <= kUnits || e < kUnits)
+        *reinterpret_cast<u32x4*>(xs + (e / CPT) * LS + (e % CPT) * 8) = v[u];
+    }
+    __syncthreads();
+    if (blk + 1 < last) fetch(blk + 1);
+
+    f32x4 acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    // (the weights are read again for each brick: without this the compiler
+    // moves all of their loads out of the brick loop, into scratch memory)
+    int wo = (grp * cout + ct0 + row) * 8;
+    asm volatile("" : "+v"(wo));
+    const uint16_t* xb = xs + (wave * kHJ * kHK + row) * LS;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      bf16x8 bfr[NT];
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) bfr[nt] = kWReg ? wreg[kWReg ? s : 0][nt] : load8(A.w + s * 32 * cout + nt * 128 + wo);
+      // the four lane groups' chunks: one lane offset per pattern of
+      // differences (few of them), the rest an immediate
+      const int o0 = chunk_off<CIN>(4 * s);
+      const int d1 = chunk_off<CIN>(4 * s + 1) - o0, d2 = chunk_off<CIN>(4 * s + 2) - o0,
+                d3 = chunk_off<CIN>(4 * s + 3) - o0;
+      const int ld = grp == 0 ? 0 : (grp == 1 ? d1 : (grp == 2 ? d2 : d3));
+      const bool qok = 4 * s + 3 < NQ || 4 * s + grp < NQ;  // chunks past the last tap (K padding) are zeroed
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const u32x4 raw = *reinterpret_cast<const u32x4*>(xb + ld + (o0 + mt * kHK * LS));
+        const bf16x8 af = qok ? __builtin_bit_cast(bf16x8, raw) : zero8();
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfr[nt], acc[mt][nt], 0, 0, 0);
       }
-      v = *reinterpret_cast<const u32x4*>(A.x + (((size_t)gi * in1 + gj) * in2 + gk) * A.cin + ch * 8);
     }
-    *reinterpret_cast<u32x4*>(xs + hv * ls + ch * 8) = v;
-  }
-  __syncthreads();
 
-  f32x4 acc[MT][NT];
+    // D layout: lane holds output channel ct0 + nt*16 + row for voxels k0 + 4*grp + r of the row
+    const int i = i0 + wave;
+    if (i < A.n0) {
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+      for (int mt = 0; mt < MT; ++mt) {
+        const int j = j0 + mt;
+        if (j >= A.n1) continue;
+        const int64_t vrow = ((int64_t)i * A.n1 + j) * A.n2;
+        if constexpr (EPI == EPI_BF16) {
+          const int q = row & 3, k = k0 + 4 * grp + q;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  const int nsteps = A.nqp >> 2;
-  for (int s = 0; s < nsteps; ++s) {
-    const int q = 4 * s + grp;
-    bf16x8 bfr[NT];
+          for (int nt = 0; nt < NT; ++nt) {
+            float f[4];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) bfr[nt] = load8(A.w + ((size_t)q * A.cout + nt * 16 + row) * 8);
-    // chunks past the last tap (K padding) read chunk 0 of tap 0 and are zeroed
-    const bool qok = q < A.nq;
-    const int tap = qok ? q / cpt : 0;
-    const int c0 = qok ? (q - tap * cpt) * 8 : 0;
-    const int di = tap / 9, dj = (tap / 3) % 3, dk = tap % 3;  // halo-relative offsets 0..2
+            for (int r = 0; r < 4; ++r) f[r] = acc[mt][nt][r] + bias[nt];
+            // lane q of a quad ends with voxel 4*grp + q, channels 4*(row/4) .. + 3
+            float t;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int r = wave * MT + mt;
-      const int hv = ((r / kBJ + di) * kHJ + (r % kBJ + dj)) * kHK + row + dk;
-      bf16x8 af = qok ? __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(xs + hv * ls + c0)) : zero8();
+            for (int r = 0; r < 4; r += 2) {
+              t = quad_swap<1>((q & 1) ? f[r] : f[r + 1]);
+              f[r] = (q & 1) ? t : f[r];
+              f[r + 1] = (q & 1) ? f[r + 1] : t;
+            }
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfr[nt], acc[mt][nt], 0, 0, 0);
-    }
-  }
-
-  // D layout: lane holds output channel nt*16 + row for voxels k0 + 4*grp + r of the row
+            for (int r = 0; r < 2; ++r) {
+              t = quad_swap<2>((q & 2) ? f[r] : f[r + 2]);
+              f[r] = (q & 2) ? t : f[r];
+              f[r + 2] = (q & 2) ? f[r + 2] : t;
+            }
+            if (k < A.n2) {
+              const int64_t at = (vrow + k) * cout + ct0 + nt * 16 + (row & 12);
+              if (A.add) {
+                const uint2 ad = *reinterpret_cast<const uint2*>(A.add + at);
+                f[0] += bf2f((uint16_t)ad.x);
+                f[1] += bf2f((uint16_t)(ad.x >> 16));
+                f[2] += bf2f((uint16_t)ad.y);
+                f[3] += bf2f((uint16_t)(ad.y >> 16));
+              }
+              if (A.relu)
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int rr = wave * MT + mt;
-    const int i = i0 + rr / kBJ, j = j0 + rr % kBJ;
-    if (i >= A.n0 || j >= A.n1) continue;
+                for (int r = 0; r < 4; ++r) f[r] = fmaxf(f[r], 0.f);
+              uint2 o = make_uint2(pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3]));
+              if (A.gate) {
+                const uint2 gt = *reinterpret_cast<const uint2*>(A.gate + at);
+                if (!(bf2f((uint16_t)gt.x) > 0.f)) o.x &= 0xffff0000u;
+                if (!(bf2f((uint16_t)(gt.x >> 16)) > 0.f)) o.x &= 0xffffu;
+                if (!(bf2f((uint16_t)gt.y) > 0.f)) o.y &= 0xffff0000u;
+                if (!(bf2f((uint16_t)(gt.y >> 16)) > 0.f)) o.y &= 0xffffu;
+              }
+              *reinterpret_cast<uint2*>(A.y + at) = o;
+            }
+          }
+        } else if (row == 0) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const int co = nt * 16 + row;
-      if (EPI != EPI_BF16 && co != 0) continue;
-      const float bco = A.bias[co];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int k = k0 + 4 * grp + r;
-        if (k >= A.n2) continue;
-        const int64_t v = ((int64_t)i * A.n1 + j) * A.n2 + k;
-        float val = acc[mt][nt][r] + bco;
-        if (EPI == EPI_BF16) {
-          if (A.add) val += bf2f(A.add[v * A.cout + co]);
-          if (A.relu) val = fmaxf(val, 0.f);
-          A.y[v * A.cout + co] = f2bf(val);
-        } else if (EPI == EPI_F32) {
-          A.y32[v] = val;
-        } else if (i < A.vn0 && j < A.vn1 && k < A.vn2) {
-          double* p = A.phi + A.goff + i * A.gsx + j * A.gsy + k;
-          *p = (A.phi_add ? *p : 0.0) + (double)val * A.scal[0] * A.phi_k;
+          for (int r = 0; r < 4; ++r) {
+            const int k = k0 + 4 * grp + r;
+            if (k >= A.n2) continue;
+            const float val = acc[mt][0][r] + bias[0];
+            if constexpr (EPI == EPI_F32) {
+              A.y32[vrow + k] = val;
+            } else if (i < A.vn0 && j < A.vn1 && k < A.vn2) {
+              double* p = A.phi + A.goff + i * A.gsx + j * A.gsy + k;
+              *p = (A.phi_add ? *p : 0.0) + (double)val * A.scal[0] * A.phi_k;
+            }
+          }
         }
       }
     }
@@ -191,78 +323,183 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs A) {
 
 // ---------------------------------------------------------------- weight gradient
 
+// dW[tap][ci][co] = sum over voxels v of x[v + tap][ci] g[v][co], and the bias
+// gradient sum g[v][co]: products whose contraction runs over the voxels, so
+// an MFMA operand wants eight neighbouring voxels of one channel where the
+// arrays hold neighbouring channels of one voxel. A workgroup stages a brick
+// of BI x BJ x 32 voxels of g, and of x with its halo, into LDS with each
+// 8-voxel x 8-channel block transposed in registers (32 byte permutes), as
+// rows [channel][voxel]. A lane then reads its fragment for the left tap of a
+// row as 16 bytes plus the next dword, and the centre and right taps are the
+// same registers shifted by one and two voxels. Each x row meets up to nine g
+// rows (held in registers), 27 products per row pair of tiles: 27 products
+// cost 3 to 7 LDS reads. The four waves take PI x PO tiles of 16 x 16
+// channels; where the layer has fewer tiles they split the brick's rows
+// (kSub) and add their sums in LDS. The bias gradient is one more product,
+// with ones. Partials of a launch's workgroups go to `part`, and
+// k_wgrad_reduce adds them in workgroup order.
+// Bound by staging: at 64^3 a workgroup has two bricks of 216 to 432 products
+// per wave. The 15 layers of a 64^3 training pair: 2.29 -> 0.20 ms (with 2-byte
+// gathers, one per voxel, tap and channel), their bias sums 1.00 ms -> none.
+constexpr int kWTile = 27 * 256 + 16;  // floats of one channel tile's partial: the taps, then the bias gradient
+constexpr int kWRow = 40;              // LDS elements of one channel's row: 34 voxels, padded to spread the banks
+
 struct WgradArgs {
   const uint16_t* x;  // layer input [voxel][cin] (half resolution when UP)
   const uint16_t* g;  // output gradient after the activation [voxel][cout]
-  float* part;        // [pair][chunk][27][16][16]
+  float* part;        // [pair][chunk][kWTile]
   int n0, n1, n2;     // output grid
-  int cin, cout, nco;  // nco = cout / 16 tiles
-  int64_t nsteps;      // 32-voxel K steps
+  int cin, cout, nci, nco;  // nci, nco: tiles of 16 channels
+  int nbrick;
 };
 
-constexpr int kWTile = 27 * 256;
+template <int PI, int PO>
+struct WgradShape {
+  static constexpr int kSub = 4 / (PI * PO);       // waves sharing a tile pair
+  static constexpr int RI = 2, RJ = kSub == 1 ? 4 : 2;  // rows of one wave
+  static constexpr int SI = kSub == 4 ? 2 : 1, SJ = kSub / SI;
+  static constexpr int BI = RI * SI, BJ = RJ * SJ;  // rows of the brick
+  static constexpr int kXRows = (BI + 2) * (BJ + 2), kGRows = BI * BJ;
+  static constexpr int kXElems = kXRows * PI * 16 * kWRow, kGElems = kGRows * PO * 16 * kWRow;
+  static constexpr size_t kStage = (size_t)(kXElems + kGElems) * sizeof(uint16_t);
+  static constexpr size_t kSum = kSub > 1 ? (size_t)PI * PO * kWTile * sizeof(float) : 0;
+  static constexpr size_t kLds = kStage > kSum ? kStage : kSum;
+  static_assert(kLds <= 81920, "two workgroups per compute unit");
+};
 
-template <bool UP>
-__global__ __launch_bounds__(256) void k_wgrad(WgradArgs A) {
-  __shared__ float red[kWTile];
+// Eight voxels of eight channels each into eight channels of eight voxels.
+__device__ inline void transpose8(const u32x4 (&v)[8], u32x4 (&t)[8]) {
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+      t[c][h] = __builtin_amdgcn_perm(v[2 * h + 1][c >> 1], v[2 * h][c >> 1], (c & 1) ? 0x07060302u : 0x05040100u);
+}
+
+template <int PI, int PO, bool UP>
+__global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs A) {
+  using W = WgradShape<PI, PO>;
+  extern __shared__ __attribute__((aligned(16))) uint16_t ws[];
+  uint16_t* xs = ws;
+  uint16_t* gs = ws + W::kXElems;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int row = lane & 15, grp = lane >> 4;
-  const int pair = blockIdx.y;
-  const int cit = pair / A.nco, cot = pair % A.nco;
-  const int ci = cit * 16 + row, co = cot * 16 + row;
-  const bool ciok = ci < A.cin;
-  const int64_t nvox = (int64_t)A.n0 * A.n1 * A.n2;
+  const int ngo = (A.nco + PO - 1) / PO;
+  const int ci0 = (blockIdx.y / ngo) * PI, co0 = (blockIdx.y % ngo) * PO;  // the group's first tiles
+  const int sub = wave / (PI * PO), pi = (wave % (PI * PO)) / PO, po = wave % PO;
+  const int si = sub / W::SJ, sj = sub % W::SJ;
+  const bool live = ci0 + pi < A.nci && co0 + po < A.nco;
+  const int nb1 = (A.n1 + W::BJ - 1) / W::BJ, nb2 = (A.n2 + 31) / 32;
   const int in1 = UP ? (A.n1 >> 1) : A.n1, in2 = UP ? (A.n2 >> 1) : A.n2;
-  f32x4 acc[27];
+  f32x4 acc[27], accb = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int t = 0; t < 27; ++t) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
 
-  for (int64_t s = (int64_t)blockIdx.x * 4 + wave; s < A.nsteps; s += (int64_t)gridDim.x * 4) {
-    const int64_t vb = s * 32 + grp * 8;
-    int vi[8], vj[8], vk[8];
-    bool vin[8];
-    uint16_t gb[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int64_t v = vb + j;
-      vin[j] = v < nvox;
-      vk[j] = (int)(v % A.n2);
-      vj[j] = (int)((v / A.n2) % A.n1);
-      vi[j] = (int)(v / ((int64_t)A.n1 * A.n2));
-      gb[j] = vin[j] ? A.g[v * A.cout + co] : (uint16_t)0;
-    }
-    u32x4 braw;
-#pragma unroll
-    for (int h = 0; h < 4; ++h) braw[h] = (uint32_t)gb[2 * h] | ((uint32_t)gb[2 * h + 1] << 16);
-    const bf16x8 bfr = __builtin_bit_cast(bf16x8, braw);
-#pragma unroll
-    for (int t = 0; t < 27; ++t) {
-      const int di = t / 9 - 1, dj = (t / 3) % 3 - 1, dk = t % 3 - 1;
-      uint16_t xa[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        int ii = vi[j] + di, jj = vj[j] + dj, kk = vk[j] + dk;
-        const bool ok = ciok && vin[j] && ii >= 0 && ii < A.n0 && jj >= 0 && jj < A.n1 && kk >= 0 && kk < A.n2;
-        uint16_t xv = 0;
-        if (ok) {
-          if (UP) {
-            ii >>= 1;
-            jj >>= 1;
-            kk >>= 1;
-          }
-          xv = A.x[(((size_t)ii * in1 + jj) * in2 + kk) * A.cin + ci];
-        }
-        xa[j] = xv;
+  for (int brick = blockIdx.x; brick < A.nbrick; brick += gridDim.x) {
+    const int b2 = brick % nb2, b1 = (brick / nb2) % nb1, b0 = brick / (nb2 * nb1);
+    const int i0 = b0 * W::BI, j0 = b1 * W::BJ, k0 = b2 * 32;
+    __syncthreads();  // the last brick's fragments have been read
+    // x rows: voxels k0 - 1 .. k0 + 32 in five blocks of eight (the last holds two)
+    for (int u = threadIdx.x; u < W::kXRows * 5 * PI * 2; u += 256) {
+      const int c8 = u % (PI * 2), o = (u / (PI * 2)) % 5, r = u / (PI * 2 * 5);
+      int gi = i0 - 1 + r / (W::BJ + 2), gj = j0 - 1 + r % (W::BJ + 2);
+      const int c = ci0 * 16 + c8 * 8;
+      const bool ok = c < A.cin && gi >= 0 && gi < A.n0 && gj >= 0 && gj < A.n1;
+      if (UP) {
+        gi >>= 1;
+        gj >>= 1;
       }
-      u32x4 araw;
+      const uint16_t* p = A.x + ((int64_t)gi * in1 + gj) * in2 * A.cin + c;
+      u32x4 v[8], t[8];
 #pragma unroll
-      for (int h = 0; h < 4; ++h) araw[h] = (uint32_t)xa[2 * h] | ((uint32_t)xa[2 * h + 1] << 16);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, araw), bfr, acc[t], 0, 0, 0);
+      for (int q = 0; q < 8; ++q) {
+        const int e = o * 8 + q;
+        int gk = k0 - 1 + e;
+        v[q] = (u32x4){0u, 0u, 0u, 0u};
+        if (ok && e < 34 && gk >= 0 && gk < A.n2) {
+          if (UP) gk >>= 1;
+          v[q] = *reinterpret_cast<const u32x4*>(p + (int64_t)gk * A.cin);
+        }
+      }
+      transpose8(v, t);
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        *reinterpret_cast<u32x4*>(xs + (r * PI * 16 + c8 * 8 + q) * kWRow + o * 8) = t[q];
     }
+    for (int u = threadIdx.x; u < W::kGRows * 4 * PO * 2; u += 256) {
+      const int c8 = u % (PO * 2), o = (u / (PO * 2)) % 4, r = u / (PO * 2 * 4);
+      const int gi = i0 + r / W::BJ, gj = j0 + r % W::BJ;
+      const int c = co0 * 16 + c8 * 8;
+      const bool ok = c < A.cout && gi < A.n0 && gj < A.n1;
+      const uint16_t* p = A.g + ((int64_t)gi * A.n1 + gj) * A.n2 * A.cout + c;
+      u32x4 v[8], t[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int gk = k0 + o * 8 + q;
+        v[q] = (u32x4){0u, 0u, 0u, 0u};
+        if (ok && gk < A.n2) v[q] = *reinterpret_cast<const u32x4*>(p + (int64_t)gk * A.cout);
+      }
+      transpose8(v, t);
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        *reinterpret_cast<u32x4*>(gs + (r * PO * 16 + c8 * 8 + q) * kWRow + o * 8) = t[q];
+    }
+    __syncthreads();
+    if (!live) continue;
+
+    bf16x8 bfr[W::RI][W::RJ];
+#pragma unroll
+    for (int ri = 0; ri < W::RI; ++ri)
+#pragma unroll
+      for (int rj = 0; rj < W::RJ; ++rj) {
+        const int r = (si * W::RI + ri) * W::BJ + sj * W::RJ + rj;
+        bfr[ri][rj] = load8(gs + (r * PO * 16 + po * 16 + row) * kWRow + grp * 8);
+        accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ones), bfr[ri][rj], accb, 0, 0, 0);
+      }
+#pragma unroll
+    for (int xi = 0; xi < W::RI + 2; ++xi)
+#pragma unroll
+      for (int xj = 0; xj < W::RJ + 2; ++xj) {
+        const int r = (si * W::RI + xi) * (W::BJ + 2) + sj * W::RJ + xj;
+        const uint16_t* p = xs + (r * PI * 16 + pi * 16 + row) * kWRow + grp * 8;
+        const u32x4 d = *reinterpret_cast<const u32x4*>(p);
+        const uint32_t d4 = *reinterpret_cast<const uint32_t*>(p + 8);
+        const u32x4 f1 = {__builtin_amdgcn_alignbit(d[1], d[0], 16), __builtin_amdgcn_alignbit(d[2], d[1], 16),
+                          __builtin_amdgcn_alignbit(d[3], d[2], 16), __builtin_amdgcn_alignbit(d4, d[3], 16)};
+        const u32x4 f2 = {d[1], d[2], d[3], d4};
+        const bf16x8 af[3] = {__builtin_bit_cast(bf16x8, d), __builtin_bit_cast(bf16x8, f1),
+                              __builtin_bit_cast(bf16x8, f2)};
+#pragma unroll
+        for (int di = 0; di < 3; ++di)
+#pragma unroll
+          for (int dj = 0; dj < 3; ++dj) {
+            const int ri = xi - di, rj = xj - dj;
+            if (ri < 0 || ri >= W::RI || rj < 0 || rj >= W::RJ) continue;
+#pragma unroll
+            for (int dk = 0; dk < 3; ++dk) {
+              const int t = (di * 3 + dj) * 3 + dk;
+              acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[dk], bfr[ri][rj], acc[t], 0, 0, 0);
+            }
+          }
+      }
   }
-  // D[m = ci local][n = co local]: lane holds n = row, m = 4*grp + r. Sum the four waves.
-  for (int w = 0; w < 4; ++w) {
-    if (wave == w) {
+  // D[m = ci local][n = co local]: lane holds n = row, m = 4*grp + r; the bias
+  // gradient is in every m
+  float* out = A.part + ((int64_t)((ci0 + pi) * A.nco + co0 + po) * gridDim.x + blockIdx.x) * kWTile;
+  if constexpr (W::kSub == 1) {
+    if (!live) return;
+#pragma unroll
+    for (int t = 0; t < 27; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[t * 256 + (4 * grp + r) * 16 + row] = acc[t][r];
+    if (grp == 0) out[27 * 256 + row] = accb[0];
+  } else {
+    // the kSub waves of a tile pair add theirs in wave order
+    float* red = reinterpret_cast<float*>(ws) + (pi * PO + po) * kWTile;
+    for (int w = 0; w < W::kSub; ++w) {
+      __syncthreads();
+      if (sub != w) continue;
 #pragma unroll
       for (int t = 0; t < 27; ++t)
 #pragma unroll
@@ -270,58 +507,61 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs A) {
           const int idx = t * 256 + (4 * grp + r) * 16 + row;
           red[idx] = (w == 0 ? 0.f : red[idx]) + acc[t][r];
         }
+      if (grp == 0) red[27 * 256 + row] = (w == 0 ? 0.f : red[27 * 256 + row]) + accb[0];
     }
     __syncthreads();
+    if (live)
+      for (int i = lane + 64 * sub; i < kWTile; i += 64 * W::kSub) out[i] = red[i];
   }
-  float* out = A.part + ((size_t)pair * gridDim.x + blockIdx.x) * kWTile;
-  for (int i = threadIdx.x; i < kWTile; i += 256) out[i] = red[i];
 }
 
-// dW[tap][ci][co] = sum over chunks (fixed order).
-__global__ void k_wgrad_reduce(const float* part, int nchunk, int cin, int cout, int nco, float* dw) {
-  const int64_t n = 27LL * cin * cout;
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  const int co = (int)(e % cout), ci = (int)((e / cout) % cin), t = (int)(e / ((int64_t)cout * cin));
-  const int pair = (ci / 16) * nco + co / 16;
-  const float* p = part + (size_t)pair * nchunk * kWTile + t * 256 + (ci % 16) * 16 + (co % 16);
-  float s = 0.f;
-  for (int k = 0; k < nchunk; ++k) s += p[(size_t)k * kWTile];
-  dw[e] = s;
-}
+// Partials into dW[tap][ci][co] and db[co], one block of 256 threads per 64
+// elements of a tile: each wavefront adds a quarter of the chunks (64
+// neighbouring floats per chunk), the quarters are added in order. All of a
+// backward pass's layers go through one launch (15 launches of a few blocks
+// each took 1.38 ms at 64^3, one takes 0.035 ms).
+constexpr int kWMaxLayers = 16;
+struct WreduceLayer {
+  const float* part;
+  float *dw, *db;
+  int nchunk, cin, cout, nco;
+  int block0;  // first block of the layer
+};
+struct WreduceArgs {
+  WreduceLayer l[kWMaxLayers];
+  int n;
+};
+constexpr int kWredBlocks = (kWTile + 63) / 64;  // per tile
 
-// Column sums of g [nvox][cout] -> per-block partials.
-__global__ __launch_bounds__(256) void k_colsum(const uint16_t* g, int64_t nvox, int cout, float* part) {
-  __shared__ float s[256];
-  const int lanes = 256 / cout;  // cout in {16, 32, 48, 64}: 48 leaves 16 idle threads
-  const int co = threadIdx.x % cout, vl = threadIdx.x / cout;
+__global__ __launch_bounds__(256) void k_wgrad_reduce(WreduceArgs A) {
+  __shared__ float s[4][64];
+  int li = 0;
+  while (li + 1 < A.n && (int)blockIdx.x >= A.l[li + 1].block0) ++li;
+  const WreduceLayer& L = A.l[li];
+  const int b = blockIdx.x - L.block0;
+  const int pair = b / kWredBlocks, e = (b % kWredBlocks) * 64 + (threadIdx.x & 63);
+  const int w = threadIdx.x >> 6, k0 = L.nchunk * w / 4, k1 = L.nchunk * (w + 1) / 4;
   float acc = 0.f;
-  if (vl < lanes)
-    for (int64_t v = (int64_t)blockIdx.x * lanes + vl; v < nvox; v += (int64_t)gridDim.x * lanes)
-      acc += bf2f(g[v * cout + co]);
-  s[threadIdx.x] = vl < lanes ? acc : 0.f;
-  __syncthreads();
-  if (threadIdx.x < cout) {
-    float t = 0.f;
-    for (int l = 0; l < lanes; ++l) t += s[l * cout + threadIdx.x];
-    part[(size_t)blockIdx.x * cout + threadIdx.x] = t;
+  if (e < kWTile) {
+    const float* p = L.part + (int64_t)pair * L.nchunk * kWTile + e;
+#pragma unroll 8
+    for (int k = k0; k < k1; ++k) acc += p[(int64_t)k * kWTile];
   }
-}
-
-__global__ void k_colsum_reduce(const float* part, int nb, int cout, float* db) {
-  const int co = threadIdx.x;
-  if (co >= cout) return;
-  float t = 0.f;
-  for (int b = 0; b < nb; ++b) t += part[(size_t)b * cout + co];
-  db[co] = t;
+  s[w][threadIdx.x & 63] = acc;
+  __syncthreads();
+  if (w != 0 || e >= kWTile) return;
+  const int l = threadIdx.x;
+  const float v = ((s[0][l] + s[1][l]) + s[2][l]) + s[3][l];
+  const int cit = pair / L.nco, cot = pair % L.nco;
+  if (e < 27 * 256) {
+    const int t = e / 256, ci = cit * 16 + (e / 16) % 16, co = cot * 16 + e % 16;
+    if (ci < L.cin) L.dw[((int64_t)t * L.cin + ci) * L.cout + co] = v;
+  } else if (cit == 0) {
+    L.db[cot * 16 + (e - 27 * 256)] = v;
+  }
 }
 
 // ---------------------------------------------------------------- elementwise
-
-__global__ void k_relu_bwd(uint16_t* g, const uint16_t* y, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && !(bf2f(y[i]) > 0.f)) g[i] = 0;
-}
 
 // 2x2x2 mean: coarse [nc][C] from fine [2nc][C]; one thread per 8 channels.
 __global__ void k_pool(const uint16_t* xf, uint16_t* xc, int c0, int c1, int c2, int C) {
@@ -344,35 +584,70 @@ __global__ void k_pool(const uint16_t* xf, uint16_t* xc, int c0, int c1, int c2,
   for (int q = 0; q < 8; ++q) o[q] = f2bf(s[q] * 0.125f);
 }
 
-// Gradient through the mean pool, plus the skip-connection gradient:
-// gf[fine] = 0.125 * gc[fine / 2] + skip[fine].
-__global__ void k_pool_bwd(const uint16_t* gc, const uint16_t* skip, uint16_t* gf, int f0, int f1, int f2, int C) {
-  const int64_t n = (int64_t)f0 * f1 * f2 * C;
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  const int ch = (int)(e % C);
-  const int64_t v = e / C;
-  const int k = (int)(v % f2), j = (int)((v / f2) % f1), i = (int)(v / ((int64_t)f1 * f2));
-  const size_t vc = ((size_t)(i >> 1) * (f1 >> 1) + (j >> 1)) * (f2 >> 1) + (k >> 1);
-  gf[e] = f2bf(0.125f * bf2f(gc[vc * C + ch]) + bf2f(skip[e]));
+// Eight BF16 values as floats and back.
+__device__ inline void widen8(const uint16_t* p, float (&f)[8]) {
+  const u32x4 v = *reinterpret_cast<const u32x4*>(p);
+#pragma unroll
+  for (int q = 0; q < 8; ++q) f[q] = bf2f((uint16_t)(v[q >> 1] >> (16 * (q & 1))));
 }
 
-// Gradient through nearest upsampling: coarse = sum of its 8 fine children.
-__global__ void k_upsum(const uint16_t* gf, uint16_t* gc, int c0, int c1, int c2, int C) {
-  const int64_t n = (int64_t)c0 * c1 * c2 * C;
+__device__ inline void narrow8(const float (&f)[8], uint16_t* p) {
+  u32x4 v;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = (uint32_t)f2bf(f[2 * q]) | ((uint32_t)f2bf(f[2 * q + 1]) << 16);
+  *reinterpret_cast<u32x4*>(p) = v;
+}
+
+// Gradient through the mean pool, plus the skip-connection gradient, through
+// the ReLU of the pooled layer's output y: gf[fine] = 0.125 * gc[fine / 2] +
+// skip[fine] where y > 0, else 0. One thread per 8 channels.
+__global__ void k_pool_bwd(const uint16_t* gc, const uint16_t* skip, const uint16_t* y, uint16_t* gf, int f0, int f1,
+                           int f2, int C) {
+  const int cc = C >> 3;
+  const int64_t n = (int64_t)f0 * f1 * f2 * cc;
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n) return;
-  const int ch = (int)(e % C);
-  const int64_t v = e / C;
+  const int h = (int)(e % cc) * 8;
+  const int64_t v = e / cc;
+  const int k = (int)(v % f2), j = (int)((v / f2) % f1), i = (int)(v / ((int64_t)f1 * f2));
+  const size_t vc = ((size_t)(i >> 1) * (f1 >> 1) + (j >> 1)) * (f2 >> 1) + (k >> 1);
+  float a[8], b[8], g[8], o[8];
+  widen8(gc + vc * C + h, a);
+  widen8(skip + v * C + h, b);
+  widen8(y + v * C + h, g);
+#pragma unroll
+  for (int q = 0; q < 8; ++q) o[q] = g[q] > 0.f ? 0.125f * a[q] + b[q] : 0.f;
+  narrow8(o, gf + v * C + h);
+}
+
+// Gradient through nearest upsampling (coarse = sum of its 8 fine children)
+// and the ReLU of the coarse layer's output y. One thread per 8 channels.
+__global__ void k_upsum(const uint16_t* gf, const uint16_t* y, uint16_t* gc, int c0, int c1, int c2, int C) {
+  const int cc = C >> 3;
+  const int64_t n = (int64_t)c0 * c1 * c2 * cc;
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= n) return;
+  const int h = (int)(e % cc) * 8;
+  const int64_t v = e / cc;
   const int k = (int)(v % c2), j = (int)((v / c2) % c1), i = (int)(v / ((int64_t)c1 * c2));
-  float s = 0.f;
+  float s[8] = {0, 0, 0, 0, 0, 0, 0, 0}, g[8];
+#pragma unroll
   for (int a = 0; a < 2; ++a)
+#pragma unroll
     for (int b = 0; b < 2; ++b)
+#pragma unroll
       for (int c = 0; c < 2; ++c) {
         const size_t f = ((size_t)(2 * i + a) * (2 * c1) + (2 * j + b)) * (2 * c2) + (2 * k + c);
-        s += bf2f(gf[f * C + ch]);
+        float t[8];
+        widen8(gf + f * C + h, t);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s[q] += t[q];
       }
-  gc[e] = f2bf(s);
+  widen8(y + v * C + h, g);
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (!(g[q] > 0.f)) s[q] = 0.f;
+  narrow8(s, gc + v * C + h);
 }
 
 // Weight packing. Forward: wp[q][co][j] = W[tap][c0 + j][co] with q = (tap, c0/8)
@@ -615,11 +890,18 @@ __global__ void k_res_grad(const float* q, float k_over_n, Geo G, uint16_t* g) {
   *reinterpret_cast<u32x4*>(g + v * 16 + 8) = (u32x4){0u, 0u, 0u, 0u};
 }
 
-__global__ void k_sum_into(const double* part, int nb, double scale, double* out) {
-  if (threadIdx.x != 0) return;
+// *out = scale * sum of the partials (one block of 256 threads, fixed tree).
+__global__ __launch_bounds__(256) void k_sum_into(const double* part, int nb, double scale, double* out) {
+  __shared__ double s[256];
   double t = 0.0;
-  for (int b = 0; b < nb; ++b) t += part[b];
-  *out = t * scale;
+  for (int b = threadIdx.x; b < nb; b += 256) t += part[b];
+  s[threadIdx.x] = t;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *out = s[0] * scale;
 }
 
 // Training-data objects: axis-aligned boxes of cells. Cells inside get the
@@ -697,7 +979,9 @@ struct GuessNet {
   DBuf<uint16_t> gOUT, gE0, gD0, gE1, gD1, gE2, gD2, gB3, gA3, gP2, gS2, gA2, gP1, gS1, gA1, gP0, gS0, gA0;
   DBuf<uint16_t> T0, T1, T2;
   bool train_alloc = false;
-  DBuf<float> wpart, cpart;  // weight- and bias-gradient partial sums
+  std::vector<DBuf<float>> wpart;  // weight- and bias-gradient partial sums, one buffer per layer
+  WreduceArgs wred{};              // the layers whose partials wait for k_wgrad_reduce
+  int wred_blocks = 0;
   DBuf<double> dpart, scal, loss_acc;
   DBuf<uint8_t> cellmask;  // training-data objects
   DBuf<double> rwarm;      // eps0 (b - A phi) of the warm start at the interior nodes (modes 2 and 3)
@@ -751,45 +1035,70 @@ void pack_all(Ctx& c, GuessNet& g) {
   }
 }
 
-template <int NT, int EPI, bool UP>
-void launch_conv_t(hipStream_t st, const ConvArgs& a) {
-  const int64_t nb = (int64_t)div_up(a.n0, kBI) * div_up(a.n1, kBJ) * div_up(a.n2, kBK);
-  const size_t lds = conv_lds_bytes(a.cin);
-  static size_t granted = 65536;  // dynamic LDS this instance may use (raised once as needed)
-  const size_t most = conv_lds_bytes(64);
-  if (lds > granted) {
-    FOPIS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_conv<NT, EPI, UP>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)most));
-    granted = most;
-  }
-  k_conv<NT, EPI, UP><<<(unsigned)nb, 256, lds, st>>>(a);
+// Raises an instance's dynamic LDS limit once.
+template <class K>
+void grant_lds(K* kernel, size_t bytes, size_t& granted) {
+  if (bytes <= granted) return;
+  FOPIS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)bytes));
+  granted = bytes;
 }
 
-template <int EPI, bool UP>
-void launch_conv_nt(hipStream_t st, const ConvArgs& a) {
-  switch (a.cout / 16) {
-    case 1: launch_conv_t<1, EPI, UP>(st, a); break;
-    case 2: launch_conv_t<2, EPI, UP>(st, a); break;
-    case 3: launch_conv_t<3, EPI, UP>(st, a); break;
-    case 4: launch_conv_t<4, EPI, UP>(st, a); break;
-    default: throw Error(FOPIS_E_ARG, "conv: output channels must be 16, 32, 48 or 64");
+template <int CIN, int NT, int EPI>
+void launch_conv_t(hipStream_t st, ConvArgs& a) {
+  constexpr size_t lds = conv_lds_bytes(CIN);
+  static size_t granted = 65536;
+  grant_lds(&k_conv<CIN, NT, EPI>, lds, granted);
+  a.nbrick = div_up(a.n0, kBI) * div_up(a.n1, kBJ) * div_up(a.n2, kBK);
+  // a few workgroups per compute unit, as many as its LDS holds, so that one
+  // brick's loads and stores overlap another's products
+  const int most = 256 * (int)std::max<size_t>(1, std::min<size_t>(NT <= 2 ? 3 : 2, 163840 / lds));
+  k_conv<CIN, NT, EPI><<<dim3(std::min(a.nbrick, most), a.cout / (16 * NT)), 256, lds, st>>>(a);
+}
+
+template <int CIN>
+void launch_conv_nt(hipStream_t st, ConvArgs& a) {
+  // One tile per workgroup below 512 bricks: two workgroups per compute unit
+  // want more of them than there are bricks, and the weights then fit the
+  // registers (64 -> 64 at 16^3: 22.7 us with all four tiles, 15.2 us; 48 ->
+  // 48 at 32^3 inside the network 30.8 and 20.3 us). From 512 bricks on every
+  // fragment read serves all tiles (32 -> 32 at 64^3: 30 us).
+  const int nbrick = div_up(a.n0, kBI) * div_up(a.n1, kBJ) * div_up(a.n2, kBK);
+  switch (nbrick < 512 ? 1 : a.cout / 16) {
+    case 1: launch_conv_t<CIN, 1, EPI_BF16>(st, a); break;
+    case 2: launch_conv_t<CIN, 2, EPI_BF16>(st, a); break;
+    case 3: launch_conv_t<CIN, 3, EPI_BF16>(st, a); break;
+    case 4: launch_conv_t<CIN, 4, EPI_BF16>(st, a); break;
   }
 }
 
-void launch_conv(hipStream_t st, const ConvArgs& a, int epi, bool up) {
-  if (a.cin % 8 != 0 || a.cin > 64 || a.cin < 8) throw Error(FOPIS_E_ARG, "conv: input channels must be 8..64, multiple of 8");
+void launch_conv(hipStream_t st, ConvArgs a, int epi, bool up) {
   if (up && (a.n0 % 2 || a.n1 % 2 || a.n2 % 2)) throw Error(FOPIS_E_ARG, "conv: upsampled grid must be even");
-  if (epi == EPI_BF16) {
-    if (up) launch_conv_nt<EPI_BF16, true>(st, a); else launch_conv_nt<EPI_BF16, false>(st, a);
-  } else if (epi == EPI_F32) {
-    if (up) launch_conv_nt<EPI_F32, true>(st, a); else launch_conv_nt<EPI_F32, false>(st, a);
-  } else {
-    if (up) launch_conv_nt<EPI_PHI, true>(st, a); else launch_conv_nt<EPI_PHI, false>(st, a);
+  if (a.cout < 16 || a.cout > 64 || a.cout % 16)
+    throw Error(FOPIS_E_ARG, "conv: output channels must be 16, 32, 48 or 64");
+  a.up = up ? 1 : 0;
+  if (epi != EPI_BF16) {  // the output layer
+    if (a.cin != 16 || a.cout != 16 || up) throw Error(FOPIS_E_ARG, "conv: the output layer is 16 -> 16 channels");
+    if (epi == EPI_F32)
+      launch_conv_t<16, 1, EPI_F32>(st, a);
+    else
+      launch_conv_t<16, 1, EPI_PHI>(st, a);
+    return;
+  }
+  switch (a.cin) {
+    case 8: launch_conv_nt<8>(st, a); break;
+    case 16: launch_conv_nt<16>(st, a); break;
+    case 24: launch_conv_nt<24>(st, a); break;
+    case 32: launch_conv_nt<32>(st, a); break;
+    case 40: launch_conv_nt<40>(st, a); break;
+    case 48: launch_conv_nt<48>(st, a); break;
+    case 56: launch_conv_nt<56>(st, a); break;
+    case 64: launch_conv_nt<64>(st, a); break;
+    default: throw Error(FOPIS_E_ARG, "conv: input channels must be 8..64, multiple of 8");
   }
 }
 
-ConvArgs conv_args(const int* d, int cin, int cout, int nq, int nqp, const uint16_t* x, const uint16_t* w,
-                   const float* b, int relu) {
+ConvArgs conv_args(const int* d, int cin, int cout, const uint16_t* x, const uint16_t* w, const float* b, int relu) {
   ConvArgs a{};
   a.x = x;
   a.w = w;
@@ -799,17 +1108,34 @@ ConvArgs conv_args(const int* d, int cin, int cout, int nq, int nqp, const uint1
   a.n2 = d[2];
   a.cin = cin;
   a.cout = cout;
-  a.nq = nq;
-  a.nqp = nqp;
   a.relu = relu;
   return a;
 }
 
-// Weight and bias gradient of one layer into the flat gradient vector.
-void wgrad(Ctx& c, GuessNet& g, const int* d, int cin, int cout, bool up, const uint16_t* x, const uint16_t* gy,
-           float* dw, float* db) {
-  const int64_t nvox = nvox_of(d);
-  const int nci = (cin + 15) / 16, nco = cout / 16, npairs = nci * nco;
+template <int PI, int PO>
+int wgrad_chunks(const WgradArgs& a) {
+  using W = WgradShape<PI, PO>;
+  const int groups = div_up(a.nci, PI) * div_up(a.nco, PO);
+  const int nbrick = div_up(a.n0, W::BI) * div_up(a.n1, W::BJ) * div_up(a.n2, 32);
+  // one workgroup per compute unit: more of them add partials (two per unit:
+  // the sum of the partials of a 64^3 pair took 54 us instead of 35, the
+  // gradients the same)
+  return std::min(nbrick, std::max(1, 256 / groups));
+}
+
+template <int PI, int PO, bool UP>
+void launch_wgrad_t(hipStream_t st, WgradArgs& a, int nchunk) {
+  using W = WgradShape<PI, PO>;
+  static size_t granted = 65536;
+  grant_lds(&k_wgrad<PI, PO, UP>, W::kLds, granted);
+  a.nbrick = div_up(a.n0, W::BI) * div_up(a.n1, W::BJ) * div_up(a.n2, 32);
+  k_wgrad<PI, PO, UP><<<dim3(nchunk, div_up(a.nci, PI) * div_up(a.nco, PO)), 256, W::kLds, st>>>(a);
+}
+
+// Weight and bias gradient of one layer: the partials now, dw and db when
+// wgrad_flush runs. `slot` names the layer's partial buffer.
+void wgrad(Ctx& c, GuessNet& g, int slot, const int* d, int cin, int cout, bool up, const uint16_t* x,
+           const uint16_t* gy, float* dw, float* db) {
   WgradArgs a{};
   a.x = x;
   a.g = gy;
@@ -818,26 +1144,42 @@ void wgrad(Ctx& c, GuessNet& g, const int* d, int cin, int cout, bool up, const 
   a.n2 = d[2];
   a.cin = cin;
   a.cout = cout;
-  a.nco = nco;
-  a.nsteps = (nvox + 31) / 32;
-  int nchunk = (int)std::min<int64_t>(std::max(1, 1024 / npairs), (a.nsteps + 3) / 4);
-  nchunk = std::max(nchunk, 1);
+  a.nci = (cin + 15) / 16;
+  a.nco = cout / 16;
+  const int kind = (a.nci > 1 ? 2 : 0) + (a.nco > 1 ? 1 : 0);
+  const int nchunk = kind == 0 ? wgrad_chunks<1, 1>(a) : kind == 1 ? wgrad_chunks<1, 2>(a)
+                     : kind == 2 ? wgrad_chunks<2, 1>(a) : wgrad_chunks<2, 2>(a);
+  const int npairs = a.nci * a.nco;
   const size_t need = (size_t)npairs * nchunk * kWTile;
-  if (g.wpart.n < need) {
+  if ((int)g.wpart.size() <= slot) g.wpart.resize(slot + 1);
+  if (g.wpart[slot].n < need) {
     FOPIS_HIP(hipStreamSynchronize(c.stream));
-    g.wpart.alloc(need);
+    g.wpart[slot].alloc(need);
   }
-  a.part = g.wpart.p;
+  a.part = g.wpart[slot].p;
+  auto go = [&](auto up_c) {
+    constexpr bool U = decltype(up_c)::value;
+    if (kind == 0)
+      launch_wgrad_t<1, 1, U>(c.stream, a, nchunk);
+    else if (kind == 1)
+      launch_wgrad_t<1, 2, U>(c.stream, a, nchunk);
+    else if (kind == 2)
+      launch_wgrad_t<2, 1, U>(c.stream, a, nchunk);
+    else
+      launch_wgrad_t<2, 2, U>(c.stream, a, nchunk);
+  };
   if (up)
-    k_wgrad<true><<<dim3(nchunk, npairs), 256, 0, c.stream>>>(a);
+    go(std::true_type{});
   else
-    k_wgrad<false><<<dim3(nchunk, npairs), 256, 0, c.stream>>>(a);
-  const int64_t nw = 27LL * cin * cout;
-  k_wgrad_reduce<<<div_up(nw, 256), 256, 0, c.stream>>>(g.wpart.p, nchunk, cin, cout, nco, dw);
-  const int nb = (int)std::min<int64_t>(1024, std::max<int64_t>(1, nvox / 256));
-  if (!g.cpart.p) g.cpart.alloc((size_t)1024 * 64);
-  k_colsum<<<nb, 256, 0, c.stream>>>(gy, nvox, cout, g.cpart.p);
-  k_colsum_reduce<<<1, 64, 0, c.stream>>>(g.cpart.p, nb, cout, db);
+    go(std::false_type{});
+  g.wred.l[g.wred.n++] = WreduceLayer{a.part, dw, db, nchunk, cin, cout, a.nco, g.wred_blocks};
+  g.wred_blocks += npairs * kWredBlocks;
+}
+
+void wgrad_flush(Ctx& c, GuessNet& g) {
+  if (g.wred.n > 0) k_wgrad_reduce<<<g.wred_blocks, 256, 0, c.stream>>>(g.wred);
+  g.wred.n = 0;
+  g.wred_blocks = 0;
 }
 
 void alloc_train(GuessNet& g) {
@@ -876,7 +1218,7 @@ void forward(Ctx& c, GuessNet& g, int epi, bool phi_add = false) {
   hipStream_t st = c.stream;
   auto conv = [&](int li, const uint16_t* x, const uint16_t* add, uint16_t* y) {
     GuessLayer& l = g.L[li];
-    ConvArgs a = conv_args(g.lv[l.lvl], l.cin, l.cout, l.nq, l.nqp, x, l.wp.p, g.master.p + l.boff, l.relu);
+    ConvArgs a = conv_args(g.lv[l.lvl], l.cin, l.cout, x, l.wp.p, g.master.p + l.boff, l.relu);
     a.add = add;
     a.y = y;
     launch_conv(st, a, EPI_BF16, l.up != 0);
@@ -903,7 +1245,7 @@ void forward(Ctx& c, GuessNet& g, int epi, bool phi_add = false) {
   conv(D0A, g.E1.p, g.S0.p, g.D0.p);
   conv(D0B, g.D0.p, nullptr, g.E0.p);
   GuessLayer& lo = g.L[OUTL];
-  ConvArgs a = conv_args(g.lv[0], lo.cin, lo.cout, lo.nq, lo.nqp, g.E0.p, lo.wp.p, g.master.p + lo.boff, 0);
+  ConvArgs a = conv_args(g.lv[0], lo.cin, lo.cout, g.E0.p, lo.wp.p, g.master.p + lo.boff, 0);
   if (epi == EPI_F32) {
     a.y32 = g.OUT.p;
   } else {
@@ -924,79 +1266,64 @@ void forward(Ctx& c, GuessNet& g, int epi, bool phi_add = false) {
 // Backward pass from g.gOUT; fills g.grad.
 void backward(Ctx& c, GuessNet& g) {
   hipStream_t st = c.stream;
-  auto relu_bwd = [&](uint16_t* gy, const uint16_t* y, int lvl, int C) {
-    const int64_t n = nvox_of(g.lv[lvl]) * C;
-    k_relu_bwd<<<div_up(n, 256), 256, 0, st>>>(gy, y, n);
-  };
   auto wg = [&](int li, const uint16_t* x, const uint16_t* gy) {
     GuessLayer& l = g.L[li];
-    wgrad(c, g, g.lv[l.lvl], l.cin, l.cout, l.up != 0, x, gy, g.grad.p + l.woff, g.grad.p + l.boff);
+    wgrad(c, g, li, g.lv[l.lvl], l.cin, l.cout, l.up != 0, x, gy, g.grad.p + l.woff, g.grad.p + l.boff);
   };
-  // data gradient of layer li at its output grid into dx ([out voxels][cin])
-  auto dg = [&](int li, const uint16_t* gy, uint16_t* dx) {
+  // data gradient of layer li at its output grid into dx ([out voxels][cin]),
+  // through the ReLU of the layer's input y where that is a layer's output
+  auto dg = [&](int li, const uint16_t* gy, uint16_t* dx, const uint16_t* y = nullptr) {
     GuessLayer& l = g.L[li];
     const float* zero_bias = g.master.p + g.nparams;  // cin zeros kept after the parameters
-    ConvArgs a = conv_args(g.lv[l.lvl], l.cout, l.cin, l.nqd, l.nqpd, gy, l.wd.p, zero_bias, 0);
+    ConvArgs a = conv_args(g.lv[l.lvl], l.cout, l.cin, gy, l.wd.p, zero_bias, 0);
     a.y = dx;
+    a.gate = y;
     launch_conv(st, a, EPI_BF16, false);
   };
-  auto upsum = [&](const uint16_t* gf, uint16_t* gcoarse, int lc, int C) {
+  auto upsum = [&](const uint16_t* gf, const uint16_t* y, uint16_t* gcoarse, int lc, int C) {
     const int* d = g.lv[lc];
-    k_upsum<<<div_up(nvox_of(d) * C, 256), 256, 0, st>>>(gf, gcoarse, d[0], d[1], d[2], C);
+    k_upsum<<<div_up(nvox_of(d) * (C / 8), 256), 256, 0, st>>>(gf, y, gcoarse, d[0], d[1], d[2], C);
   };
-  auto poolb = [&](const uint16_t* gcoarse, const uint16_t* skip, uint16_t* gf, int lf, int C) {
+  auto poolb = [&](const uint16_t* gcoarse, const uint16_t* skip, const uint16_t* y, uint16_t* gf, int lf, int C) {
     const int* d = g.lv[lf];
-    k_pool_bwd<<<div_up(nvox_of(d) * C, 256), 256, 0, st>>>(gcoarse, skip, gf, d[0], d[1], d[2], C);
+    k_pool_bwd<<<div_up(nvox_of(d) * (C / 8), 256), 256, 0, st>>>(gcoarse, skip, y, gf, d[0], d[1], d[2], C);
   };
   wg(OUTL, g.E0.p, g.gOUT.p);
-  dg(OUTL, g.gOUT.p, g.gE0.p);
-  relu_bwd(g.gE0.p, g.E0.p, 0, 16);
+  dg(OUTL, g.gOUT.p, g.gE0.p, g.E0.p);
   wg(D0B, g.D0.p, g.gE0.p);
-  dg(D0B, g.gE0.p, g.gD0.p);
-  relu_bwd(g.gD0.p, g.D0.p, 0, 16);
+  dg(D0B, g.gE0.p, g.gD0.p, g.D0.p);
   wg(D0A, g.E1.p, g.gD0.p);
   dg(D0A, g.gD0.p, g.T0.p);
-  upsum(g.T0.p, g.gE1.p, 1, 32);
-  relu_bwd(g.gE1.p, g.E1.p, 1, 32);
+  upsum(g.T0.p, g.E1.p, g.gE1.p, 1, 32);
   wg(D1B, g.D1.p, g.gE1.p);
-  dg(D1B, g.gE1.p, g.gD1.p);
-  relu_bwd(g.gD1.p, g.D1.p, 1, 32);
+  dg(D1B, g.gE1.p, g.gD1.p, g.D1.p);
   wg(D1A, g.E2.p, g.gD1.p);
   dg(D1A, g.gD1.p, g.T1.p);
-  upsum(g.T1.p, g.gE2.p, 2, 48);
-  relu_bwd(g.gE2.p, g.E2.p, 2, 48);
+  upsum(g.T1.p, g.E2.p, g.gE2.p, 2, 48);
   wg(D2B, g.D2.p, g.gE2.p);
-  dg(D2B, g.gE2.p, g.gD2.p);
-  relu_bwd(g.gD2.p, g.D2.p, 2, 48);
+  dg(D2B, g.gE2.p, g.gD2.p, g.D2.p);
   wg(D2A, g.B3.p, g.gD2.p);
   dg(D2A, g.gD2.p, g.T2.p);
-  upsum(g.T2.p, g.gB3.p, 3, 64);
-  relu_bwd(g.gB3.p, g.B3.p, 3, 64);
+  upsum(g.T2.p, g.B3.p, g.gB3.p, 3, 64);
   wg(E3B, g.A3.p, g.gB3.p);
-  dg(E3B, g.gB3.p, g.gA3.p);
-  relu_bwd(g.gA3.p, g.A3.p, 3, 64);
+  dg(E3B, g.gB3.p, g.gA3.p, g.A3.p);
   wg(E3A, g.P2.p, g.gA3.p);
   dg(E3A, g.gA3.p, g.gP2.p);
-  poolb(g.gP2.p, g.gD2.p, g.gS2.p, 2, 48);
-  relu_bwd(g.gS2.p, g.S2.p, 2, 48);
+  poolb(g.gP2.p, g.gD2.p, g.S2.p, g.gS2.p, 2, 48);
   wg(E2B, g.A2.p, g.gS2.p);
-  dg(E2B, g.gS2.p, g.gA2.p);
-  relu_bwd(g.gA2.p, g.A2.p, 2, 48);
+  dg(E2B, g.gS2.p, g.gA2.p, g.A2.p);
   wg(E2A, g.P1.p, g.gA2.p);
   dg(E2A, g.gA2.p, g.gP1.p);
-  poolb(g.gP1.p, g.gD1.p, g.gS1.p, 1, 32);
-  relu_bwd(g.gS1.p, g.S1.p, 1, 32);
+  poolb(g.gP1.p, g.gD1.p, g.S1.p, g.gS1.p, 1, 32);
   wg(E1B, g.A1.p, g.gS1.p);
-  dg(E1B, g.gS1.p, g.gA1.p);
-  relu_bwd(g.gA1.p, g.A1.p, 1, 32);
+  dg(E1B, g.gS1.p, g.gA1.p, g.A1.p);
   wg(E1A, g.P0.p, g.gA1.p);
   dg(E1A, g.gA1.p, g.gP0.p);
-  poolb(g.gP0.p, g.gD0.p, g.gS0.p, 0, 16);
-  relu_bwd(g.gS0.p, g.S0.p, 0, 16);
+  poolb(g.gP0.p, g.gD0.p, g.S0.p, g.gS0.p, 0, 16);
   wg(E0B, g.A0.p, g.gS0.p);
-  dg(E0B, g.gS0.p, g.gA0.p);
-  relu_bwd(g.gA0.p, g.A0.p, 0, 16);
+  dg(E0B, g.gS0.p, g.gA0.p, g.A0.p);
   wg(E0A, g.X0.p, g.gA0.p);
+  wgrad_flush(c, g);
 }
 
 GuessNet& net(Ctx& c) {
@@ -1024,7 +1351,7 @@ void launch_loss(Ctx& c, GuessNet& g, int slot, double* dst) {
     k_loss<<<nb, 256, 0, c.stream>>>(g.OUT.p, g.ds_phi.p + (size_t)slot * n, (float)(1.0 / g.k_out), g.G,
                                      (float)(1.0 / nvalid), g.gOUT.p, g.dpart.p);
   }
-  k_sum_into<<<1, 1, 0, c.stream>>>(g.dpart.p, nb, 1.0 / nvalid, dst);
+  k_sum_into<<<1, 256, 0, c.stream>>>(g.dpart.p, nb, 1.0 / nvalid, dst);
 }
 
 double loss_and_grad(Ctx& c, GuessNet& g, int slot, bool sync) {
@@ -1465,7 +1792,7 @@ void nn_conv3d(int n0, int n1, int n2, int cin, int cout, int up, int relu, cons
   }
   k_pack<<<div_up((int64_t)nqp * cout * 8, 256), 256, 0, ts.s>>>(dw.p, dwp.p, cin, cout, nqp, 0);
   const int dims[3] = {n0, n1, n2};
-  ConvArgs a = conv_args(dims, cin, cout, nq, nqp, dx.p, dwp.p, db.p, relu);
+  ConvArgs a = conv_args(dims, cin, cout, dx.p, dwp.p, db.p, relu);
   a.add = add ? dadd.p : nullptr;
   a.y = dy.p;
   launch_conv(ts.s, a, EPI_BF16, up != 0);
@@ -1510,14 +1837,15 @@ void nn_conv3d_backward(int n0, int n1, int n2, int cin, int cout, int up, const
   Ctx cc;
   cc.stream = ts.s;
   const int dims[3] = {n0, n1, n2};
-  wgrad(cc, tmp, dims, cin, cout, up != 0, dx.p, dg.p, dgw.p, dgb.p);
+  wgrad(cc, tmp, 0, dims, cin, cout, up != 0, dx.p, dg.p, dgw.p, dgb.p);
+  wgrad_flush(cc, tmp);
   cc.stream = nullptr;
   if (dx_out) {
     const int nqd = 27 * cout / 8, nqpd = (nqd + 3) / 4 * 4;
     dwd.alloc((size_t)nqpd * cin * 8);
     k_pack<<<div_up((int64_t)nqpd * cin * 8, 256), 256, 0, ts.s>>>(dw.p, dwd.p, cin, cout, nqpd, 1);
     ddx.alloc(nv * cin);
-    ConvArgs a = conv_args(dims, cout, cin, nqd, nqpd, dg.p, dwd.p, zb.p, 0);
+    ConvArgs a = conv_args(dims, cout, cin, dg.p, dwd.p, zb.p, 0);
     a.y = ddx.p;
     launch_conv(ts.s, a, EPI_BF16, false);
     FOPIS_HIP(hipStreamSynchronize(ts.s));

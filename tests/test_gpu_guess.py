@@ -80,6 +80,36 @@ def test_conv_backward_matches_oracle(shape, cin, cout, up):
             _close_bf16(dx, rdx)
 
 
+@pytest.mark.parametrize("shape,cin,cout,up", [
+    ((1, 2, 3), 16, 16, False),     # smaller than a brick along every axis
+    ((9, 5, 33), 8, 32, False),     # remainders of the 4 x 4 x 16 brick and of the 32-voxel run
+    ((10, 6, 34), 24, 48, True),    # channel counts between the tiles, odd tile groups
+    ((5, 9, 17), 40, 16, False),
+    ((6, 2, 18), 56, 64, True),
+    ((20, 20, 520), 16, 16, False),  # several bricks per workgroup, weights in registers
+    ((16, 32, 272), 32, 32, False),  # 544 bricks: all output tiles in one workgroup
+])
+def test_conv_brick_edges_match_oracle(shape, cin, cout, up):
+    """Forward with the skip addend and ReLU, weight, bias and data gradient
+    where bricks, channel tiles and workgroups end; the bars of the two tests above."""
+    rng = np.random.default_rng(13)
+    xs = tuple(s // 2 for s in shape) if up else shape
+    x = _bf16_input(rng, xs + (cin,))
+    W = (rng.standard_normal((27, cin, cout)) * np.sqrt(2.0 / (27 * cin))).astype(np.float32)
+    b = rng.uniform(-0.2, 0.2, cout).astype(np.float32)
+    a = _bf16_input(rng, shape + (cout,), 0.5)
+    xf = GU.from_bf16(x).astype(np.float64)
+    y = GU.conv3d(x, W, b, up=up, relu=True, add_bf16=a)
+    _close_bf16(y, np.maximum(unet.conv3d(xf, unet.bf16_round(W), b.astype(np.float64), up) + GU.from_bf16(a), 0.0))
+    gy = _bf16_input(rng, shape + (cout,))
+    dw, db, dx = GU.conv3d_backward(x, W, gy, up=up, want_dx=cin % 16 == 0)
+    rW, rb, rdx = unet.conv3d_backward(xf, unet.bf16_round(W), GU.from_bf16(gy).astype(np.float64), up)
+    np.testing.assert_allclose(dw, rW, rtol=1e-4, atol=1e-4 * np.max(np.abs(rW)))
+    np.testing.assert_allclose(db, rb, rtol=1e-4, atol=1e-4 * np.max(np.abs(rb)))
+    if cin % 16 == 0 and not up:
+        _close_bf16(dx, rdx)
+
+
 def _desc(n):
     return F.make_desc(n, n, n, [(-1.0, 1.0, 1.0)], eps0=1.0, mg_precision=F.FP64)
 
