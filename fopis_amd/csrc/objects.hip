@@ -116,12 +116,21 @@ __global__ void k_gj_elim(double* A, double* I, int n, int c, const double* f) {
   I[(size_t)r * n + q] -= fr * I[(size_t)c * n + q];
 }
 
-// colsum[j] = sum_i C(i,j) (i ascending) and the Cmatrix::total order
-__global__ void k_colsum(const double* C, int n, double* colsum) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
+// colsum[j] = sum_i C(i,j): 64 columns per workgroup, each of its 16
+// wavefronts adds a sixteenth of the rows, their sums are added in row order
+// (a thread per column alone kept 7 workgroups busy for 1538 dependent rows)
+__global__ __launch_bounds__(1024) void k_colsum(const double* C, int n, double* colsum) {
+  __shared__ double sh[16][64];
+  const int j = blockIdx.x * 64 + (threadIdx.x & 63), w = threadIdx.x >> 6;
+  const int i0 = (int)((int64_t)n * w / 16), i1 = (int)((int64_t)n * (w + 1) / 16);
   double s = 0.0;
-  for (int i = 0; i < n; ++i) s += C[(size_t)i * n + j];
+  if (j < n)
+#pragma unroll 8
+    for (int i = i0; i < i1; ++i) s += C[(size_t)i * n + j];
+  sh[w][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (w != 0 || j >= n) return;
+  for (int q = 1; q < 16; ++q) s += sh[q][threadIdx.x];
   colsum[j] = s;
 }
 
@@ -336,7 +345,7 @@ int objects_lit_nodes(Ctx& c, int o, int axis, int sign, const int32_t** dev_ijk
 
 static void finish_cmatrix(Ctx& c, ObjectDev& ob) {
   const int n = ob.ncmat;
-  k_colsum<<<div_up(n, 256), 256, 0, c.stream>>>(ob.C.p, n, ob.colsum.p);
+  k_colsum<<<div_up(n, 64), 1024, 0, c.stream>>>(ob.C.p, n, ob.colsum.p);
   k_total<<<1, 256, 0, c.stream>>>(ob.colsum.p, n, ob.scal.p + 3);
   FOPIS_HIP(hipMemcpyAsync(&ob.total_cmat, ob.scal.p + 3, sizeof(double), hipMemcpyDeviceToHost, c.stream));
   FOPIS_HIP(hipStreamSynchronize(c.stream));
@@ -420,23 +429,34 @@ __global__ void k_pair_products(const double* S, int m, int w, double* P) {
   P[i] = S[(int64_t)k * w + a] * S[(int64_t)k * w + b];
 }
 
-// B(col,row): one wavefront per (col, row) pair, lanes over k_a; a bounded
-// grid strides over the pairs (n^2 wavefronts of 64 lanes would pass the
-// 2^32 work-items a launch can hold once n exceeds 8192)
-__global__ __launch_bounds__(256) void k_green_pairs(const double* __restrict__ U, const double* __restrict__ Sa,
+// B(col,row): one wavefront per pair row <= col, lanes over k_a, written to
+// both places (the sums are the same products in the same order either way).
+// Pa is k_pair_products' table of axis a, so both factors are read along k. A
+// bounded grid strides over the pairs (n^2 wavefronts of 64 lanes would pass
+// the 2^32 work-items a launch can hold once n exceeds 8192). Bound by L2
+// reads, 2 KB per pair at 127 nodes: 1538 surface nodes 0.84 -> 0.33 ms.
+__global__ __launch_bounds__(256) void k_green_pairs(const double* __restrict__ U, const double* __restrict__ Pa,
                                                      const int32_t* __restrict__ box, int n, int ma, int wa,
                                                      int wb, int wc, double scale, double* __restrict__ B) {
   const int lane = threadIdx.x & 63;
-  const int64_t npair = (int64_t)n * n;
+  const int64_t npair = (int64_t)n * (n + 1) / 2;
   for (int64_t pair = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); pair < npair; pair += (int64_t)gridDim.x * 4) {
-    const int col = (int)(pair / n), row = (int)(pair % n);
+    // pair = col (col + 1) / 2 + row; the square root is exact to one
+    int col = (int)((sqrt(8.0 * (double)pair + 1.0) - 1.0) * 0.5);
+    if ((int64_t)col * (col + 1) / 2 > pair) --col;
+    if ((int64_t)(col + 1) * (col + 2) / 2 <= pair) ++col;
+    const int row = (int)(pair - (int64_t)col * (col + 1) / 2);
     const int aa = box[3 * col], ab = box[3 * col + 1], ac = box[3 * col + 2];
     const int ba = box[3 * row], bb = box[3 * row + 1], bc = box[3 * row + 2];
     const double* u = U + (((int64_t)ab * wb + bb) * (wc * wc) + (int64_t)ac * wc + bc) * ma;
+    const double* p = Pa + ((int64_t)aa * wa + ba) * ma;
     double s = 0.0;
-    for (int k = lane; k < ma; k += 64) s += Sa[(int64_t)k * wa + aa] * Sa[(int64_t)k * wa + ba] * u[k];
+    for (int k = lane; k < ma; k += 64) s += p[k] * u[k];
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if (lane == 0) B[(size_t)col * n + row] = s * scale;
+    if (lane == 0) {
+      B[(size_t)col * n + row] = s * scale;
+      B[(size_t)row * n + col] = s * scale;
+    }
   }
 }
 
@@ -515,12 +535,244 @@ static bool spectral_unit_responses(Ctx& c, ObjectDev& ob, double* B) {
   DBuf<int32_t> box;
   box.alloc(hbox.size());
   FOPIS_HIP(hipMemcpyAsync(box.p, hbox.data(), hbox.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
-  const int64_t pairs = (int64_t)n * n;
+  DBuf<double> Pa;
+  Pa.alloc((size_t)wa * wa * ma);
+  k_pair_products<<<div_up((int64_t)wa * wa * ma, 256), 256, 0, st>>>(S[A_].p, ma, wa, Pa.p);
+  const int64_t pairs = (int64_t)n * (n + 1) / 2;
   const int64_t gblocks = std::min<int64_t>(div_up(pairs, 4), (int64_t)1 << 20);
-  k_green_pairs<<<(unsigned)gblocks, 256, 0, st>>>(U.p, S[A_].p, box.p, n, ma, wa, wb, wc, 1.0 / c.d.eps0, B);
+  k_green_pairs<<<(unsigned)gblocks, 256, 0, st>>>(U.p, Pa.p, box.p, n, ma, wa, wb, wc, 1.0 / c.d.eps0, B);
   FOPIS_HIP(hipGetLastError());
   FOPIS_HIP(hipStreamSynchronize(st));
   return true;
+}
+
+// ---- C = B^-1 for the sine-transform responses
+//
+// That B is a principal block of A^-1, symmetric and positive definite, so its
+// inverse needs no pivots. Blocked Gauss-Jordan in place on a copy padded to
+// whole 64 x 64 tiles (the padding is the identity): per block column, the
+// block row is multiplied by the diagonal tile's inverse and the block column
+// set aside (k_bj_panel), and every other tile takes one 64-deep product
+// (k_bj_update, v_mfma_f64_16x16x4), the first of them inverting the next
+// diagonal tile behind the others. The matrix is read and written once per 64
+// columns instead of once per column, by 2 launches instead of 256: 1538 nodes 36 -> 1.2 ms (bound by the 64 serial
+// steps of the diagonal tiles, 25 us each), the whole build at 6146 nodes
+// 1.6 s -> 42 ms (bound by the tiles' traffic). A pivot
+// that is not safely positive (surface nodes given twice) sets *bad, and the
+// caller falls back on the pivoted elimination.
+constexpr int kBJ = 64;
+constexpr int kBJA = 68, kBJB = 80;  // LDS row lengths: the fragment reads then spread over the banks
+
+__global__ void k_bj_load(const double* __restrict__ B, int n, double* __restrict__ W, int np) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (int64_t)np * np) return;
+  const int r = (int)(i / np), c = (int)(i % np);
+  W[i] = r < n && c < n ? B[(int64_t)r * n + c] : (r == c ? 1.0 : 0.0);
+}
+
+__global__ void k_bj_store(const double* __restrict__ W, int np, double* __restrict__ C, int n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (int64_t)n * n) return;
+  C[i] = W[(i / n) * np + i % n];
+}
+
+// Inverse of the diagonal tile at k0 by one workgroup: every thread holds a
+// 4 x 4 piece, and each elimination step passes its row and column through
+// LDS (two pairs of buffers, so one barrier a step).
+struct BjDiag {
+  double row[2][kBJ], col[2][kBJ], diag[kBJ];
+};
+
+__device__ void bj_diag(BjDiag& s, const double* W, int np, int k0, const double* __restrict__ B, int n, double* Dinv,
+                        int* bad) {
+  const int tr = threadIdx.x / 16 * 4, tc = threadIdx.x % 16 * 4;
+  double m[4][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) m[u][v] = W[(int64_t)(k0 + tr + u) * np + k0 + tc + v];
+  if (threadIdx.x < kBJ) {
+    const int d = k0 + threadIdx.x;
+    s.diag[threadIdx.x] = d < n ? B[(int64_t)d * n + d] : 1.0;
+  }
+  bool ok = true;
+  for (int c4 = 0; c4 < kBJ; c4 += 4)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int c = c4 + q;
+      double* row = s.row[q & 1];
+      double* col = s.col[q & 1];
+      if (tr == c4)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) row[tc + v] = m[q][v];
+      if (tc == c4)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) col[tr + u] = m[u][q];
+      __syncthreads();
+      const double p = row[c];
+      ok = ok && p > 1e-13 * s.diag[c];
+      const double ip = 1.0 / p;
+      double rv[4], cv[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) rv[v] = row[tc + v] * ip;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) cv[u] = col[tr + u];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) m[u][v] = __builtin_fma(-cv[u], rv[v], m[u][v]);
+      if (tc == c4)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) m[u][q] = -cv[u] * ip;
+      if (tr == c4)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) m[q][v] = tc + v == c ? ip : rv[v];
+    }
+  if (threadIdx.x == 0 && !ok) *bad = 1;
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) Dinv[(tr + u) * kBJ + tc + v] = m[u][v];
+}
+
+__global__ __launch_bounds__(256) void k_bj_diag(const double* W, int np, int k0, const double* __restrict__ B, int n,
+                                                 double* Dinv, int* bad) {
+  __shared__ BjDiag s;
+  bj_diag(s, W, np, k0, B, n, Dinv, bad);
+}
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+// acc (32 x 32 per wavefront, as 2 x 2 MFMA tiles) += a (rows) x b (columns), 64 deep, both in LDS.
+__device__ inline void bj_mma(const double* a, const double* b, int lane, f64x4 (&acc)[2][2]) {
+  const int l16 = lane & 15, l4 = lane >> 4;
+#pragma unroll 4
+  for (int k = 0; k < kBJ; k += 4) {
+    double fa[2], fb[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) fa[u] = a[(u * 16 + l16) * kBJA + k + l4];
+#pragma unroll
+    for (int v = 0; v < 2; ++v) fb[v] = b[(k + l4) * kBJB + v * 16 + l16];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int v = 0; v < 2; ++v) acc[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[u], fb[v], acc[u][v], 0, 0, 0);
+  }
+}
+
+// 64 x 64 tile of a row-major matrix into LDS rows of length `ls`.
+__device__ inline void bj_stage(const double* __restrict__ src, int64_t ld, double* dst, int ls) {
+  for (int q = threadIdx.x; q < kBJ * kBJ / 2; q += 256) {
+    const int r = q / (kBJ / 2), c = q % (kBJ / 2) * 2;
+    *reinterpret_cast<double2*>(dst + r * ls + c) = *reinterpret_cast<const double2*>(src + r * ld + c);
+  }
+}
+
+// Workgroup j < np / 64: R(:, j) = Dinv x W(k, j) (Dinv itself at j = k).
+// The others set tile i of block column k aside.
+__global__ __launch_bounds__(256) void k_bj_panel(const double* __restrict__ W, int np, int kt,
+                                                  const double* __restrict__ Dinv, double* __restrict__ R,
+                                                  double* __restrict__ Cw) {
+  __shared__ __attribute__((aligned(16))) double sa[kBJ * kBJA], sb[kBJ * kBJB];
+  const int nt = np / kBJ;
+  if ((int)blockIdx.x >= nt) {
+    const int64_t i0 = (int64_t)(blockIdx.x - nt) * kBJ;
+    for (int q = threadIdx.x; q < kBJ * kBJ / 2; q += 256) {
+      const int r = q / (kBJ / 2), c = q % (kBJ / 2) * 2;
+      *reinterpret_cast<double2*>(Cw + (i0 + r) * kBJ + c) =
+          *reinterpret_cast<const double2*>(W + (i0 + r) * np + (int64_t)kt * kBJ + c);
+    }
+    return;
+  }
+  const int j0 = blockIdx.x * kBJ;
+  if ((int)blockIdx.x == kt) {
+    for (int q = threadIdx.x; q < kBJ * kBJ; q += 256) R[(int64_t)(q / kBJ) * np + j0 + q % kBJ] = Dinv[q];
+    return;
+  }
+  bj_stage(Dinv, kBJ, sa, kBJA);
+  bj_stage(W + (int64_t)kt * kBJ * np + j0, np, sb, kBJB);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wr = wave / 2 * 32, wc = wave % 2 * 32;
+  f64x4 acc[2][2] = {};
+  bj_mma(sa + wr * kBJA, sb + wc, lane, acc);
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        R[(int64_t)(wr + u * 16 + 4 * r + (lane >> 4)) * np + j0 + wc + v * 16 + (lane & 15)] = acc[u][v][r];
+}
+
+// Tile (i, j): W(i, j) - Cw(i) x R(j), starting from 0 in block column k;
+// block row k becomes R. (D of the product: lane holds column lane % 16 of
+// rows 4 r + lane / 16.) The first workgroup has the next diagonal tile and
+// inverts it while the others work.
+__global__ __launch_bounds__(256) void k_bj_update(double* W, int np, int kt, const double* __restrict__ Cw,
+                                                   const double* __restrict__ R, const double* __restrict__ B, int n,
+                                                   double* Dinv, int* bad) {
+  __shared__ __attribute__((aligned(16))) double sa[kBJ * kBJA], sb[kBJ * kBJB];
+  const int nt = np / kBJ;
+  const int it = (blockIdx.y + kt + 1) % nt, jt = (blockIdx.x + kt + 1) % nt;
+  const int64_t i0 = (int64_t)it * kBJ, j0 = (int64_t)jt * kBJ;
+  if (it == kt) {
+    for (int q = threadIdx.x; q < kBJ * kBJ / 2; q += 256) {
+      const int r = q / (kBJ / 2), c = q % (kBJ / 2) * 2;
+      *reinterpret_cast<double2*>(W + (i0 + r) * np + j0 + c) =
+          *reinterpret_cast<const double2*>(R + (int64_t)r * np + j0 + c);
+    }
+    return;
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wr = wave / 2 * 32, wc = wave % 2 * 32;
+  double* w = W + (i0 + wr + (lane >> 4)) * np + j0 + wc + (lane & 15);
+  f64x4 old[2][2] = {}, acc[2][2] = {};
+  if (jt != kt)
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int v = 0; v < 2; ++v)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) old[u][v][r] = w[(int64_t)(u * 16 + 4 * r) * np + v * 16];
+  bj_stage(Cw + i0 * kBJ, kBJ, sa, kBJA);
+  bj_stage(R + j0, np, sb, kBJB);
+  __syncthreads();
+  bj_mma(sa + wr * kBJA, sb + wc, lane, acc);
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) w[(int64_t)(u * 16 + 4 * r) * np + v * 16] = old[u][v][r] - acc[u][v][r];
+  if (blockIdx.x == 0 && blockIdx.y == 0 && kt + 1 < nt) {
+    __syncthreads();  // the tile is stored, sa is free
+    bj_diag(*reinterpret_cast<BjDiag*>(sa), W, np, (kt + 1) * kBJ, B, n, Dinv, bad);
+  }
+}
+
+// C = B^-1 without pivots; false when a pivot was not safely positive (C is then undefined).
+static bool invert_definite(Ctx& c, const double* B, double* C, int n) {
+  hipStream_t st = c.stream;
+  const int nt = div_up(n, kBJ), np = nt * kBJ;
+  DBuf<double> W, R, Cw, Dinv;
+  DBuf<int> bad;
+  W.alloc((size_t)np * np);
+  R.alloc((size_t)kBJ * np);
+  Cw.alloc((size_t)kBJ * np);
+  Dinv.alloc(kBJ * kBJ);
+  bad.alloc(1);
+  FOPIS_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), st));
+  k_bj_load<<<div_up((int64_t)np * np, 256), 256, 0, st>>>(B, n, W.p, np);
+  k_bj_diag<<<1, 256, 0, st>>>(W.p, np, 0, B, n, Dinv.p, bad.p);
+  for (int k = 0; k < nt; ++k) {
+    k_bj_panel<<<2 * nt, 256, 0, st>>>(W.p, np, k, Dinv.p, R.p, Cw.p);
+    k_bj_update<<<dim3(nt, nt), 256, 0, st>>>(W.p, np, k, Cw.p, R.p, B, n, Dinv.p, bad.p);
+  }
+  k_bj_store<<<div_up((int64_t)n * n, 256), 256, 0, st>>>(W.p, np, C, n);
+  FOPIS_HIP(hipGetLastError());
+  int h = 0;
+  FOPIS_HIP(hipMemcpyAsync(&h, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
+  FOPIS_HIP(hipStreamSynchronize(st));
+  return h == 0;
 }
 
 void objects_build_cmatrix(Ctx& c, int o) {
@@ -533,7 +785,8 @@ void objects_build_cmatrix(Ctx& c, int o) {
   B.alloc((size_t)n * n);
   const char* sp = std::getenv("FOPIS_CMAT_SPECTRAL");
   const bool spectral = !(sp && sp[0] == '0');  // FOPIS_CMAT_SPECTRAL=0: one solve per node
-  if (!spectral || !spectral_unit_responses(c, ob, B.p)) {
+  const bool definite = spectral && spectral_unit_responses(c, ob, B.p);
+  if (!definite) {
     // one unit-charge multigrid solve per surface node (RootGridObject.cpp:102-125)
     std::vector<int64_t> nodes(n);
     FOPIS_HIP(hipMemcpy(nodes.data(), ob.cmat_node.p, n * sizeof(int64_t), hipMemcpyDeviceToHost));
@@ -549,7 +802,12 @@ void objects_build_cmatrix(Ctx& c, int o) {
     // the reference leaves phi and rho cleared after the unit solves (RootGridObject.cpp:83-85)
     k_zero_d<<<div_up(nn, 256), 256, 0, st>>>(c.phi.p, nn);
   }
-  // C = B^-1 by Gauss-Jordan with partial pivoting
+  if (definite && invert_definite(c, B.p, ob.C.p, n)) {
+    finish_cmatrix(c, ob);
+    return;
+  }
+  // C = B^-1 by Gauss-Jordan with partial pivoting: B from the solves, which
+  // Neumann faces or nodes on a face leave unsymmetric, or a B that is not definite
   k_identity<<<div_up((int64_t)n * n, 256), 256, 0, st>>>(ob.C.p, n);
   DBuf<double> f;
   f.alloc(n + 2);

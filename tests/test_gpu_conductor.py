@@ -81,6 +81,35 @@ def test_cmatrix_device_build_is_inverse_of_exact_b(tmp_path, shape):
     np.testing.assert_allclose(Cm, Cm.T, rtol=1e-8, atol=1e-8 * np.abs(Cx).max())
 
 
+@pytest.mark.parametrize("n,dup", [(1, False), (63, False), (64, False), (65, False), (200, False), (70, True)])
+def test_cmatrix_tile_edges(n, dup):
+    """Node counts around the inversion's 64-wide tiles, on scattered nodes of
+    an uneven grid; a node given twice makes B singular, which the call
+    completes on as the pivoted elimination does (its values mean nothing)."""
+    dims = (14, 11, 18)
+    ctx = F.Context(F.make_desc(*dims, [(-1.0, 1.0, 1.0)], 2.5, mg_precision=F.FP64))
+    rng = np.random.default_rng(n)
+    inner = np.stack(np.meshgrid(*[np.arange(2, v) for v in dims], indexing="ij"), -1).reshape(-1, 3)
+    nodes = inner[rng.permutation(len(inner))[:n]].astype(np.int32)
+    if dup:
+        nodes[-1] = nodes[0]
+    mask = np.zeros([v + 1 for v in dims], np.uint8)
+    mask[5, 5, 5] = 1
+    ctx.set_object(0, mask, nodes)
+    ctx.build_cmatrix(0)
+    Cm = ctx.get_cmatrix(0)
+    if dup:
+        return
+    B = np.zeros((n, n))
+    for j in range(n):
+        b = np.zeros([v - 2 for v in dims])
+        b[tuple(nodes[j] - 2)] = 1.0 / 2.5
+        B[j] = dst_poisson(b)[tuple((nodes - 2).T)]
+    Cx = np.linalg.inv(B)
+    # FP64 elimination of a positive definite B: a few n eps cond(B), cond < 1e3 here
+    assert np.max(np.abs(Cm - Cx)) <= 1e-11 * np.max(np.abs(Cx))
+
+
 @pytest.mark.parametrize("nx", [17, 41])
 def test_capture_charge_and_current(nx):
     """At nx = 41 most tiles lie more than a tile away from the cube and skip
