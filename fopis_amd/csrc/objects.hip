@@ -116,21 +116,21 @@ __global__ void k_gj_elim(double* A, double* I, int n, int c, const double* f) {
   I[(size_t)r * n + q] -= fr * I[(size_t)c * n + q];
 }
 
-// colsum[j] = sum_i C(i,j): 64 columns per workgroup, each of its 16
-// wavefronts adds a sixteenth of the rows, their sums are added in row order
-// (a thread per column alone kept 7 workgroups busy for 1538 dependent rows)
-__global__ __launch_bounds__(1024) void k_colsum(const double* C, int n, double* colsum) {
-  __shared__ double sh[16][64];
-  const int j = blockIdx.x * 64 + (threadIdx.x & 63), w = threadIdx.x >> 6;
-  const int i0 = (int)((int64_t)n * w / 16), i1 = (int)((int64_t)n * (w + 1) / 16);
+// colsum[j] = sum_i C(i,j) (i ascending) and the Cmatrix::total order: a
+// thread per column, its next 16 loads in flight while the last are added
+__global__ void k_colsum(const double* C, int n, double* colsum) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= n) return;
   double s = 0.0;
-  if (j < n)
-#pragma unroll 8
-    for (int i = i0; i < i1; ++i) s += C[(size_t)i * n + j];
-  sh[w][threadIdx.x & 63] = s;
-  __syncthreads();
-  if (w != 0 || j >= n) return;
-  for (int q = 1; q < 16; ++q) s += sh[q][threadIdx.x];
+  int i = 0;
+  for (; i + 16 <= n; i += 16) {
+    double v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = C[(size_t)(i + u) * n + j];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) s += v[u];
+  }
+  for (; i < n; ++i) s += C[(size_t)i * n + j];
   colsum[j] = s;
 }
 
@@ -345,7 +345,7 @@ int objects_lit_nodes(Ctx& c, int o, int axis, int sign, const int32_t** dev_ijk
 
 static void finish_cmatrix(Ctx& c, ObjectDev& ob) {
   const int n = ob.ncmat;
-  k_colsum<<<div_up(n, 64), 1024, 0, c.stream>>>(ob.C.p, n, ob.colsum.p);
+  k_colsum<<<div_up(n, 64), 64, 0, c.stream>>>(ob.C.p, n, ob.colsum.p);
   k_total<<<1, 256, 0, c.stream>>>(ob.colsum.p, n, ob.scal.p + 3);
   FOPIS_HIP(hipMemcpyAsync(&ob.total_cmat, ob.scal.p + 3, sizeof(double), hipMemcpyDeviceToHost, c.stream));
   FOPIS_HIP(hipStreamSynchronize(c.stream));
@@ -548,26 +548,32 @@ static bool spectral_unit_responses(Ctx& c, ObjectDev& ob, double* B) {
 
 // ---- C = B^-1 for the sine-transform responses
 //
-// That B is a principal block of A^-1, symmetric and positive definite, so its
-// inverse needs no pivots. Blocked Gauss-Jordan in place on a copy padded to
-// whole 64 x 64 tiles (the padding is the identity): per block column, the
-// block row is multiplied by the diagonal tile's inverse and the block column
-// set aside (k_bj_panel), and every other tile takes one 64-deep product
-// (k_bj_update, v_mfma_f64_16x16x4), the first of them inverting the next
-// diagonal tile behind the others. The matrix is read and written once per 64
-// columns instead of once per column, by 2 launches instead of 256: 1538 nodes 36 -> 1.2 ms (bound by the 64 serial
-// steps of the diagonal tiles, 25 us each), the whole build at 6146 nodes
-// 1.6 s -> 42 ms (bound by the tiles' traffic). A pivot
-// that is not safely positive (surface nodes given twice) sets *bad, and the
-// caller falls back on the pivoted elimination.
+// That B is a Green's function of the walk that the Dirichlet faces stop, and
+// so is what remains of it after each elimination step: its columns peak on
+// the diagonal, and the pivoted Gauss-Jordan below never exchanges rows. Its
+// steps are then done in place (the unit columns of the n x 2n form are not
+// stored), 64 columns at a time, every element taking the same products,
+// quotients and differences in the same order, so C is the same bit for bit:
+// per block column k, the diagonal tile goes through its 64 steps alone
+// (k_bj_diag), which gives the scaled pivot row and the pivot column of each
+// step inside the tile; the tiles of block column k and of block row k follow
+// them (k_bj_panel), which gives the factors of their rows and their scaled
+// pivot rows; and every other tile subtracts its 64 products in order
+// (k_bj_update), the first of them also taking the next diagonal tile through
+// its steps, behind the others. The matrix is read and written once per 64
+// columns instead of twice over per column, by 2 launches instead of 256:
+// 1538 nodes 36 -> 2.1 ms (bound by the serial steps of the diagonal tiles and
+// the tiles beside them), the whole build at 6146 nodes 1.6 s -> 50 ms. Where a
+// step would have exchanged rows (nodes given twice) *bad is set, and the
+// caller runs the pivoted elimination.
 constexpr int kBJ = 64;
-constexpr int kBJA = 68, kBJB = 80;  // LDS row lengths: the fragment reads then spread over the banks
+constexpr int kBJL = 66;  // LDS row length (16-byte rows off the same banks)
 
 __global__ void k_bj_load(const double* __restrict__ B, int n, double* __restrict__ W, int np) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (int64_t)np * np) return;
   const int r = (int)(i / np), c = (int)(i % np);
-  W[i] = r < n && c < n ? B[(int64_t)r * n + c] : (r == c ? 1.0 : 0.0);
+  W[i] = r < n && c < n ? B[(int64_t)r * n + c] : (r == c ? 1.0 : 0.0);  // (identity in the last tile's rest)
 }
 
 __global__ void k_bj_store(const double* __restrict__ W, int np, double* __restrict__ C, int n) {
@@ -576,25 +582,28 @@ __global__ void k_bj_store(const double* __restrict__ W, int np, double* __restr
   C[i] = W[(i / n) * np + i % n];
 }
 
-// Inverse of the diagonal tile at k0 by one workgroup: every thread holds a
-// 4 x 4 piece, and each elimination step passes its row and column through
-// LDS (two pairs of buffers, so one barrier a step).
-struct BjDiag {
-  double row[2][kBJ], col[2][kBJ], diag[kBJ];
+// What the steps of a diagonal tile leave for the other tiles: step c's pivot,
+// its scaled row and its column before the step (by step, then column or row).
+struct BjSteps {
+  double d[kBJ], p[kBJ][kBJ], f[kBJ][kBJ];
 };
 
-__device__ void bj_diag(BjDiag& s, const double* W, int np, int k0, const double* __restrict__ B, int n, double* Dinv,
-                        int* bad) {
-  const int tr = threadIdx.x / 16 * 4, tc = threadIdx.x % 16 * 4;
-  double m[4][4];
+struct BjDiag {
+  double row[2][kBJ], col[2][kBJ];
+};
+
+// The diagonal tile at k0 by one workgroup: every thread holds a 4 x 4 piece.
+// A row's 16 threads are neighbouring lanes, so step c's pivot reaches them
+// without a barrier; they divide the row, and it goes with the column through
+// LDS (two pairs of buffers, one barrier a step). What the steps leave stays in
+// registers until the end: a barrier waits for the stores before it.
+__device__ void bj_diag(BjDiag& s, double* W, int np, int k0, BjSteps* out, int* bad) {
+  const int tr = threadIdx.x / 16 * 4, tc = threadIdx.x % 16 * 4, lane = threadIdx.x & 63;
+  double m[4][4], kf[4][4], kp[4][4];
 #pragma unroll
   for (int u = 0; u < 4; ++u)
 #pragma unroll
     for (int v = 0; v < 4; ++v) m[u][v] = W[(int64_t)(k0 + tr + u) * np + k0 + tc + v];
-  if (threadIdx.x < kBJ) {
-    const int d = k0 + threadIdx.x;
-    s.diag[threadIdx.x] = d < n ? B[(int64_t)d * n + d] : 1.0;
-  }
   bool ok = true;
   for (int c4 = 0; c4 < kBJ; c4 += 4)
 #pragma unroll
@@ -602,170 +611,174 @@ __device__ void bj_diag(BjDiag& s, const double* W, int np, int k0, const double
       const int c = c4 + q;
       double* row = s.row[q & 1];
       double* col = s.col[q & 1];
-      if (tr == c4)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) row[tc + v] = m[q][v];
       if (tc == c4)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) col[tr + u] = m[u][q];
+        for (int u = 0; u < 4; ++u) {
+          col[tr + u] = m[u][q];
+          kf[u][q] = m[u][q];
+        }
+      // (a row's 16 lanes take the branch together with the lane that holds the pivot)
+      if (tr == c4) {
+        const double d = __shfl(m[q][q], (lane & ~15) + c4 / 4, 64);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const double x = (tc + v == c ? 1.0 : m[q][v]) / d;
+          row[tc + v] = x;
+          kp[q][v] = x;
+        }
+      }
       __syncthreads();
-      const double p = row[c];
-      ok = ok && p > 1e-13 * s.diag[c];
-      const double ip = 1.0 / p;
       double rv[4], cv[4];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) rv[v] = row[tc + v] * ip;
+      for (int v = 0; v < 4; ++v) rv[v] = row[tc + v];
 #pragma unroll
       for (int u = 0; u < 4; ++u) cv[u] = col[tr + u];
+      const double d = col[c];
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) m[u][v] = __builtin_fma(-cv[u], rv[v], m[u][v]);
+        for (int v = 0; v < 4; ++v) m[u][v] = m[u][v] - cv[u] * rv[v];
       if (tc == c4)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) m[u][q] = -cv[u] * ip;
+        for (int u = 0; u < 4; ++u) {
+          ok = ok && (tr + u <= c || fabs(cv[u]) <= fabs(d));
+          m[u][q] = 0.0 - cv[u] * rv[q];
+        }
       if (tr == c4)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) m[q][v] = tc + v == c ? ip : rv[v];
+        for (int v = 0; v < 4; ++v) m[q][v] = rv[v];
     }
-  if (threadIdx.x == 0 && !ok) *bad = 1;
+  if (!ok) *bad = 1;
 #pragma unroll
   for (int u = 0; u < 4; ++u)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) Dinv[(tr + u) * kBJ + tc + v] = m[u][v];
-}
-
-__global__ __launch_bounds__(256) void k_bj_diag(const double* W, int np, int k0, const double* __restrict__ B, int n,
-                                                 double* Dinv, int* bad) {
-  __shared__ BjDiag s;
-  bj_diag(s, W, np, k0, B, n, Dinv, bad);
-}
-
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-
-// acc (32 x 32 per wavefront, as 2 x 2 MFMA tiles) += a (rows) x b (columns), 64 deep, both in LDS.
-__device__ inline void bj_mma(const double* a, const double* b, int lane, f64x4 (&acc)[2][2]) {
-  const int l16 = lane & 15, l4 = lane >> 4;
-#pragma unroll 4
-  for (int k = 0; k < kBJ; k += 4) {
-    double fa[2], fb[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) fa[u] = a[(u * 16 + l16) * kBJA + k + l4];
-#pragma unroll
-    for (int v = 0; v < 2; ++v) fb[v] = b[(k + l4) * kBJB + v * 16 + l16];
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int v = 0; v < 2; ++v) acc[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[u], fb[v], acc[u][v], 0, 0, 0);
-  }
-}
-
-// 64 x 64 tile of a row-major matrix into LDS rows of length `ls`.
-__device__ inline void bj_stage(const double* __restrict__ src, int64_t ld, double* dst, int ls) {
-  for (int q = threadIdx.x; q < kBJ * kBJ / 2; q += 256) {
-    const int r = q / (kBJ / 2), c = q % (kBJ / 2) * 2;
-    *reinterpret_cast<double2*>(dst + r * ls + c) = *reinterpret_cast<const double2*>(src + r * ld + c);
-  }
-}
-
-// Workgroup j < np / 64: R(:, j) = Dinv x W(k, j) (Dinv itself at j = k).
-// The others set tile i of block column k aside.
-__global__ __launch_bounds__(256) void k_bj_panel(const double* __restrict__ W, int np, int kt,
-                                                  const double* __restrict__ Dinv, double* __restrict__ R,
-                                                  double* __restrict__ Cw) {
-  __shared__ __attribute__((aligned(16))) double sa[kBJ * kBJA], sb[kBJ * kBJB];
-  const int nt = np / kBJ;
-  if ((int)blockIdx.x >= nt) {
-    const int64_t i0 = (int64_t)(blockIdx.x - nt) * kBJ;
-    for (int q = threadIdx.x; q < kBJ * kBJ / 2; q += 256) {
-      const int r = q / (kBJ / 2), c = q % (kBJ / 2) * 2;
-      *reinterpret_cast<double2*>(Cw + (i0 + r) * kBJ + c) =
-          *reinterpret_cast<const double2*>(W + (i0 + r) * np + (int64_t)kt * kBJ + c);
+    for (int v = 0; v < 4; ++v) {
+      W[(int64_t)(k0 + tr + u) * np + k0 + tc + v] = m[u][v];
+      out->f[tc + v][tr + u] = kf[u][v];  // step tc + v, row tr + u
+      out->p[tr + u][tc + v] = kp[u][v];  // step tr + u, column tc + v
+      if (tr + u == tc + v) out->d[tc + v] = kf[u][v];
     }
-    return;
-  }
-  const int j0 = blockIdx.x * kBJ;
-  if ((int)blockIdx.x == kt) {
-    for (int q = threadIdx.x; q < kBJ * kBJ; q += 256) R[(int64_t)(q / kBJ) * np + j0 + q % kBJ] = Dinv[q];
-    return;
-  }
-  bj_stage(Dinv, kBJ, sa, kBJA);
-  bj_stage(W + (int64_t)kt * kBJ * np + j0, np, sb, kBJB);
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wr = wave / 2 * 32, wc = wave % 2 * 32;
-  f64x4 acc[2][2] = {};
-  bj_mma(sa + wr * kBJA, sb + wc, lane, acc);
-#pragma unroll
-  for (int u = 0; u < 2; ++u)
-#pragma unroll
-    for (int v = 0; v < 2; ++v)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        R[(int64_t)(wr + u * 16 + 4 * r + (lane >> 4)) * np + j0 + wc + v * 16 + (lane & 15)] = acc[u][v][r];
 }
 
-// Tile (i, j): W(i, j) - Cw(i) x R(j), starting from 0 in block column k;
-// block row k becomes R. (D of the product: lane holds column lane % 16 of
-// rows 4 r + lane / 16.) The first workgroup has the next diagonal tile and
-// inverts it while the others work.
-__global__ __launch_bounds__(256) void k_bj_update(double* W, int np, int kt, const double* __restrict__ Cw,
-                                                   const double* __restrict__ R, const double* __restrict__ B, int n,
-                                                   double* Dinv, int* bad) {
-  __shared__ __attribute__((aligned(16))) double sa[kBJ * kBJA], sb[kBJ * kBJB];
+__global__ __launch_bounds__(256) void k_bj_diag(double* W, int np, int k0, BjSteps* out, int* bad) {
+  __shared__ BjDiag s;
+  bj_diag(s, W, np, k0, out, bad);
+}
+
+// The tiles beside a diagonal tile, one per workgroup: a line (a row of block
+// column k, a column of block row k) is held by four neighbouring lanes, 16
+// elements each; the lane that holds element c passes it on at step c.
+// Block column: the element is the row's factor f, every other element takes
+// f times the step's scaled row. Block row: the element is divided by the
+// pivot, every other element takes it times the step's column.
+__global__ __launch_bounds__(256) void k_bj_panel(double* __restrict__ W, int np, int kt,
+                                                  const BjSteps* __restrict__ st, double* __restrict__ F,
+                                                  double* __restrict__ V, int* bad) {
+  __shared__ __attribute__((aligned(16))) double step[kBJ][kBJ], piv[kBJ];
+  const int nt = np / kBJ;
+  const bool colblk = (int)blockIdx.x < nt;
+  const int t = colblk ? blockIdx.x : blockIdx.x - nt;
+  if (t == kt) return;
+  const double(*src)[kBJ] = colblk ? st->p : st->f;
+  for (int q = threadIdx.x; q < kBJ * kBJ; q += 256) step[q / kBJ][q % kBJ] = src[q / kBJ][q % kBJ];
+  if (threadIdx.x < kBJ) piv[threadIdx.x] = st->d[threadIdx.x];
+  __syncthreads();
+  const int line = threadIdx.x >> 2, g = threadIdx.x & 3, lane = threadIdx.x & 63;
+  double* w = colblk ? W + ((int64_t)t * kBJ + line) * np + (int64_t)kt * kBJ + 16 * g
+                     : W + ((int64_t)kt * kBJ + 16 * g) * np + (int64_t)t * kBJ + line;
+  const int64_t ws = colblk ? 1 : np;
+  double m[16], keep[16];
+#pragma unroll
+  for (int u = 0; u < 16; ++u) m[u] = w[u * ws];
+  bool ok = true;
+  for (int b = 0; b < 4; ++b) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int c = 16 * b + q;
+      const double d = piv[c];
+      const double own = colblk ? m[q] : m[q] / d;
+      const double f = __shfl(own, (lane & ~3) + b, 64);
+      if (colblk && t > kt) ok = ok && fabs(f) <= fabs(d);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) m[u] = m[u] - f * step[c][16 * g + u];
+      if (g == b) {
+        keep[q] = f;
+        m[q] = colblk ? 0.0 - f * step[c][c] : f;
+      }
+    }
+  }
+  if (!ok) *bad = 1;
+  // the line's elements, and what it passed on in its own 16 steps
+  double* o = colblk ? F + ((int64_t)t * kBJ + line) * kBJ + 16 * g : V + (int64_t)(16 * g) * np + (int64_t)t * kBJ + line;
+  const int64_t os = colblk ? 1 : np;
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    w[u * ws] = m[u];
+    o[u * os] = keep[u];
+  }
+}
+
+// Tile (i, j) off block row and column k: the 64 products of its rows' factors
+// and the scaled pivot rows, in step order.
+__global__ __launch_bounds__(256) void k_bj_update(double* W, int np, int kt, const double* __restrict__ F,
+                                                   const double* __restrict__ V, BjSteps* next, int* bad) {
+  __shared__ __attribute__((aligned(16))) double sf[kBJ][kBJL], sv[kBJ][kBJ];
   const int nt = np / kBJ;
   const int it = (blockIdx.y + kt + 1) % nt, jt = (blockIdx.x + kt + 1) % nt;
-  const int64_t i0 = (int64_t)it * kBJ, j0 = (int64_t)jt * kBJ;
-  if (it == kt) {
-    for (int q = threadIdx.x; q < kBJ * kBJ / 2; q += 256) {
-      const int r = q / (kBJ / 2), c = q % (kBJ / 2) * 2;
-      *reinterpret_cast<double2*>(W + (i0 + r) * np + j0 + c) =
-          *reinterpret_cast<const double2*>(R + (int64_t)r * np + j0 + c);
-    }
-    return;
+  if (it == kt || jt == kt) return;
+  const int tr = threadIdx.x / 16 * 4, tc = threadIdx.x % 16 * 4;
+  double* w = W + ((int64_t)it * kBJ + tr) * np + (int64_t)jt * kBJ + tc;
+  double m[4][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) m[u][v] = w[(int64_t)u * np + v];
+  for (int q = threadIdx.x; q < kBJ * kBJ; q += 256) {
+    const int a = q / kBJ, b = q % kBJ;
+    sf[b][a] = F[((int64_t)it * kBJ + a) * kBJ + b];  // (by step, then row)
+    sv[a][b] = V[(int64_t)a * np + (int64_t)jt * kBJ + b];
   }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wr = wave / 2 * 32, wc = wave % 2 * 32;
-  double* w = W + (i0 + wr + (lane >> 4)) * np + j0 + wc + (lane & 15);
-  f64x4 old[2][2] = {}, acc[2][2] = {};
-  if (jt != kt)
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int v = 0; v < 2; ++v)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) old[u][v][r] = w[(int64_t)(u * 16 + 4 * r) * np + v * 16];
-  bj_stage(Cw + i0 * kBJ, kBJ, sa, kBJA);
-  bj_stage(R + j0, np, sb, kBJB);
   __syncthreads();
-  bj_mma(sa + wr * kBJA, sb + wc, lane, acc);
+#pragma unroll 4
+  for (int c = 0; c < kBJ; ++c) {
+    double f[4], v[4];
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < 4; ++u) f[u] = sf[c][tr + u];
 #pragma unroll
-    for (int v = 0; v < 2; ++v)
+    for (int u = 0; u < 4; ++u) v[u] = sv[c][tc + u];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) w[(int64_t)(u * 16 + 4 * r) * np + v * 16] = old[u][v][r] - acc[u][v][r];
-  if (blockIdx.x == 0 && blockIdx.y == 0 && kt + 1 < nt) {
-    __syncthreads();  // the tile is stored, sa is free
-    bj_diag(*reinterpret_cast<BjDiag*>(sa), W, np, (kt + 1) * kBJ, B, n, Dinv, bad);
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) m[u][x] = m[u][x] - f[u] * v[x];
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) w[(int64_t)u * np + v] = m[u][v];
+  if (blockIdx.x == 0 && blockIdx.y == 0) {  // (it == jt == kt + 1 while there is such a tile)
+    __syncthreads();  // the tile is stored, sf is free
+    if (kt + 1 < nt) bj_diag(*reinterpret_cast<BjDiag*>(sf), W, np, (kt + 1) * kBJ, next, bad);
   }
 }
 
-// C = B^-1 without pivots; false when a pivot was not safely positive (C is then undefined).
-static bool invert_definite(Ctx& c, const double* B, double* C, int n) {
+// C = B^-1 without exchanging rows; false where that would have happened (C is then undefined).
+static bool invert_in_order(Ctx& c, const double* B, double* C, int n) {
   hipStream_t st = c.stream;
   const int nt = div_up(n, kBJ), np = nt * kBJ;
-  DBuf<double> W, R, Cw, Dinv;
+  DBuf<double> W, F, V;
+  DBuf<BjSteps> steps;
   DBuf<int> bad;
   W.alloc((size_t)np * np);
-  R.alloc((size_t)kBJ * np);
-  Cw.alloc((size_t)kBJ * np);
-  Dinv.alloc(kBJ * kBJ);
+  F.alloc((size_t)kBJ * np);
+  V.alloc((size_t)kBJ * np);
+  steps.alloc(2);
   bad.alloc(1);
   FOPIS_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), st));
   k_bj_load<<<div_up((int64_t)np * np, 256), 256, 0, st>>>(B, n, W.p, np);
-  k_bj_diag<<<1, 256, 0, st>>>(W.p, np, 0, B, n, Dinv.p, bad.p);
+  k_bj_diag<<<1, 256, 0, st>>>(W.p, np, 0, steps.p, bad.p);
   for (int k = 0; k < nt; ++k) {
-    k_bj_panel<<<2 * nt, 256, 0, st>>>(W.p, np, k, Dinv.p, R.p, Cw.p);
-    k_bj_update<<<dim3(nt, nt), 256, 0, st>>>(W.p, np, k, Cw.p, R.p, B, n, Dinv.p, bad.p);
+    k_bj_panel<<<2 * nt, 256, 0, st>>>(W.p, np, k, steps.p + (k & 1), F.p, V.p, bad.p);
+    if (nt > 1) k_bj_update<<<dim3(nt, nt), 256, 0, st>>>(W.p, np, k, F.p, V.p, steps.p + ((k + 1) & 1), bad.p);
   }
   k_bj_store<<<div_up((int64_t)n * n, 256), 256, 0, st>>>(W.p, np, C, n);
   FOPIS_HIP(hipGetLastError());
@@ -785,8 +798,8 @@ void objects_build_cmatrix(Ctx& c, int o) {
   B.alloc((size_t)n * n);
   const char* sp = std::getenv("FOPIS_CMAT_SPECTRAL");
   const bool spectral = !(sp && sp[0] == '0');  // FOPIS_CMAT_SPECTRAL=0: one solve per node
-  const bool definite = spectral && spectral_unit_responses(c, ob, B.p);
-  if (!definite) {
+  const bool peaked = spectral && spectral_unit_responses(c, ob, B.p);
+  if (!peaked) {
     // one unit-charge multigrid solve per surface node (RootGridObject.cpp:102-125)
     std::vector<int64_t> nodes(n);
     FOPIS_HIP(hipMemcpy(nodes.data(), ob.cmat_node.p, n * sizeof(int64_t), hipMemcpyDeviceToHost));
@@ -802,12 +815,12 @@ void objects_build_cmatrix(Ctx& c, int o) {
     // the reference leaves phi and rho cleared after the unit solves (RootGridObject.cpp:83-85)
     k_zero_d<<<div_up(nn, 256), 256, 0, st>>>(c.phi.p, nn);
   }
-  if (definite && invert_definite(c, B.p, ob.C.p, n)) {
+  if (peaked && invert_in_order(c, B.p, ob.C.p, n)) {
     finish_cmatrix(c, ob);
     return;
   }
-  // C = B^-1 by Gauss-Jordan with partial pivoting: B from the solves, which
-  // Neumann faces or nodes on a face leave unsymmetric, or a B that is not definite
+  // C = B^-1 by Gauss-Jordan with partial pivoting: B from the per-node solves
+  // (Neumann faces, nodes on a face), or one whose columns do not peak on the diagonal
   k_identity<<<div_up((int64_t)n * n, 256), 256, 0, st>>>(ob.C.p, n);
   DBuf<double> f;
   f.alloc(n + 2);

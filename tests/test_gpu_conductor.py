@@ -85,7 +85,8 @@ def test_cmatrix_device_build_is_inverse_of_exact_b(tmp_path, shape):
 def test_cmatrix_tile_edges(n, dup):
     """Node counts around the inversion's 64-wide tiles, on scattered nodes of
     an uneven grid; a node given twice makes B singular, which the call
-    completes on as the pivoted elimination does (its values mean nothing)."""
+    completes on as the pivoted elimination does (its values mean nothing).
+    C is the one-column-at-a-time elimination's, element by element."""
     dims = (14, 11, 18)
     ctx = F.Context(F.make_desc(*dims, [(-1.0, 1.0, 1.0)], 2.5, mg_precision=F.FP64))
     rng = np.random.default_rng(n)
@@ -108,6 +109,18 @@ def test_cmatrix_tile_edges(n, dup):
     Cx = np.linalg.inv(B)
     # FP64 elimination of a positive definite B: a few n eps cond(B), cond < 1e3 here
     assert np.max(np.abs(Cm - Cx)) <= 1e-11 * np.max(np.abs(Cx))
+    # the inverse of C in the same arithmetic: B's columns peak on the diagonal, C's do as well
+    M = Cm.copy()
+    I = np.eye(n)
+    for c in range(n):
+        assert np.argmax(np.abs(M[c:, c])) == 0
+        d = M[c, c]
+        M[c], I[c] = M[c] / d, I[c] / d
+        f = M[:, c].copy()
+        f[c] = 0.0
+        M -= f[:, None] * M[c]
+        I -= f[:, None] * I[c]
+    assert np.max(np.abs(I - B)) <= 1e-11 * np.max(np.abs(B))
 
 
 @pytest.mark.parametrize("nx", [17, 41])
