@@ -246,6 +246,11 @@ struct MgLevel {
   DBuf<float> e32, r32, t32;   // FP32 level arrays
 };
 
+// One level of the single-workgroup tail (see TailLv in poisson.hip).
+struct TailPlan {
+  int sx, sy, oe, orr, ot, count, red, list, fine, corner;
+};
+
 struct GuessNet;  // learned initial guess (guess.hip)
 
 struct Ctx {
@@ -320,13 +325,18 @@ struct Ctx {
   bool mg_rb = false;
   DBuf<float> erb, rrb;
   int64_t rb_cs = 0, rb_sx = 0, rb_sy = 0;
+  bool mg_fused = false;      // V(2,2): a level's half of a cycle runs as one launch (FOPIS_MG_FUSED=0: separate passes)
   bool mg_use_graph = true;   // replay the captured cycle (FOPIS_MG_GRAPH=0 launches it kernel by kernel)
   DBuf<double> mg_r64;        // FP64 level-0 residual when the V-cycle is FP32
   int mg_hist[2] = {1, 1};    // cycles of the last two solves (batch size of the next)
   int mg_tail = 0;            // first level solved by the single-workgroup LDS kernel
   size_t mg_tail_bytes = 0;   // its LDS bytes
   size_t mg_tail_esz = 0;     // element size the tail was planned for
-  bool mg_tail15 = false;     // the tail is the cubic 15 -> 7 -> 3 -> 1 chain
+  std::vector<TailPlan> mg_tail_plan;  // its levels
+  bool mg_tail15 = false;              // it is the cubic 15 -> 7 -> 3 -> 1 chain
+  int mg_tail_elems = 0;               // LDS elements of its arrays
+  DBuf<uint16_t> mg_tail_tab;          // its point lists
+  DBuf<int32_t> mg_tail_idx;           // its first level's points in that level's array
   size_t lds_max = 65536;     // LDS bytes per workgroup on the device
   GuessNet* guess = nullptr;  // owned; released by guess_free
 

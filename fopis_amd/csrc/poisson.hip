@@ -734,6 +734,269 @@ __global__ __launch_bounds__(256) void k_pair_resid_rb(Rb R, Lv L, double* part,
   }
 }
 
+// ---- a level's smoothing with its transfer in one launch
+//
+// One V(2,2) visit of a level was about ten launches of 4-6 us (first sweep,
+// half-sweeps, residual, restriction, prolongation), each reading the level
+// again. Here a workgroup holds a tile of the level with a halo in LDS and does
+// the whole downward half (two sweeps, residual, full weighting) or the whole
+// upward half (interpolation, two sweeps) on it, recomputing the halo its
+// neighbours also compute: every half-sweep narrows the valid region by one
+// point. All sums are those of the separate kernels, in their order, so the
+// result is the same bit for bit. The upward half reads its neighbours' points,
+// so it writes to the level's second array; the downward half reads nothing
+// but the right-hand side when it starts from zero.
+//
+// Halo points beyond the interior stay 0, as the levels' borders do. Tiles of
+// 8^3 points: a launch is a chain of ten phases of latency, which more
+// workgroups and fewer points each shorten. In a solve
+// the visit of a 31^3 level went from ten launches, 38 us, to two, 13 us, of a
+// 63^3 level from 40 to 19 us.
+constexpr int kTileEdge = 8;
+
+// q / D for 0 <= q <= MAXQ by one 24-bit product and a shift (the level
+// kernels are bound by vector instructions, and the compiler's division by a
+// constant takes a high product at a quarter of the rate).
+template <int D, int MAXQ>
+struct SmallDiv {
+  static constexpr bool fits(int s) {
+    const uint64_t m = ((1ull << s) + D - 1) / D;
+    return m < (1u << 24) && MAXQ < (1 << 24) && (uint64_t)MAXQ * m < (1ull << 32) &&
+           (uint64_t)MAXQ * (m * D - (1ull << s)) < (1ull << s);
+  }
+  static constexpr int shift() {
+    int s = 4;
+    while (s < 31 && !fits(s)) ++s;
+    return s;
+  }
+  static constexpr int S = shift();
+  static_assert(fits(S), "no exact multiplier");
+  static constexpr uint32_t M = (uint32_t)(((1ull << S) + D - 1) / D);
+  static __device__ inline int div(int q) { return (int)(__umul24((uint32_t)q, M) >> S); }
+};
+
+// (a, b, c) of point q of an NA x NB x NC box in row order.
+template <int NA, int NB, int NC>
+__device__ inline void box_point(int q, int& a, int& b, int& c) {
+  const int ab = SmallDiv<NC, NA * NB * NC + 2048>::div(q);
+  c = q - ab * NC;
+  a = SmallDiv<NB, NA * NB + 2048 / NC + 1>::div(ab);
+  b = ab - a * NB;
+}
+
+template <class P, bool ZERO>
+struct DownDim {
+  static constexpr int kLo = ZERO ? 4 : 5;               // halo below the tile's first point
+  static constexpr int N = kTileEdge + 2 * kLo + 1;      // points per axis
+  static constexpr int SB = N + (N & 1), SA = N * SB;    // row and plane length (SA even: the two colours' lanes
+  static constexpr size_t kLds = 2 * (size_t)N * SA * sizeof(P);  // then read different banks)
+  static_assert(SA % 2 == 0 && kLds <= 163840, "tile fits the LDS");
+};
+template <class P>
+struct UpDim {
+  static constexpr int kLo = 4, N = kTileEdge + 8, SB = N, SA = N * SB;
+  static constexpr int NC = N / 2 + 1, SCB = NC, SCA = NC * NC;  // the coarse points they interpolate from
+  static constexpr size_t kLds = (2 * (size_t)N * SA + (size_t)NC * SCA) * sizeof(P);
+  static_assert(SA % 2 == 0 && kLds <= 163840, "tile fits the LDS");
+};
+constexpr int kTileThreads = 1024;
+
+// The N^3 points of a tile with origin (oa, ob, oc) from a level array, 0
+// outside the level's border; all of a thread's loads are in flight at once
+// (a loop of one load and one LDS store an iteration spent the launch waiting:
+// the data come from another XCD's writes, past this one's L2).
+template <class P, int N, int SA, int SB, int NTHR>
+struct TileLoad {
+  static constexpr int IT = (N * N * N + NTHR - 1) / NTHR;
+  P v[IT];
+  __device__ inline void fetch(const P* __restrict__ src, const Lv& L, int oa, int ob, int oc) {
+#pragma unroll
+    for (int u = 0; u < IT; ++u) {
+      const int q = threadIdx.x + u * NTHR;
+      int a, b, c;
+      box_point<N, N, N>(q, a, b, c);
+      const int ga = oa + a, gb = ob + b, gc = oc + c;
+      v[u] = 0;
+      if ((unsigned)ga <= (unsigned)(L.n0 + 1) && (unsigned)gb <= (unsigned)(L.n1 + 1) &&
+          (unsigned)gc <= (unsigned)(L.n2 + 1) && q < N * N * N)
+        v[u] = src[ga * L.sx + gb * L.sy + gc];
+    }
+  }
+  __device__ inline void put(P* dst) const {
+#pragma unroll
+    for (int u = 0; u < IT; ++u) {
+      const int q = threadIdx.x + u * NTHR;
+      int a, b, c;
+      box_point<N, N, N>(q, a, b, c);
+      if (q < N * N * N) dst[a * SA + b * SB + c] = v[u];
+    }
+  }
+};
+
+// Red-black half-sweep (k_smooth) of the tile's points at least M from its
+// edge: a thread takes two points of the colour of one (b, c) column, their
+// reads before either's store.
+template <class P, int N, int SA, int SB, int M>
+__device__ inline void tile_smooth(P* e, const P* r, const Lv& L, int oa, int ob, int oc, int color, P w1, P w6) {
+  constexpr int W = N - 2 * M, PAIRS = (W + 3) / 4;
+  for (int q = threadIdx.x; q < PAIRS * W * W; q += kTileThreads) {
+    int s, b, c;
+    box_point<PAIRS, W, W>(q, s, b, c);
+    b += M;
+    c += M;
+    const int gb = ob + b, gc = oc + c;
+    if (gb < 1 || gb > L.n1 || gc < 1 || gc > L.n2) continue;
+    const int alo = max(M, 1 - oa), ahi = min(N - 1 - M, L.n0 - oa);
+    const int a = alo + ((oa + alo + gb + gc + color) & 1) + 4 * s;  // (ga + gb + gc) % 2 == color
+    if (a > ahi) continue;
+    P* p = e + a * SA + b * SB + c;
+    const P* rp = r + a * SA + b * SB + c;
+    const bool two = a + 2 <= ahi;
+    const int o = two ? 2 * SA : 0;  // (a lone point is read twice)
+    const P mid = p[SA];
+    const P n0 = p[-SA] + mid + p[-SB] + p[SB] + p[-1] + p[1];
+    const P n1 = mid + p[o + SA] + p[o - SB] + p[o + SB] + p[o - 1] + p[o + 1];
+    const P v0 = w1 * p[0] + w6 * (n0 + rp[0]);
+    const P v1 = w1 * p[o] + w6 * (n1 + rp[o]);
+    p[0] = v0;
+    if (two) p[2 * SA] = v1;
+  }
+}
+
+template <class P, bool ZERO>
+__global__ __launch_bounds__(kTileThreads) void k_level_down(P* __restrict__ eo, const P* __restrict__ ei,
+                                                                const P* __restrict__ r, Lv F, P* __restrict__ rc,
+                                                                Lv C, P w1, P w6, const int* __restrict__ done) {
+  if (*done) return;
+  using D = DownDim<P, ZERO>;
+  constexpr int N = D::N, SA = D::SA, SB = D::SB, T = kTileEdge, NT = kTileThreads, LO = D::kLo, M0 = ZERO ? 0 : 1;
+  extern __shared__ __attribute__((aligned(16))) char tile_lds[];
+  P* se = reinterpret_cast<P*>(tile_lds);
+  P* sr = se + N * SA;
+  int bx, by, bz;
+  block3(bx, by, bz);
+  const int s0 = bz * T + 1, s1 = by * T + 1, s2 = bx * T + 1;  // the tile's first point
+  const int oa = s0 - LO, ob = s1 - LO, oc = s2 - LO;
+  {
+    TileLoad<P, N, SA, SB, NT> lr;
+    lr.fetch(r, F, oa, ob, oc);
+    if constexpr (!ZERO) {
+      TileLoad<P, N, SA, SB, NT> le;
+      le.fetch(ei, F, oa, ob, oc);
+      le.put(se);
+    }
+    lr.put(sr);
+  }
+  __syncthreads();
+  if constexpr (ZERO) {
+    // red points of the first sweep from e = 0; black ones and the border 0
+    for (int q = threadIdx.x; q < N * SA; q += NT) {
+      int a, b, c;
+      box_point<N, N, SB>(q, a, b, c);
+      const bool red = ((oa + a + ob + b + oc + c) & 1) == 0;
+      const bool in = c < N && oa + a >= 1 && oa + a <= F.n0 && ob + b >= 1 && ob + b <= F.n1 && oc + c >= 1 &&
+                      oc + c <= F.n2;
+      se[q] = red && in ? w6 * sr[q] : (P)0;
+    }
+  } else {
+    tile_smooth<P, N, SA, SB, M0>(se, sr, F, oa, ob, oc, 0, w1, w6);
+  }
+  __syncthreads();
+  tile_smooth<P, N, SA, SB, M0 + 1>(se, sr, F, oa, ob, oc, 1, w1, w6);
+  __syncthreads();
+  tile_smooth<P, N, SA, SB, M0 + 2>(se, sr, F, oa, ob, oc, 0, w1, w6);
+  __syncthreads();
+  tile_smooth<P, N, SA, SB, M0 + 3>(se, sr, F, oa, ob, oc, 1, w1, w6);
+  __syncthreads();
+  // the tile's points out; the residual (over r, in place) of the tile and one point above
+  for (int q = threadIdx.x; q < (T + 1) * (T + 1) * (T + 1); q += NT) {
+    int a, b, c;
+    box_point<T + 1, T + 1, T + 1>(q, a, b, c);
+    const int g = (a + LO) * SA + (b + LO) * SB + c + LO;
+    const bool in = s0 + a <= F.n0 && s1 + b <= F.n1 && s2 + c <= F.n2;
+    const P e = se[g];
+    if (in) {
+      sr[g] = sr[g] - ((P)6 * e - (se[g - SA] + se[g + SA] + se[g - SB] + se[g + SB] + se[g - 1] + se[g + 1]));
+      if (a < T && b < T && c < T) eo[(s0 + a) * F.sx + (s1 + b) * F.sy + s2 + c] = e;
+    }
+  }
+  __syncthreads();
+  // full weighting (k_restrict_resid) at the coarse points inside the tile
+  constexpr int TC = T / 2;
+  for (int q = threadIdx.x; q < TC * TC * TC; q += NT) {
+    const int a = q / (TC * TC), b = (q / TC) % TC, c = q % TC;
+    const int A = s0 / 2 + 1 + a, B = s1 / 2 + 1 + b, Cc = s2 / 2 + 1 + c;  // fine 2A = s0 + 1 + 2a (s0 is odd)
+    if (A > C.n0 || B > C.n1 || Cc > C.n2) continue;
+    const int f = (2 * a + 1 + LO) * SA + (2 * b + 1 + LO) * SB + 2 * c + 1 + LO;
+    P acc = 0;
+#pragma unroll
+    for (int da = -1; da <= 1; ++da)
+#pragma unroll
+      for (int db = -1; db <= 1; ++db)
+#pragma unroll
+        for (int dc = -1; dc <= 1; ++dc) acc += fw_weight<P>(da, db, dc) * sr[f + da * SA + db * SB + dc];
+    rc[A * C.sx + B * C.sy + Cc] = acc * (P)0.5;  // (4/8) * sum
+  }
+}
+
+template <class P>
+__global__ __launch_bounds__(kTileThreads) void k_level_up(P* __restrict__ eo, const P* __restrict__ ei,
+                                                              const P* __restrict__ r, Lv F,
+                                                              const P* __restrict__ ec, Lv C, P w1, P w6,
+                                                              const int* __restrict__ done) {
+  if (*done) return;
+  using D = UpDim<P>;
+  constexpr int N = D::N, SA = D::SA, SB = D::SB, T = kTileEdge, NT = kTileThreads, LO = D::kLo;
+  extern __shared__ __attribute__((aligned(16))) char tile_lds[];
+  P* se = reinterpret_cast<P*>(tile_lds);
+  P* sr = se + N * SA;
+  P* sc = sr + N * SA;
+  int bx, by, bz;
+  block3(bx, by, bz);
+  const int s0 = bz * T + 1, s1 = by * T + 1, s2 = bx * T + 1;
+  const int oa = s0 - LO, ob = s1 - LO, oc = s2 - LO;
+  const int ca = oa >> 1, cb = ob >> 1, cc = oc >> 1;  // the first coarse point (floor: oa may be negative)
+  {
+    TileLoad<P, D::NC, D::SCA, D::SCB, NT> lc;
+    TileLoad<P, N, SA, SB, NT> le, lr;
+    lc.fetch(ec, C, ca, cb, cc);
+    le.fetch(ei, F, oa, ob, oc);
+    lr.fetch(r, F, oa, ob, oc);
+    lc.put(sc);
+    le.put(se);
+    lr.put(sr);
+  }
+  __syncthreads();
+  // e += trilinear interpolation of the coarse correction (k_prolong)
+  for (int q = threadIdx.x; q < N * N * N; q += NT) {
+    int a, b, c;
+    box_point<N, N, N>(q, a, b, c);
+    const int ga = oa + a, gb = ob + b, gc = oc + c;
+    if (ga < 1 || ga > F.n0 || gb < 1 || gb > F.n1 || gc < 1 || gc > F.n2) continue;
+    const int a0 = ((ga >> 1) - ca) * D::SCA, a1 = (((ga + 1) >> 1) - ca) * D::SCA;
+    const int b0 = ((gb >> 1) - cb) * D::SCB, b1 = (((gb + 1) >> 1) - cb) * D::SCB;
+    const int c0 = (gc >> 1) - cc, c1 = ((gc + 1) >> 1) - cc;
+    const P v = (sc[a0 + b0 + c0] + sc[a1 + b0 + c0] + sc[a0 + b1 + c0] + sc[a1 + b1 + c0] + sc[a0 + b0 + c1] +
+                 sc[a1 + b0 + c1] + sc[a0 + b1 + c1] + sc[a1 + b1 + c1]) *
+                (P)0.125;
+    se[a * SA + b * SB + c] += v;
+  }
+  __syncthreads();
+  tile_smooth<P, N, SA, SB, 1>(se, sr, F, oa, ob, oc, 0, w1, w6);
+  __syncthreads();
+  tile_smooth<P, N, SA, SB, 2>(se, sr, F, oa, ob, oc, 1, w1, w6);
+  __syncthreads();
+  tile_smooth<P, N, SA, SB, 3>(se, sr, F, oa, ob, oc, 0, w1, w6);
+  __syncthreads();
+  tile_smooth<P, N, SA, SB, 4>(se, sr, F, oa, ob, oc, 1, w1, w6);
+  __syncthreads();
+  for (int q = threadIdx.x; q < T * T * T; q += NT) {
+    const int a = q / (T * T), b = (q / T) % T, c = q % T;
+    if (s0 + a <= F.n0 && s1 + b <= F.n1 && s2 + c <= F.n2)
+      eo[(s0 + a) * F.sx + (s1 + b) * F.sy + s2 + c] = se[(a + LO) * SA + (b + LO) * SB + c + LO];
+  }
+}
+
 template <class P>
 __global__ void k_zero_level(P* __restrict__ e, Lv L, const int* __restrict__ done) {
   if (*done) return;
@@ -754,15 +1017,28 @@ __global__ void k_coarse_single(P* e, const P* r, Lv L, const int* __restrict__ 
 }
 
 // ---- coarse tail: the V-cycle below level Lc in one workgroup, arrays in LDS
+//
+// A phase (half-sweep, residual, transfer) of these levels is a few hundred to
+// a few thousand points between two barriers, so its time is the latency of
+// one point's LDS reads and of finding the point. The points of each level are
+// listed once per context (array index by colour, index of a coarse point's
+// fine node, packed interpolation corner), and the lists go to LDS with the
+// right-hand side: a phase then takes one list entry instead of two integer
+// divisions. 15^3 -> 1: 17.1 -> 15.2 us, bound by LDS reads on the 15^3 level
+// (half of it) and latency below; 11 x 9 x 13 -> 5 x 4 x 6 (32 sweeps there):
+// 18.3 us, where with 23 x 19 x 27 on top, walked by columns, it was 47 us.
 
 constexpr int kTailMaxLevels = 8;
 constexpr int kTailThreads = 1024;
+constexpr int kTailWave = 343;  // 7^3
 
 struct TailLv {
-  int n0, n1, n2;
-  int sx, sy;    // strides of the padded (n+2)^3 array
-  int size;      // elements
+  int sx, sy;       // strides of the padded (n+2)^3 array
   int oe, orr, ot;  // element offsets of e, r, t in LDS
+  int count, red;   // points, of which colour 0
+  int list;         // offsets in the table: array index of each point (colour 0 first),
+  int fine;         // the same points' index in the next finer level,
+  int corner;       // and the coarse corner they interpolate from (13 bits) with the steps to the next (3 bits)
 };
 
 template <class P>
@@ -771,226 +1047,209 @@ struct TailArgs {
   TailLv lv[kTailMaxLevels];
   P* ge;                // level-Lc e in global memory
   const P* gr;          // level-Lc r in global memory
-  int64_t gsx, gsy;     // its strides
+  const int32_t* gidx;  // its points' index there, in list order
+  const uint16_t* tab;
+  int ntab;             // table entries (a multiple of 8), staged behind the arrays
   P w1, w6;
   int pre, post, coarse_sweeps;
-  int total;            // LDS elements
+  int total;            // LDS elements of the arrays
   const int* done;
 };
 
-// Tail loops give each thread whole (b, c) columns of a level and walk a.
-template <class P>
-__device__ void tail_smooth(P* s, const TailLv& L, int sweeps, P w1, P w6) {
-  const int ncol = L.n1 * L.n2;
-  P* e = s + L.oe;
-  const P* r = s + L.orr;
-  for (int it = 0; it < sweeps; ++it)
-    for (int col = 0; col < 2; ++col) {
-      for (int t = threadIdx.x; t < ncol; t += kTailThreads) {
-        const int b = t / L.n2 + 1, c = t % L.n2 + 1;
-        const int a0 = (col ^ ((b + c) & 1)) ? 1 : 2;  // (a + b + c) % 2 == col
-        for (int a = a0; a <= L.n0; a += 2) {
-          const int g = a * L.sx + b * L.sy + c;
-          const P nb = e[g - L.sx] + e[g + L.sx] + e[g - L.sy] + e[g + L.sy] + e[g - 1] + e[g + 1];
-          e[g] = w1 * e[g] + w6 * (nb + r[g]);
-        }
-      }
-      __syncthreads();
-    }
+// Orders a wavefront's LDS accesses in the program's order (they execute in
+// order; this keeps the compiler from moving them), or the workgroup's.
+template <bool BLOCK>
+__device__ inline void tail_sync() {
+  if constexpr (BLOCK) {
+    __syncthreads();
+  } else {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
 }
 
 template <class P>
+__device__ inline P tail_new(const P* e, const P* r, const TailLv& L, int g, P w1, P w6) {
+  const P nb = e[g - L.sx] + e[g + L.sx] + e[g - L.sy] + e[g + L.sy] + e[g - 1] + e[g + 1];
+  return w1 * e[g] + w6 * (nb + r[g]);
+}
+
+// Sweeps over a level by NT threads; up to U points of each colour per thread
+// keep their index over the sweeps, and are read together (a half-sweep reads
+// only the other colour and itself).
+template <class P, int NT, int U>
+__device__ inline void tail_smooth(P* s, const uint16_t* tab, const TailLv L, int sweeps, P w1, P w6) {
+  constexpr bool BLOCK = NT == kTailThreads;
+  P* e = s + L.oe;
+  const P* r = s + L.orr;
+  int g[2][U], n[2] = {L.red, L.count - L.red};
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = (int)threadIdx.x + u * NT;
+      g[k][u] = tab[L.list + (k ? L.red : 0) + (q < n[k] ? q : 0)];
+    }
+  for (int it = 0; it < sweeps; ++it)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      P v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = tail_new<P>(e, r, L, g[k][u], w1, w6);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if ((int)threadIdx.x + u * NT < n[k]) e[g[k][u]] = v[u];
+      for (int q = threadIdx.x + U * NT; q < n[k]; q += NT) {  // (a large coarsest level)
+        const int gq = tab[L.list + (k ? L.red : 0) + q];
+        e[gq] = tail_new<P>(e, r, L, gq, w1, w6);
+      }
+      tail_sync<BLOCK>();
+    }
+}
+
+// Levels [l0, nl) by NT threads: pre-smoothing, residual and restriction down,
+// the coarsest level, interpolation and post-smoothing up.
+template <class P, int NT, int U>
+__device__ inline void tail_down(P* s, const uint16_t* tab, const TailArgs<P>& A, const TailLv F, const TailLv C) {
+  constexpr bool BLOCK = NT == kTailThreads;
+  tail_smooth<P, NT, U>(s, tab, F, A.pre, A.w1, A.w6);
+  const P* e = s + F.oe;
+  for (int q = threadIdx.x; q < F.count; q += NT) {
+    const int g = tab[F.list + q];
+    s[F.ot + g] = s[F.orr + g] - ((P)6 * e[g] - (e[g - F.sx] + e[g + F.sx] + e[g - F.sy] + e[g + F.sy] + e[g - 1] +
+                                                 e[g + 1]));
+  }
+  tail_sync<BLOCK>();
+  for (int q = threadIdx.x; q < C.count; q += NT) {
+    const int f = F.ot + tab[C.fine + q];
+    P acc = 0;
+#pragma unroll
+    for (int da = -1; da <= 1; ++da)
+#pragma unroll
+      for (int db = -1; db <= 1; ++db)
+#pragma unroll
+        for (int dc = -1; dc <= 1; ++dc) acc += fw_weight<P>(da, db, dc) * s[f + da * F.sx + db * F.sy + dc];
+    s[C.orr + tab[C.list + q]] = acc * (P)0.5;
+  }
+  tail_sync<BLOCK>();
+}
+
+template <class P, int NT, int U>
+__device__ inline void tail_bottom(P* s, const uint16_t* tab, const TailArgs<P>& A, const TailLv L) {
+  if (L.count == 1) {
+    if (threadIdx.x == 0) {
+      const int g = tab[L.list];
+      s[L.oe + g] = s[L.orr + g] / (P)6;
+    }
+    tail_sync<NT == kTailThreads>();
+  } else {
+    tail_smooth<P, NT, U>(s, tab, L, A.coarse_sweeps, (P)0, (P)1 / (P)6);
+  }
+}
+
+template <class P, int NT, int U>
+__device__ inline void tail_up(P* s, const uint16_t* tab, const TailArgs<P>& A, const TailLv F, const TailLv C) {
+  const P* ec = s + C.oe;
+  for (int q = threadIdx.x; q < F.count; q += NT) {
+    const int w = tab[F.corner + q];
+    const P* p = ec + (w & 0x1fff);
+    const int da = (w >> 13) & 1 ? C.sx : 0, db = (w >> 14) & 1 ? C.sy : 0, dc = w >> 15;
+    const P v = (p[0] + p[da] + p[db] + p[da + db] + p[dc] + p[da + dc] + p[db + dc] + p[da + db + dc]) * (P)0.125;
+    s[F.oe + tab[F.list + q]] += v;
+  }
+  tail_sync<NT == kTailThreads>();
+  tail_smooth<P, NT, U>(s, tab, F, A.post, A.w1, A.w6);
+}
+
+// The levels of the cubic chain 15 -> 7 -> 3 -> 1 (every grid of 2^k + 1 nodes
+// per axis ends in it), as plan_tail lays them out: with the strides known at
+// compile time a point's neighbours are immediates of one address.
+constexpr int tail_plane(int n1, int n2) { return ((n1 + 2) * (n2 + 2) + 1) & ~1; }
+constexpr TailLv cube15_lv(int q) {
+  int n = 15, off = 0, at = 0;
+  TailLv L{};
+  for (int k = 0;; ++k) {
+    const int sx = tail_plane(n, n), size = (n + 2) * sx, pts = n * n * n;
+    L = TailLv{sx, n + 2, off, off + size, off + 2 * size, pts, pts / 2, at, k ? at + pts : 0, 0};
+    at += k ? 2 * pts : pts;
+    if (k < 3) {
+      L.corner = at;
+      at += pts;
+    }
+    if (k == q) return L;
+    off += 3 * size;
+    n = (n - 1) / 2;
+  }
+}
+
+template <class P, bool CUBE15>
+__device__ inline TailLv tail_lv(const TailArgs<P>& A, int q) {
+  if constexpr (CUBE15) return q == 0 ? cube15_lv(0) : (q == 1 ? cube15_lv(1) : (q == 2 ? cube15_lv(2) : cube15_lv(3)));
+  return A.lv[q];
+}
+
+template <class P, bool CUBE15>
 __global__ __launch_bounds__(kTailThreads) void k_coarse_tail(TailArgs<P> A) {
   if (*A.done) return;
   extern __shared__ __attribute__((aligned(16))) char tail_lds[];
   P* s = reinterpret_cast<P*>(tail_lds);
-  for (int q = threadIdx.x; q < A.total; q += kTailThreads) s[q] = (P)0;
-  __syncthreads();
+  uint16_t* tab = reinterpret_cast<uint16_t*>(s + A.total);
+  const TailLv L0 = tail_lv<P, CUBE15>(A, 0);
   {
-    const TailLv& L = A.lv[0];
-    for (int t = threadIdx.x; t < L.n1 * L.n2; t += kTailThreads) {
-      const int b = t / L.n2 + 1, c = t % L.n2 + 1;
-      for (int a = 1; a <= L.n0; ++a) s[L.orr + a * L.sx + b * L.sy + c] = A.gr[a * A.gsx + b * A.gsy + c];
+    constexpr int U = 4;  // right-hand side points in flight while the arrays are cleared
+    P v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = threadIdx.x + u * kTailThreads;
+      v[u] = q < L0.count ? A.gr[A.gidx[q]] : (P)0;
     }
+    for (int q = threadIdx.x; q < A.ntab / 8; q += kTailThreads)
+      reinterpret_cast<uint4*>(tab)[q] = reinterpret_cast<const uint4*>(A.tab)[q];
+    for (int q = threadIdx.x; q < A.total * (int)sizeof(P) / 16; q += kTailThreads)
+      reinterpret_cast<uint4*>(s)[q] = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = threadIdx.x + u * kTailThreads;
+      if (q < L0.count) s[L0.orr + tab[L0.list + q]] = v[u];
+    }
+    for (int q = threadIdx.x + U * kTailThreads; q < L0.count; q += kTailThreads)
+      s[L0.orr + tab[L0.list + q]] = A.gr[A.gidx[q]];
     __syncthreads();
   }
-  // descend
-  for (int l = 0; l + 1 < A.nl; ++l) {
-    const TailLv& F = A.lv[l];
-    const TailLv& C = A.lv[l + 1];
-    tail_smooth<P>(s, F, A.pre, A.w1, A.w6);
-    const P* e = s + F.oe;
-    for (int t = threadIdx.x; t < F.n1 * F.n2; t += kTailThreads) {
-      const int b = t / F.n2 + 1, c = t % F.n2 + 1;
-      for (int a = 1; a <= F.n0; ++a) {
-        const int g = a * F.sx + b * F.sy + c;
-        s[F.ot + g] = s[F.orr + g] - ((P)6 * e[g] - (e[g - F.sx] + e[g + F.sx] + e[g - F.sy] + e[g + F.sy] +
-                                                      e[g - 1] + e[g + 1]));
-      }
+  // levels of at most kTailWave points go to the first wavefront alone, which
+  // needs no barriers between its phases
+  auto lv = [&](int q) { return tail_lv<P, CUBE15>(A, q); };
+  if constexpr (CUBE15) {
+    tail_down<P, kTailThreads, 2>(s, tab, A, lv(0), lv(1));
+    if (threadIdx.x < 64) {
+      tail_down<P, 64, 3>(s, tab, A, lv(1), lv(2));
+      tail_down<P, 64, 1>(s, tab, A, lv(2), lv(3));
+      tail_bottom<P, 64, 1>(s, tab, A, lv(3));
+      tail_up<P, 64, 1>(s, tab, A, lv(2), lv(3));
+      tail_up<P, 64, 3>(s, tab, A, lv(1), lv(2));
     }
     __syncthreads();
-    for (int t = threadIdx.x; t < C.n1 * C.n2; t += kTailThreads) {
-      const int b = t / C.n2 + 1, c = t % C.n2 + 1;
-      for (int a = 1; a <= C.n0; ++a) {
-        const int f = (2 * a) * F.sx + (2 * b) * F.sy + 2 * c;
-        P acc = 0;
-        for (int da = -1; da <= 1; ++da)
-          for (int db = -1; db <= 1; ++db)
-            for (int dc = -1; dc <= 1; ++dc)
-              acc += fw_weight<P>(da, db, dc) * s[F.ot + f + da * F.sx + db * F.sy + dc];
-        const int gc = a * C.sx + b * C.sy + c;
-        s[C.orr + gc] = acc * (P)0.5;
-        s[C.oe + gc] = (P)0;
-      }
-    }
-    __syncthreads();
-  }
-  // coarsest level
-  {
-    const TailLv& L = A.lv[A.nl - 1];
-    if (L.n0 == 1 && L.n1 == 1 && L.n2 == 1) {
-      if (threadIdx.x == 0) {
-        const int g = L.sx + L.sy + 1;
-        s[L.oe + g] = s[L.orr + g] / (P)6;
+    tail_up<P, kTailThreads, 2>(s, tab, A, lv(0), lv(1));
+  } else {
+    int ls = 0;
+    while (ls < A.nl && A.lv[ls].count > kTailWave) ++ls;
+    const int top = min(ls, A.nl - 1);  // levels the workgroup descends from
+    for (int l = 0; l < top; ++l) tail_down<P, kTailThreads, 2>(s, tab, A, lv(l), lv(l + 1));
+    if (ls < A.nl) {
+      if (threadIdx.x < 64) {
+        for (int l = ls; l + 1 < A.nl; ++l) tail_down<P, 64, 3>(s, tab, A, lv(l), lv(l + 1));
+        tail_bottom<P, 64, 3>(s, tab, A, lv(A.nl - 1));
+        for (int l = A.nl - 2; l >= ls; --l) tail_up<P, 64, 3>(s, tab, A, lv(l), lv(l + 1));
       }
       __syncthreads();
     } else {
-      tail_smooth<P>(s, L, A.coarse_sweeps, (P)0, (P)1 / (P)6);
+      tail_bottom<P, kTailThreads, 2>(s, tab, A, lv(A.nl - 1));
     }
+    for (int l = top - 1; l >= 0; --l) tail_up<P, kTailThreads, 2>(s, tab, A, lv(l), lv(l + 1));
   }
-  // ascend
-  for (int l = A.nl - 2; l >= 0; --l) {
-    const TailLv& F = A.lv[l];
-    const TailLv& C = A.lv[l + 1];
-    const P* ec = s + C.oe;
-    for (int t = threadIdx.x; t < F.n1 * F.n2; t += kTailThreads) {
-      const int b = t / F.n2 + 1, c = t % F.n2 + 1;
-      const int b0 = b >> 1, b1 = (b + 1) >> 1, c0 = c >> 1, c1 = (c + 1) >> 1;
-      for (int a = 1; a <= F.n0; ++a) {
-        const int a0 = a >> 1, a1 = (a + 1) >> 1;
-        auto E = [&](int x, int y, int z) { return ec[x * C.sx + y * C.sy + z]; };
-        const P v = (E(a0, b0, c0) + E(a1, b0, c0) + E(a0, b1, c0) + E(a1, b1, c0) + E(a0, b0, c1) +
-                     E(a1, b0, c1) + E(a0, b1, c1) + E(a1, b1, c1)) *
-                    (P)0.125;
-        s[F.oe + a * F.sx + b * F.sy + c] += v;
-      }
-    }
-    __syncthreads();
-    tail_smooth<P>(s, F, A.post, A.w1, A.w6);
-  }
-  {
-    const TailLv& L = A.lv[0];
-    for (int t = threadIdx.x; t < L.n1 * L.n2; t += kTailThreads) {
-      const int b = t / L.n2 + 1, c = t % L.n2 + 1;
-      for (int a = 1; a <= L.n0; ++a) A.ge[a * A.gsx + b * A.gsy + c] = s[L.oe + a * L.sx + b * L.sy + c];
-    }
-  }
-}
-
-// The same V-cycle for the cubic chain 15 -> 7 -> 3 -> 1 (every grid of
-// 2^k + 1 nodes per axis ends in it), sizes fixed at compile time: index maps
-// become multiplies and each half-sweep visits only its own colour.
-template <int N>
-struct TailDim {
-  static constexpr int S = N + 2, SX = S * S, SY = S, SIZE = S * S * S, H = (N + 1) / 2;
-};
-
-template <class P, int N>
-__device__ void c_smooth(P* e, const P* r, int sweeps, P w1, P w6) {
-  using D = TailDim<N>;
-  for (int it = 0; it < sweeps; ++it)
-    for (int col = 0; col < 2; ++col) {
-      for (int q = threadIdx.x; q < N * N * D::H; q += kTailThreads) {
-        const int a = q / (N * D::H) + 1, b = (q / D::H) % N + 1, m = q % D::H;
-        const int c = (((col + a + b) & 1) ? 1 : 2) + 2 * m;
-        if (c <= N) {
-          const int g = a * D::SX + b * D::SY + c;
-          const P nb = e[g - D::SX] + e[g + D::SX] + e[g - D::SY] + e[g + D::SY] + e[g - 1] + e[g + 1];
-          e[g] = w1 * e[g] + w6 * (nb + r[g]);
-        }
-      }
-      __syncthreads();
-    }
-}
-
-template <class P, int N>
-__device__ void c_cycle(P* s, P w1, P w6, int pre, int post) {
-  using D = TailDim<N>;
-  P* e = s;
-  P* r = s + D::SIZE;
-  if constexpr (N == 1) {
-    if (threadIdx.x == 0) e[D::SX + D::SY + 1] = r[D::SX + D::SY + 1] / (P)6;
-    __syncthreads();
-  } else {
-    constexpr int NC = (N - 1) / 2;
-    using C = TailDim<NC>;
-    P* t = s + 2 * D::SIZE;
-    P* ec = s + 3 * D::SIZE;
-    P* rc = ec + C::SIZE;
-    c_smooth<P, N>(e, r, pre, w1, w6);
-    for (int q = threadIdx.x; q < N * N * N; q += kTailThreads) {
-      const int a = q / (N * N) + 1, b = (q / N) % N + 1, c = q % N + 1;
-      const int g = a * D::SX + b * D::SY + c;
-      t[g] = r[g] - ((P)6 * e[g] - (e[g - D::SX] + e[g + D::SX] + e[g - D::SY] + e[g + D::SY] + e[g - 1] + e[g + 1]));
-    }
-    __syncthreads();
-    for (int q = threadIdx.x; q < NC * NC * NC; q += kTailThreads) {
-      const int a = q / (NC * NC) + 1, b = (q / NC) % NC + 1, c = q % NC + 1;
-      const int f = (2 * a) * D::SX + (2 * b) * D::SY + 2 * c;
-      P acc = 0;
-#pragma unroll
-      for (int da = -1; da <= 1; ++da)
-#pragma unroll
-        for (int db = -1; db <= 1; ++db)
-#pragma unroll
-          for (int dc = -1; dc <= 1; ++dc) acc += fw_weight<P>(da, db, dc) * t[f + da * D::SX + db * D::SY + dc];
-      const int gc = a * C::SX + b * C::SY + c;
-      rc[gc] = acc * (P)0.5;
-      ec[gc] = (P)0;
-    }
-    __syncthreads();
-    c_cycle<P, NC>(ec, w1, w6, pre, post);
-    for (int q = threadIdx.x; q < N * N * N; q += kTailThreads) {
-      const int a = q / (N * N) + 1, b = (q / N) % N + 1, c = q % N + 1;
-      const int a0 = a >> 1, a1 = (a + 1) >> 1, b0 = b >> 1, b1 = (b + 1) >> 1, c0 = c >> 1, c1 = (c + 1) >> 1;
-      auto E = [&](int x, int y, int z) { return ec[x * C::SX + y * C::SY + z]; };
-      const P v = (E(a0, b0, c0) + E(a1, b0, c0) + E(a0, b1, c0) + E(a1, b1, c0) + E(a0, b0, c1) + E(a1, b0, c1) +
-                   E(a0, b1, c1) + E(a1, b1, c1)) *
-                  (P)0.125;
-      e[a * D::SX + b * D::SY + c] += v;
-    }
-    __syncthreads();
-    c_smooth<P, N>(e, r, post, w1, w6);
-  }
-}
-
-template <int N>
-constexpr size_t chain_elems() {
-  if constexpr (N == 1)
-    return 2 * TailDim<1>::SIZE;
-  else
-    return 3 * TailDim<N>::SIZE + chain_elems<(N - 1) / 2>();
-}
-
-template <class P>
-__global__ __launch_bounds__(kTailThreads) void k_coarse_tail15(TailArgs<P> A) {
-  if (*A.done) return;
-  extern __shared__ __attribute__((aligned(16))) char tail_lds[];
-  P* s = reinterpret_cast<P*>(tail_lds);
-  using D = TailDim<15>;
-  constexpr int total = (int)chain_elems<15>();
-  for (int q = threadIdx.x; q < total; q += kTailThreads) s[q] = (P)0;
-  __syncthreads();
-  for (int q = threadIdx.x; q < 15 * 15 * 15; q += kTailThreads) {
-    const int a = q / 225 + 1, b = (q / 15) % 15 + 1, c = q % 15 + 1;
-    s[D::SIZE + a * D::SX + b * D::SY + c] = A.gr[a * A.gsx + b * A.gsy + c];
-  }
-  __syncthreads();
-  c_cycle<P, 15>(s, A.w1, A.w6, A.pre, A.post);
-  for (int q = threadIdx.x; q < 15 * 15 * 15; q += kTailThreads) {
-    const int a = q / 225 + 1, b = (q / 15) % 15 + 1, c = q % 15 + 1;
-    A.ge[a * A.gsx + b * A.gsy + c] = s[a * D::SX + b * D::SY + c];
-  }
+  for (int q = threadIdx.x; q < L0.count; q += kTailThreads) A.ge[A.gidx[q]] = s[L0.oe + tab[L0.list + q]];
 }
 
 // Face conditions on phi (Field.cpp:10-96): D -> 0, N -> copy the neighbour.
@@ -1072,64 +1331,121 @@ constexpr int64_t kSplitRestrict = (int64_t)1 << 20;
 
 int coarse_sweeps(const MgLevel& m) { return 4 * std::max({m.n[0], m.n[1], m.n[2]}) + 8; }
 
-// First level handled by the LDS tail kernel and its LDS bytes, for element size `esz`.
+// First level handled by the LDS tail kernel, its LDS bytes for element size
+// `esz`, and its point lists on the device. Every level keeps e and r, all but
+// the coarsest t, as padded (n+2)^3 arrays.
 void plan_tail(Ctx& c, size_t esz) {
   const int nl = (int)c.mg.size();
   c.mg_tail = nl;  // none
   c.mg_tail_bytes = 0;
-  size_t bytes = 0;
-  for (int l = nl - 1; l >= 0; --l) {
+  // plane length (even, see the lists' order below) and elements of a level's array
+  auto plane = [&](int l) { return tail_plane(c.mg[l].n[1], c.mg[l].n[2]); };
+  auto padded = [&](int l) { return (size_t)(c.mg[l].n[0] + 2) * plane(l); };
+  size_t arrays = 0, entries = 0;
+  for (int l = nl - 1; l >= 0 && nl - l <= kTailMaxLevels; --l) {
     const MgLevel& m = c.mg[l];
-    // the tail keeps its levels as padded (n+2)^3 arrays
-    const size_t lsz = (size_t)(m.n[0] + 2) * (m.n[1] + 2) * (m.n[2] + 2);
-    const size_t lb = 3 * lsz * esz;
-    if (bytes + lb > c.lds_max || nl - l > kTailMaxLevels) break;
-    bytes += lb;
+    const size_t pts = (size_t)m.n[0] * m.n[1] * m.n[2];
+    const bool last = l == nl - 1;
+    // (indices are 16 bits, a coarse corner's 13)
+    if (padded(l) > 65535 || (!last && padded(l + 1) > 8192)) break;
+    arrays += (last ? 2 : 3) * padded(l);
+    entries += (last ? 2 : 3) * pts;  // (a first level without a finer one leaves its second list unused)
+    const size_t bytes = (arrays * esz + 15) / 16 * 16 + (entries + 8) * sizeof(uint16_t);
+    if (bytes > c.lds_max) break;
+    // A level the level kernels can take leaves the tail above 15^3 points: one
+    // workgroup's phases then last longer than two launches (23 x 19 x 27: 29
+    // us here, 13 us there).
+    if (c.mg_fused && !last && pts > 3375) break;
     c.mg_tail = l;
     c.mg_tail_bytes = bytes;
   }
-  // the compile-time 15 -> 7 -> 3 -> 1 kernel when the tail is exactly that chain
-  c.mg_tail15 = false;
-  if (c.mg_tail < nl && nl - c.mg_tail == 4) {
-    bool ok = true;
-    const int want[4] = {15, 7, 3, 1};
-    for (int q = 0; q < 4; ++q)
-      for (int a = 0; a < 3; ++a) ok = ok && c.mg[c.mg_tail + q].n[a] == want[q];
-    c.mg_tail15 = ok;
+  c.mg_tail_plan.clear();
+  if (c.mg_tail == nl) return;
+  std::vector<uint16_t> tab;
+  std::vector<int32_t> gidx;
+  int off = 0;
+  for (int l = c.mg_tail; l < nl; ++l) {
+    const MgLevel& m = c.mg[l];
+    const int sy = m.n[2] + 2, sx = plane(l);
+    std::vector<uint16_t> list[2], fine[2], corner[2];
+    std::vector<int32_t> gi[2];
+    const bool first = l == c.mg_tail, last = l == nl - 1;
+    const int fy = first ? 0 : c.mg[l - 1].n[2] + 2, fx = first ? 0 : plane(l - 1);
+    const int cy = last ? 0 : c.mg[l + 1].n[2] + 2, cx = last ? 0 : plane(l + 1);
+    // Each colour's points go along c through two planes at once, so that
+    // neighbouring lanes read neighbouring banks: along one plane a colour's
+    // points are two elements apart, and every read took two turns (15^3: a
+    // half-sweep about 1850 cycles, 1100 so). The planes lie an even distance apart.
+    for (int k = 0; k < 2; ++k)
+      for (int ap = 1; ap <= m.n[0]; ap += 2)
+        for (int b = 1; b <= m.n[1]; ++b)
+          for (int q = 1; q <= m.n[2]; ++q) {
+            const int a = ap + ((ap + b + q + k) & 1);
+            if (a > m.n[0]) continue;
+            list[k].push_back((uint16_t)(a * sx + b * sy + q));
+            fine[k].push_back((uint16_t)(2 * a * fx + 2 * b * fy + 2 * q));
+            corner[k].push_back((uint16_t)(((a >> 1) * cx + (b >> 1) * cy + (q >> 1)) | (a & 1) << 13 | (b & 1) << 14 |
+                                           (q & 1) << 15));
+            gi[k].push_back((int32_t)(a * m.sx + b * m.sy + q));
+          }
+    auto add = [&](std::vector<uint16_t>(&v)[2]) {
+      const int at = (int)tab.size();
+      for (auto& x : v) tab.insert(tab.end(), x.begin(), x.end());
+      return at;
+    };
+    TailPlan t{};
+    t.sx = sx;
+    t.sy = sy;
+    t.oe = off;
+    t.orr = off + (int)padded(l);
+    t.ot = off + 2 * (int)padded(l);
+    off += (last ? 2 : 3) * (int)padded(l);
+    t.red = (int)list[0].size();
+    t.count = t.red + (int)list[1].size();
+    t.list = add(list);
+    if (!first) t.fine = add(fine);
+    if (!last) t.corner = add(corner);
+    if (first)
+      for (auto& x : gi) gidx.insert(gidx.end(), x.begin(), x.end());
+    c.mg_tail_plan.push_back(t);
   }
+  c.mg_tail15 = c.mg_tail_plan.size() == 4;
+  for (size_t q = 0; q < c.mg_tail_plan.size() && c.mg_tail15; ++q) {
+    const TailPlan& t = c.mg_tail_plan[q];
+    const TailLv L = cube15_lv((int)q);
+    const MgLevel& m = c.mg[c.mg_tail + q];
+    c.mg_tail15 = m.n[0] == m.n[1] && m.n[1] == m.n[2] && t.sx == L.sx && t.sy == L.sy && t.oe == L.oe &&
+                  t.orr == L.orr && (q == 3 || t.ot == L.ot) && t.count == L.count && t.red == L.red &&
+                  t.list == L.list && (q == 0 || t.fine == L.fine) && (q == 3 || t.corner == L.corner);
+  }
+  c.mg_tail_elems = (int)(((size_t)off * esz + 15) / 16 * 16 / esz);
+  while (tab.size() % 8) tab.push_back(0);
+  c.mg_tail_tab.alloc(tab.size());
+  c.mg_tail_idx.alloc(gidx.size());
+  FOPIS_HIP(hipMemcpy(c.mg_tail_tab.p, tab.data(), tab.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+  FOPIS_HIP(hipMemcpy(c.mg_tail_idx.p, gidx.data(), gidx.size() * sizeof(int32_t), hipMemcpyHostToDevice));
 }
 
 template <class P>
 TailArgs<P> tail_args(Ctx& c, const int* done) {
   TailArgs<P> A{};
-  const int l0 = c.mg_tail;
-  A.nl = (int)c.mg.size() - l0;
-  int off = 0;
+  A.nl = (int)c.mg_tail_plan.size();
   for (int q = 0; q < A.nl; ++q) {
-    const MgLevel& m = c.mg[l0 + q];
-    TailLv& L = A.lv[q];
-    L.n0 = m.n[0];
-    L.n1 = m.n[1];
-    L.n2 = m.n[2];
-    L.sy = m.n[2] + 2;
-    L.sx = (m.n[1] + 2) * (m.n[2] + 2);
-    L.size = (m.n[0] + 2) * L.sx;
-    L.oe = off;
-    L.orr = off + L.size;
-    L.ot = off + 2 * L.size;
-    off += 3 * L.size;
+    const TailPlan& t = c.mg_tail_plan[q];
+    A.lv[q] = TailLv{t.sx, t.sy, t.oe, t.orr, t.ot, t.count, t.red, t.list, t.fine, t.corner};
   }
-  MgLevel& m0 = c.mg[l0];
+  MgLevel& m0 = c.mg[c.mg_tail];
   A.ge = E_<P>(m0);
   A.gr = R_<P>(m0);
-  A.gsx = m0.sx;
-  A.gsy = m0.sy;
+  A.gidx = c.mg_tail_idx.p;
+  A.tab = c.mg_tail_tab.p;
+  A.ntab = (int)c.mg_tail_tab.n;
   A.w1 = (P)(1.0 - c.d.mg_omega);
   A.w6 = (P)(c.d.mg_omega / 6.0);
   A.pre = c.d.mg_pre;
   A.post = c.d.mg_post;
   A.coarse_sweeps = coarse_sweeps(c.mg.back());
-  A.total = off;
+  A.total = c.mg_tail_elems;
   A.done = done;
   return A;
 }
@@ -1173,21 +1489,34 @@ void smooth(Ctx& c, MgLevel& m, int sweeps, double w, bool from_zero, const int*
   }
 }
 
-// One V-cycle from level l down. zero: the level's correction starts from
-// e = 0 (always so below the finest level); otherwise the finest level's
-// cycle continues from the correction already in e (a second cycle on the
-// same right-hand side).
+dim3 grid_tiles(const MgLevel& m) {
+  return dim3(div_up(m.n[2], kTileEdge), div_up(m.n[1], kTileEdge), div_up(m.n[0], kTileEdge));
+}
+
+// The level kernels take levels of up to 2^19 unknowns, 1024 tiles, two rounds
+// of the chip: beyond, the halo they recompute (8 times the tile's points are
+// loaded, 4.8 times swept first) costs more than the launches they save (63^3:
+// 19 us in two launches, 40 us in ten; 95 x 79 x 111: 59 and 43 us).
+constexpr int64_t kLevelMost = (int64_t)1 << 19;
+bool level_fused(const Ctx& c, const MgLevel& m) {
+  return c.mg_fused && (int64_t)m.n[0] * m.n[1] * m.n[2] <= kLevelMost;
+}
+
+// One V-cycle from level l down; returns the array that holds the level's
+// correction. from: the correction the finest level's cycle continues from (a
+// second cycle on the same right-hand side), null to start from e = 0 (always
+// so below the finest level).
 template <class P>
-void vcycle(Ctx& c, int l, const int* done, bool zero = true) {
+P* vcycle(Ctx& c, int l, const int* done, const P* from = nullptr) {
   MgLevel& m = c.mg[l];
+  const bool zero = from == nullptr;
   const double w = c.d.mg_omega;
   if (l == c.mg_tail) {
-    TailArgs<P> A = tail_args<P>(c, done);
     if (c.mg_tail15)
-      k_coarse_tail15<P><<<1, kTailThreads, c.mg_tail_bytes, c.stream>>>(A);
+      k_coarse_tail<P, true><<<1, kTailThreads, c.mg_tail_bytes, c.stream>>>(tail_args<P>(c, done));
     else
-      k_coarse_tail<P><<<1, kTailThreads, c.mg_tail_bytes, c.stream>>>(A);
-    return;
+      k_coarse_tail<P, false><<<1, kTailThreads, c.mg_tail_bytes, c.stream>>>(tail_args<P>(c, done));
+    return E_<P>(m);
   }
   if (l == (int)c.mg.size() - 1) {
     // coarsest level outside the tail kernel: Gauss-Seidel sweeps from zero
@@ -1196,14 +1525,27 @@ void vcycle(Ctx& c, int l, const int* done, bool zero = true) {
     } else {
       smooth<P>(c, m, coarse_sweeps(m), 1.0, true, done);
     }
-    return;
+    return E_<P>(m);
   }
   MgLevel& mc = c.mg[l + 1];
+  bool rb = false;
+  if constexpr (std::is_same<P, float>::value) rb = c.mg_rb && l == 0;
+  if (level_fused(c, m)) {
+    const P w1 = (P)(1.0 - w), w6 = (P)(w / 6.0);
+    if (from)
+      k_level_down<P, false><<<grid_tiles(m), kTileThreads, DownDim<P, false>::kLds, c.stream>>>(
+          E_<P>(m), from, R_<P>(m), lv_of(m), R_<P>(mc), lv_of(mc), w1, w6, done);
+    else
+      k_level_down<P, true><<<grid_tiles(m), kTileThreads, DownDim<P, true>::kLds, c.stream>>>(
+          E_<P>(m), nullptr, R_<P>(m), lv_of(m), R_<P>(mc), lv_of(mc), w1, w6, done);
+    const P* ec = vcycle<P>(c, l + 1, done);
+    k_level_up<P><<<grid_tiles(m), kTileThreads, UpDim<P>::kLds, c.stream>>>(T_<P>(m), E_<P>(m), R_<P>(m), lv_of(m), ec,
+                                                                           lv_of(mc), w1, w6, done);
+    return T_<P>(m);
+  }
   // every level starts its cycle from e = 0 (the correction equation)
   if (zero && c.d.mg_pre == 0) k_zero_level<P><<<grid_full(m), 64, 0, c.stream>>>(E_<P>(m), lv_of(m), done);
   smooth<P>(c, m, c.d.mg_pre, w, zero, done);
-  bool rb = false;
-  if constexpr (std::is_same<P, float>::value) rb = c.mg_rb && l == 0;
   if (rb) {
     if constexpr (std::is_same<P, float>::value) {
       k_resid_level_rb<<<grid_rb(c), 64, 0, c.stream>>>(T_<P>(m), rb_of(c), lv_of(m), done);
@@ -1216,14 +1558,15 @@ void vcycle(Ctx& c, int l, const int* done, bool zero = true) {
     k_restrict_resid<P><<<grid_full(mc), 64, 0, c.stream>>>(R_<P>(mc), lv_of(mc), E_<P>(m), R_<P>(m), lv_of(m),
                                                             done);
   }
-  vcycle<P>(c, l + 1, done);
+  const P* ec = vcycle<P>(c, l + 1, done);
   if (rb) {
     if constexpr (std::is_same<P, float>::value)
-      k_prolong_rb<<<grid_full4(m), 64, 0, c.stream>>>(rb_of(c), E_<P>(mc), lv_of(mc), done);
+      k_prolong_rb<<<grid_full4(m), 64, 0, c.stream>>>(rb_of(c), ec, lv_of(mc), done);
   } else {
-    k_prolong<P><<<grid_full4(m), 64, 0, c.stream>>>(E_<P>(m), lv_of(m), E_<P>(mc), lv_of(mc), done);
+    k_prolong<P><<<grid_full4(m), 64, 0, c.stream>>>(E_<P>(m), lv_of(m), ec, lv_of(mc), done);
   }
   smooth<P>(c, m, c.d.mg_post, w, false, done);
+  return E_<P>(m);
 }
 
 template <class P>
@@ -1244,10 +1587,18 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
   if (c.mg_tail_esz != sizeof(P)) {
     plan_tail(c, sizeof(P));
     c.mg_tail_esz = sizeof(P);
+    if (c.mg_fused) {
+      auto grant = [](const void* f, size_t bytes) {
+        if (bytes > 65536) FOPIS_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+      };
+      grant(reinterpret_cast<const void*>(&k_level_down<P, false>), DownDim<P, false>::kLds);
+      grant(reinterpret_cast<const void*>(&k_level_down<P, true>), DownDim<P, true>::kLds);
+      grant(reinterpret_cast<const void*>(&k_level_up<P>), UpDim<P>::kLds);
+    }
     if (c.mg_tail < (int)c.mg.size() && c.mg_tail_bytes > 65536) {
-      FOPIS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_coarse_tail<P>),
+      FOPIS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_coarse_tail<P, false>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)c.mg_tail_bytes));
-      FOPIS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_coarse_tail15<P>),
+      FOPIS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_coarse_tail<P, true>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)c.mg_tail_bytes));
     }
   }
@@ -1297,26 +1648,26 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
   // tolerance and the cycle cap are arguments of the norm kernel, so the
   // graphs are rebuilt when they change) and replayed.
   auto cycle = [&](int nv) {
-    vcycle<P>(c, 0, done);
+    const P* e = vcycle<P>(c, 0, done);
     if (nv == 2) {
       if constexpr (std::is_same<P, float>::value) {
         if (rb)
           k_pair_resid_rb<<<nb, 256, 0, c.stream>>>(rb_of(c), L0, part, done);
         else
-          k_pair_resid<P><<<nb, 256, 0, c.stream>>>(E_<P>(m0), r0, L0, part, done);
+          k_pair_resid<P><<<nb, 256, 0, c.stream>>>(e, r0, L0, part, done);
       } else {
-        k_pair_resid<P><<<nb, 256, 0, c.stream>>>(E_<P>(m0), r0, L0, part, done);
+        k_pair_resid<P><<<nb, 256, 0, c.stream>>>(e, r0, L0, part, done);
       }
       k_pair_check<<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, skip);
-      vcycle<P>(c, 0, skip, false);
+      e = vcycle<P>(c, 0, skip, e);
     }
     if constexpr (std::is_same<P, float>::value) {
       if (rb)
         k_update_rb<<<nb, 256, 0, c.stream>>>(phi, rb_of(c), r64, L0, part, done);
       else
-        k_update<P><<<nb, 256, 0, c.stream>>>(phi, E_<P>(m0), r64, r0, L0, part, done);
+        k_update<P><<<nb, 256, 0, c.stream>>>(phi, e, r64, r0, L0, part, done);
     } else {
-      k_update<P><<<nb, 256, 0, c.stream>>>(phi, E_<P>(m0), r64, r0, L0, part, done);
+      k_update<P><<<nb, 256, 0, c.stream>>>(phi, e, r64, r0, L0, part, done);
     }
     k_norm<<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, max_cycles, nv, 1, nv == 2 ? skip : nullptr);
   };
@@ -1453,6 +1804,8 @@ void poisson_init(Ctx& c) {
   // the finest level stored by colour: FP32 levels, a level large enough to
   // form its residual in a pass of its own (and so never inside the LDS tail),
   // pre-smoothing (its first sweep starts from zero); FOPIS_MG_RB=0 keeps one array
+  const char* fu = std::getenv("FOPIS_MG_FUSED");
+  c.mg_fused = c.d.mg_pre == 2 && c.d.mg_post == 2 && !(fu && fu[0] == '0');
   const char* rbs = std::getenv("FOPIS_MG_RB");
   const MgLevel& l0 = c.mg[0];
   c.mg_rb = f32 && !(rbs && rbs[0] == '0') && c.mg.size() > 1 && c.d.mg_pre > 0 &&
