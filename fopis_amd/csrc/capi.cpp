@@ -195,6 +195,7 @@ int fopis_create(const fopis_desc* desc, fopis_ctx** out) {
     delete h;
     return rc;
   }
+  host_copy_retain();
   *out = h;
   return FOPIS_OK;
 }
@@ -208,6 +209,7 @@ int fopis_destroy(fopis_ctx* ctx) {
   poisson_free(ctx->c);
   delete ctx;
   if (st) (void)hipStreamDestroy(st);
+  host_copy_release();
   return FOPIS_OK;
 }
 

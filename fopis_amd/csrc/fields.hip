@@ -277,19 +277,16 @@ void fields_get(Ctx& c, int which, int s, double* out) {
     DBuf<double> tmp;
     tmp.alloc(n);
     k_edge<<<div_up((int64_t)n, 256), 256, 0, c.stream>>>(c.phi.p, tmp.p, which - FOPIS_EX, c.cx, c.cy, c.cz);
-    FOPIS_HIP(hipMemcpyAsync(out, tmp.p, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-    FOPIS_HIP(hipStreamSynchronize(c.stream));
+    copy_out(out, tmp.p, n * sizeof(double), c.stream);
     return;
   }
-  FOPIS_HIP(hipMemcpyAsync(out, field_ptr(c, which, s), n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-  FOPIS_HIP(hipStreamSynchronize(c.stream));
+  copy_out(out, field_ptr(c, which, s), n * sizeof(double), c.stream);
 }
 
 void fields_set(Ctx& c, int which, int s, const double* in) {
   if (which >= FOPIS_EX && which <= FOPIS_EZ) throw Error(FOPIS_E_ARG, "edge fields are derived from phi");
   const size_t n = field_len(c, which);
-  FOPIS_HIP(hipMemcpyAsync(field_ptr(c, which, s), in, n * sizeof(double), hipMemcpyHostToDevice, c.stream));
-  FOPIS_HIP(hipStreamSynchronize(c.stream));
+  copy_in(field_ptr(c, which, s), in, n * sizeof(double), c.stream);
 }
 
 void fields_energy_queue(Ctx& c, double* part, double* sum) {

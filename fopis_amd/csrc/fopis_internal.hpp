@@ -348,6 +348,19 @@ struct Ctx {
   size_t id3(int i, int j, int k) const { return ((size_t)i * cy + j) * cz + k; }
 };
 
+// ---- copies between the caller's pageable arrays and the device (hostcopy.cpp) ----
+struct HostSeg {
+  void* host;
+  void* dev;
+  size_t bytes;
+};
+// a context keeps the pinned block of large copies alive
+void host_copy_retain();
+void host_copy_release();
+void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st);
+void copy_out(void* host, const void* dev, size_t bytes, hipStream_t st);
+void copy_in(void* dev, const void* host, size_t bytes, hipStream_t st);
+
 // ---- entry points implemented in the .hip units ----
 void particles_init(Ctx& c);
 void particles_set(Ctx& c, int s, int64_t n, const double* const* host6);

@@ -1608,9 +1608,9 @@ void guess_dataset_get(Ctx& c, int slot, uint16_t* rho_hat, uint8_t* mask, uint1
   check_slot(g, slot);
   const int64_t n = nvox_of(g.lv[0]);
   FOPIS_HIP(hipStreamSynchronize(c.stream));
-  if (rho_hat) FOPIS_HIP(hipMemcpy(rho_hat, g.ds_rho.p + (size_t)slot * n, n * 2, hipMemcpyDeviceToHost));
-  if (mask) FOPIS_HIP(hipMemcpy(mask, g.ds_mask.p + (size_t)slot * n, n, hipMemcpyDeviceToHost));
-  if (phi_hat) FOPIS_HIP(hipMemcpy(phi_hat, g.ds_phi.p + (size_t)slot * n, n * 2, hipMemcpyDeviceToHost));
+  if (rho_hat) copy_out(rho_hat, g.ds_rho.p + (size_t)slot * n, n * 2, c.stream);
+  if (mask) copy_out(mask, g.ds_mask.p + (size_t)slot * n, n, c.stream);
+  if (phi_hat) copy_out(phi_hat, g.ds_phi.p + (size_t)slot * n, n * 2, c.stream);
 }
 
 void guess_dataset_set(Ctx& c, int slot, const uint16_t* rho_hat, const uint8_t* mask, const uint16_t* phi_hat) {
@@ -1618,9 +1618,9 @@ void guess_dataset_set(Ctx& c, int slot, const uint16_t* rho_hat, const uint8_t*
   check_slot(g, slot);
   const int64_t n = nvox_of(g.lv[0]);
   FOPIS_HIP(hipStreamSynchronize(c.stream));
-  FOPIS_HIP(hipMemcpy(g.ds_rho.p + (size_t)slot * n, rho_hat, n * 2, hipMemcpyHostToDevice));
-  FOPIS_HIP(hipMemcpy(g.ds_mask.p + (size_t)slot * n, mask, n, hipMemcpyHostToDevice));
-  FOPIS_HIP(hipMemcpy(g.ds_phi.p + (size_t)slot * n, phi_hat, n * 2, hipMemcpyHostToDevice));
+  copy_in(g.ds_rho.p + (size_t)slot * n, rho_hat, n * 2, c.stream);
+  copy_in(g.ds_mask.p + (size_t)slot * n, mask, n, c.stream);
+  copy_in(g.ds_phi.p + (size_t)slot * n, phi_hat, n * 2, c.stream);
   double s = 0.0;
   for (int64_t v = 0; v < n; ++v) {
     const double x = bf2f(phi_hat[v]);
@@ -1641,7 +1641,7 @@ double guess_grad(Ctx& c, int slot, float* grad_out) {
   double l = 0.0;
   FOPIS_HIP(hipMemcpyAsync(&l, g.loss_acc.p, sizeof(double), hipMemcpyDeviceToHost, c.stream));
   FOPIS_HIP(hipStreamSynchronize(c.stream));
-  if (grad_out) FOPIS_HIP(hipMemcpy(grad_out, g.grad.p, g.nparams * sizeof(float), hipMemcpyDeviceToHost));
+  if (grad_out) copy_out(grad_out, g.grad.p, g.nparams * sizeof(float), c.stream);
   FOPIS_HIP(hipGetLastError());
   return l;
 }
@@ -1783,13 +1783,12 @@ void nn_conv3d(int n0, int n1, int n2, int cin, int cout, int up, int relu, cons
   dw.alloc(27LL * cin * cout);
   db.alloc(cout);
   dwp.alloc((size_t)nqp * cout * 8);
-  FOPIS_HIP(hipMemcpy(dx.p, x, nin * cin * 2, hipMemcpyHostToDevice));
-  FOPIS_HIP(hipMemcpy(dw.p, w, 27LL * cin * cout * 4, hipMemcpyHostToDevice));
-  FOPIS_HIP(hipMemcpy(db.p, b, cout * 4, hipMemcpyHostToDevice));
-  if (add) {
-    dadd.alloc(nv * cout);
-    FOPIS_HIP(hipMemcpy(dadd.p, add, nv * cout * 2, hipMemcpyHostToDevice));
-  }
+  if (add) dadd.alloc(nv * cout);
+  const HostSeg up_seg[4] = {{const_cast<uint16_t*>(x), dx.p, (size_t)(nin * cin * 2)},
+                             {const_cast<float*>(w), dw.p, (size_t)(27LL * cin * cout * 4)},
+                             {const_cast<float*>(b), db.p, (size_t)cout * 4},
+                             {const_cast<uint16_t*>(add), dadd.p, (size_t)(nv * cout * 2)}};
+  host_copy(up_seg, add ? 4 : 3, false, ts.s);
   k_pack<<<div_up((int64_t)nqp * cout * 8, 256), 256, 0, ts.s>>>(dw.p, dwp.p, cin, cout, nqp, 0);
   const int dims[3] = {n0, n1, n2};
   ConvArgs a = conv_args(dims, cin, cout, dx.p, dwp.p, db.p, relu);
@@ -1811,7 +1810,7 @@ void nn_conv3d(int n0, int n1, int n2, int cin, int cout, int up, int relu, cons
   }
   FOPIS_HIP(hipStreamSynchronize(ts.s));
   FOPIS_HIP(hipGetLastError());
-  FOPIS_HIP(hipMemcpy(y, dy.p, nv * cout * 2, hipMemcpyDeviceToHost));
+  copy_out(y, dy.p, nv * cout * 2, ts.s);
 }
 
 void nn_conv3d_backward(int n0, int n1, int n2, int cin, int cout, int up, const uint16_t* x, const float* w,
@@ -1828,10 +1827,11 @@ void nn_conv3d_backward(int n0, int n1, int n2, int cin, int cout, int up, const
   dgw.alloc(27LL * cin * cout);
   dgb.alloc(cout);
   zb.alloc(64);
-  FOPIS_HIP(hipMemcpy(dx.p, x, nin * cin * 2, hipMemcpyHostToDevice));
-  FOPIS_HIP(hipMemcpy(dg.p, gy, nv * cout * 2, hipMemcpyHostToDevice));
-  FOPIS_HIP(hipMemcpy(dw.p, w, 27LL * cin * cout * 4, hipMemcpyHostToDevice));
-  FOPIS_HIP(hipMemset(zb.p, 0, 64 * 4));
+  const HostSeg up_seg[3] = {{const_cast<uint16_t*>(x), dx.p, (size_t)(nin * cin * 2)},
+                             {const_cast<uint16_t*>(gy), dg.p, (size_t)(nv * cout * 2)},
+                             {const_cast<float*>(w), dw.p, (size_t)(27LL * cin * cout * 4)}};
+  host_copy(up_seg, 3, false, ts.s);
+  FOPIS_HIP(hipMemsetAsync(zb.p, 0, 64 * 4, ts.s));
   // weight and bias gradients through a throwaway network object
   GuessNet tmp;
   Ctx cc;
@@ -1848,12 +1848,11 @@ void nn_conv3d_backward(int n0, int n1, int n2, int cin, int cout, int up, const
     ConvArgs a = conv_args(dims, cout, cin, dg.p, dwd.p, zb.p, 0);
     a.y = ddx.p;
     launch_conv(ts.s, a, EPI_BF16, false);
-    FOPIS_HIP(hipStreamSynchronize(ts.s));
-    FOPIS_HIP(hipMemcpy(dx_out, ddx.p, nv * cin * 2, hipMemcpyDeviceToHost));
+    copy_out(dx_out, ddx.p, nv * cin * 2, ts.s);
   }
   FOPIS_HIP(hipStreamSynchronize(ts.s));
   FOPIS_HIP(hipGetLastError());
-  FOPIS_HIP(hipMemcpy(dw_out, dgw.p, 27LL * cin * cout * 4, hipMemcpyDeviceToHost));
+  copy_out(dw_out, dgw.p, 27LL * cin * cout * 4, ts.s);
   FOPIS_HIP(hipMemcpy(db_out, dgb.p, cout * 4, hipMemcpyDeviceToHost));
 }
 

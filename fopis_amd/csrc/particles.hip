@@ -1997,12 +1997,20 @@ static void set_impl(Ctx& c, int s, int64_t n, const double* const* h) {
   Soa<R> flat;
   if (n > 0) {
     flat.alloc(n);
-    Soa<double> raw;
-    raw.alloc(n);
-    for (int q = 0; q < 6; ++q)
-      FOPIS_HIP(hipMemcpyAsync(raw.c[q].p, h[q], n * sizeof(double), hipMemcpyHostToDevice, st));
-    k_from_f64<R><<<div_up(n, 256), 256, 0, st>>>(ptrs(flat), ptrs(raw), n);
-    FOPIS_HIP(hipStreamSynchronize(st));
+    auto upload = [&](Soa<double>& to) {
+      HostSeg seg[6];
+      for (int q = 0; q < 6; ++q) seg[q] = HostSeg{const_cast<double*>(h[q]), to.c[q].p, n * sizeof(double)};
+      host_copy(seg, 6, false, st);
+    };
+    if constexpr (sizeof(R) == 8) {
+      upload(flat);
+    } else {
+      Soa<double> raw;
+      raw.alloc(n);
+      upload(raw);
+      k_from_f64<R><<<div_up(n, 256), 256, 0, st>>>(ptrs(flat), ptrs(raw), n);
+      FOPIS_HIP(hipStreamSynchronize(st));
+    }
   }
   FOPIS_HIP(hipMemsetAsync(c.status.p + kStat * s, 0, kStat * sizeof(int32_t), st));
   bin_flat<R>(c, s, flat, n, false);
@@ -2126,10 +2134,9 @@ static void get_impl(Ctx& c, int s, int64_t cap, double* const* h, int64_t* nout
   std::vector<double> tmp;
   if (b.has_invalid && n > 0) {
     tmp.resize(6 * (size_t)n);
-    for (int q = 0; q < 6; ++q)
-      FOPIS_HIP(hipMemcpyAsync(tmp.data() + q * (size_t)n, out.c[q].p, n * sizeof(double), hipMemcpyDeviceToHost,
-                               c.stream));
-    FOPIS_HIP(hipStreamSynchronize(c.stream));
+    HostSeg seg[6];
+    for (int q = 0; q < 6; ++q) seg[q] = HostSeg{tmp.data() + q * (size_t)n, out.c[q].p, n * sizeof(double)};
+    host_copy(seg, 6, true, c.stream);
     nv = 0;
     for (int64_t i = 0; i < n; ++i)
       if (!std::isnan(tmp[i])) {
@@ -2142,9 +2149,9 @@ static void get_impl(Ctx& c, int s, int64_t cap, double* const* h, int64_t* nout
   if (b.has_invalid) {
     for (int q = 0; q < 6 && nv > 0; ++q) std::memcpy(h[q], tmp.data() + q * (size_t)n, nv * sizeof(double));
   } else {
-    for (int q = 0; q < 6 && n > 0; ++q)
-      FOPIS_HIP(hipMemcpyAsync(h[q], out.c[q].p, n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-    FOPIS_HIP(hipStreamSynchronize(c.stream));
+    HostSeg seg[6];
+    for (int q = 0; q < 6; ++q) seg[q] = HostSeg{h[q], out.c[q].p, n * sizeof(double)};
+    host_copy(seg, n > 0 ? 6 : 0, true, c.stream);
   }
   for (int q = 0; q < 6 && nh > 0; ++q) std::memcpy(h[q] + nv, b.host_inbox.c[q], nh * sizeof(double));
   for (int q = 0; q < 6; ++q)
@@ -2358,8 +2365,7 @@ static void keys_impl(Ctx& c, int s, int64_t cap, int32_t* keys, int64_t* nout) 
   DBuf<int32_t> k;
   k.alloc(n);
   k_cell_keys<R><<<div_up(n, 256), 256, 0, c.stream>>>(ptrs(flat), n, c.ny + 1, c.nz + 1, k.p);
-  FOPIS_HIP(hipMemcpyAsync(keys, k.p, n * sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
-  FOPIS_HIP(hipStreamSynchronize(c.stream));
+  copy_out(keys, k.p, n * sizeof(int32_t), c.stream);
 }
 
 void particles_cell_keys(Ctx& c, int s, int64_t cap, int32_t* keys, int64_t* n) {
