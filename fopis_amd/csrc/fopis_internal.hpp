@@ -331,7 +331,6 @@ struct Ctx {
   int mg_hist[2] = {1, 1};    // cycles of the last two solves (batch size of the next)
   int mg_tail = 0;            // first level solved by the single-workgroup LDS kernel
   size_t mg_tail_bytes = 0;   // its LDS bytes
-  size_t mg_tail_esz = 0;     // element size the tail was planned for
   std::vector<TailPlan> mg_tail_plan;  // its levels
   bool mg_tail15 = false;              // it is the cubic 15 -> 7 -> 3 -> 1 chain
   int mg_tail_elems = 0;               // LDS elements of its arrays

@@ -1584,25 +1584,6 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
   double* dst = c.mg_part.p + 2 * nb;
   int* st = c.mg_state.p;
   const int* done = st;
-  if (c.mg_tail_esz != sizeof(P)) {
-    plan_tail(c, sizeof(P));
-    c.mg_tail_esz = sizeof(P);
-    if (c.mg_fused) {
-      auto grant = [](const void* f, size_t bytes) {
-        if (bytes > 65536) FOPIS_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-      };
-      grant(reinterpret_cast<const void*>(&k_level_down<P, false>), DownDim<P, false>::kLds);
-      grant(reinterpret_cast<const void*>(&k_level_down<P, true>), DownDim<P, true>::kLds);
-      grant(reinterpret_cast<const void*>(&k_level_up<P>), UpDim<P>::kLds);
-    }
-    if (c.mg_tail < (int)c.mg.size() && c.mg_tail_bytes > 65536) {
-      FOPIS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_coarse_tail<P, false>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)c.mg_tail_bytes));
-      FOPIS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_coarse_tail<P, true>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)c.mg_tail_bytes));
-    }
-  }
-
   // level-0 FP64 residual kept by the cycle updates (the level's own array when P is double)
   double* r64 = std::is_same<P, double>::value ? reinterpret_cast<double*>(r0) : c.mg_r64.p + off;
   const int* never = st + 3;  // stays 0: the final residual always runs
@@ -1755,6 +1736,24 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
   return cycles;
 }
 
+// Plans the tail and lets the level kernels and the tail have the LDS they take.
+template <typename P>
+void plan_levels(Ctx& c) {
+  plan_tail(c, sizeof(P));
+  auto grant = [](const void* f, size_t bytes) {
+    if (bytes > 65536) FOPIS_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+  };
+  if (c.mg_fused) {
+    grant(reinterpret_cast<const void*>(&k_level_down<P, false>), DownDim<P, false>::kLds);
+    grant(reinterpret_cast<const void*>(&k_level_down<P, true>), DownDim<P, true>::kLds);
+    grant(reinterpret_cast<const void*>(&k_level_up<P>), UpDim<P>::kLds);
+  }
+  if (c.mg_tail < (int)c.mg.size()) {
+    grant(reinterpret_cast<const void*>(&k_coarse_tail<P, false>), c.mg_tail_bytes);
+    grant(reinterpret_cast<const void*>(&k_coarse_tail<P, true>), c.mg_tail_bytes);
+  }
+}
+
 }  // namespace
 
 void poisson_init(Ctx& c) {
@@ -1833,7 +1832,10 @@ void poisson_init(Ctx& c) {
   hipDeviceProp_t pr;
   FOPIS_HIP(hipGetDeviceProperties(&pr, dev));
   c.lds_max = pr.sharedMemPerBlock;
-  c.mg_tail_esz = 0;
+  if (f32)
+    plan_levels<float>(c);
+  else
+    plan_levels<double>(c);
   c.mg_hist[0] = c.mg_hist[1] = 1;
   FOPIS_HIP(hipStreamSynchronize(c.stream));
 }
