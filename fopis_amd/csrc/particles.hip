@@ -1123,11 +1123,6 @@ __global__ void k_tile_starts(const uint32_t* keys, int64_t n, int shift, uint32
   first[u] = lo;
 }
 
-__global__ void k_i32_from_i64(const int64_t* in, int32_t* out, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = (int32_t)in[i];
-}
-
 __global__ void k_counts_from_starts(const int64_t* first, uint32_t ntiles, uint32_t* cnt) {
   const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
   if (u > ntiles) return;
@@ -1179,9 +1174,171 @@ __global__ void k_fill_regions(SoaPtr<R> dst, const int64_t* start, SoaPtr<R> sr
   const int64_t pos = start[t] + (i - first[t]);
   const uint32_t j = perm[i];
   int o[3] = {0, 0, 0};
-  if (sizeof(R) == 4 && t1 > 0) tile_origin(t, t1, t2, o);
+  if (sizeof(R) == 4) tile_origin(t, t1, t2, o);
 #pragma unroll
   for (int c = 0; c < 6; ++c) dst.c[c][pos] = src.c[c][j] - (c < 3 ? (R)o[c] : (R)0);
+}
+
+// ---- staged particles into tile order (prepare_inbox)
+//
+// A stable LSD radix sort of the staged particles of every species at once
+// (blockIdx.y is the species): a step has a few thousand to a few 100 000 of
+// them, so what counts is the number of launches and the length of each one's
+// serial chain. Two digits (129^3 nodes: 4096 tiles) take five launches, one
+// digit (up to 255 tiles) three; the general sort with its copies, scans of
+// three launches each and all of it per species took 45, 120 us of a step more
+// at 33^3 (826 us, now 705), 240 at 97 x 81 x 113 with three species (2285 us,
+// now 2040). A wave keeps to its own run of items, so ranks need no barrier; a
+// scatter block forms its own offsets from the blocks' histograms.
+struct InboxArgs {
+  struct Sp {
+    const double* h;  // uploaded host-staged particles: component q at h + q * hs
+    int64_t hs, nh;
+    const double* d;  // the ones drawn on the device follow them
+    int64_t ds, n;    // n: both together
+    double* dst;
+    int64_t dsts;
+    uint32_t *key[2], *idx[2];
+    uint32_t* hist;  // [block][256]
+    int32_t* ibeg;
+    int items, nb;  // items of a thread in a block, blocks
+  } sp[FOPIS_MAX_SPECIES];
+  int N[3], T[3];
+  double xmax[3];
+  uint32_t nt;
+};
+
+// The tile of a position, nt outside the domain (those sort last and are not copied).
+__device__ __forceinline__ uint32_t tile_key(const InboxArgs& a, double x, double y, double z) {
+  const bool ok = x >= 0.0 && y >= 0.0 && z >= 0.0 && x <= a.xmax[0] && y <= a.xmax[1] && z <= a.xmax[2];
+  if (!ok) return a.nt;
+  const int ci = min((int)floor(x), a.N[0] - 1), cj = min((int)floor(y), a.N[1] - 1),
+            ck = min((int)floor(z), a.N[2] - 1);
+  return (uint32_t)(((ci / kTile) * a.T[1] + (cj / kTile)) * a.T[2] + (ck / kTile));
+}
+
+// Histogram of one digit per block; the first pass forms the keys too.
+template <bool FIRST>
+__global__ __launch_bounds__(256) void k_inbox_count(InboxArgs a, int from, int shift, uint32_t dmask) {
+  const InboxArgs::Sp& s = a.sp[blockIdx.y];
+  if ((int)blockIdx.x >= s.nb) return;
+  __shared__ uint32_t h[256];
+  h[threadIdx.x] = 0;
+  __syncthreads();
+  const int64_t base = (int64_t)blockIdx.x * s.items * 256 + threadIdx.x;
+  for (int q = 0; q < s.items; ++q) {
+    const int64_t i = base + (int64_t)q * 256;
+    if (i >= s.n) break;
+    uint32_t k;
+    if constexpr (FIRST) {
+      const double* p = i < s.nh ? s.h + i : s.d + (i - s.nh);
+      const int64_t st = i < s.nh ? s.hs : s.ds;
+      k = tile_key(a, p[0], p[st], p[2 * st]);
+      s.key[0][i] = k;
+    } else {
+      k = s.key[from][i];
+    }
+    atomicAdd(&h[(k >> shift) & dmask], 1u);
+  }
+  __syncthreads();
+  s.hist[(int64_t)blockIdx.x * 256 + threadIdx.x] = h[threadIdx.x];
+}
+
+// One digit's stable scatter from buffer `from` to the other one.
+template <bool FIRST>
+__global__ __launch_bounds__(256) void k_inbox_scatter(InboxArgs a, int from, int shift, int bits) {
+  const InboxArgs::Sp& s = a.sp[blockIdx.y];
+  if ((int)blockIdx.x >= s.nb) return;
+  __shared__ uint32_t wcnt[4][256], wsum[4];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const uint32_t dmask = (1u << bits) - 1u;
+  const uint32_t* kin = s.key[from];
+  uint32_t* kout = s.key[from ^ 1];
+  const uint32_t* vin = s.idx[from];
+  uint32_t* vout = s.idx[from ^ 1];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) wcnt[q][tid] = 0;
+  // digit tid: its count in all blocks and in the earlier ones
+  uint32_t total = 0, before = 0;
+#pragma unroll 16
+  for (int r = 0; r < s.nb; ++r) {
+    const uint32_t c = s.hist[(int64_t)r * 256 + tid];
+    total += c;
+    before += r < (int)blockIdx.x ? c : 0u;
+  }
+  __syncthreads();
+  // this wave's own run of items
+  const int64_t wbase = ((int64_t)blockIdx.x * 4 + w) * s.items * 64 + lane;
+  for (int q = 0; q < s.items; ++q) {
+    const int64_t i = wbase + (int64_t)q * 64;
+    if (i < s.n) atomicAdd(&wcnt[w][(kin[i] >> shift) & dmask], 1u);
+  }
+  uint32_t inc = total;  // inclusive over the lanes
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += t;
+  }
+  if (lane == 63) wsum[w] = inc;
+  __syncthreads();
+  uint32_t run = inc - total + before;
+  for (int q = 0; q < w; ++q) run += wsum[q];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t c = wcnt[q][tid];
+    wcnt[q][tid] = run;
+    run += c;
+  }
+  __syncthreads();
+  const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  for (int q = 0; q < s.items; ++q) {
+    const int64_t i = wbase + (int64_t)q * 64;
+    const bool act = i < s.n;
+    const uint32_t k = act ? kin[i] : 0u;
+    const uint32_t v = FIRST ? (uint32_t)i : (act ? vin[i] : 0u);
+    const uint32_t d = (k >> shift) & dmask;
+    unsigned long long m = __ballot(act);
+    for (int b = 0; b < bits; ++b) {
+      const bool bit = (d >> b) & 1u;
+      const unsigned long long bb = __ballot(bit);
+      m &= bit ? bb : ~bb;
+    }
+    // the first lane of each digit advances its offset for all of them
+    const int rank = __popcll(m & lt);
+    uint32_t at = 0;
+    if (act && rank == 0) at = atomicAdd(&wcnt[w][d], (uint32_t)__popcll(m));
+    at = __shfl(at, act ? __ffsll(m) - 1 : 0, 64);
+    if (act) {
+      kout[at + rank] = k;
+      vout[at + rank] = v;
+    }
+  }
+}
+
+// The sorted particles, and each tile's first one by binary search (ibeg[nt]
+// counts the ones inside the domain).
+__global__ __launch_bounds__(256) void k_inbox_place(InboxArgs a, int from) {
+  const InboxArgs::Sp& s = a.sp[blockIdx.y];
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const uint32_t* keys = s.key[from];
+  if (i < s.n && keys[i] < a.nt) {
+    const int64_t j = s.idx[from][i];
+    const double* p = j < s.nh ? s.h + j : s.d + (j - s.nh);
+    const int64_t st = j < s.nh ? s.hs : s.ds;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) s.dst[c * s.dsts + i] = p[c * st];
+  }
+  if (i <= (int64_t)a.nt) {
+    int64_t lo = 0, hi = s.n;
+    while (lo < hi) {
+      const int64_t mid = lo + ((hi - lo) >> 1);
+      if ((int64_t)keys[mid] < i)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    s.ibeg[i] = (int32_t)lo;
+  }
 }
 
 // Tile regions into one flat set in tile order, in absolute coordinates of
@@ -1562,6 +1719,7 @@ namespace {
 struct Scratch {
   RadixSorter sorter;
   DBuf<uint32_t> keys, perm, cnt, capa, ocapa;
+  DBuf<uint32_t> ibuf;  // keys, indices and histograms of the staged particles' sort
   DBuf<int64_t> first, tmp;
   DBuf<unsigned long long> ucount;
 };
@@ -1766,30 +1924,64 @@ void rebin(Ctx& c, int s) {
   FOPIS_HIP(hipStreamSynchronize(c.stream));
 }
 
-// Uploads the host-staged new particles and sorts them by tile.
+// Uploads the host-staged new particles of every species and sorts the staged
+// ones by tile, keeping their order inside one: host-staged first, then the
+// ones drawn on the device.
 template <class R>
-void prepare_inbox(Ctx& c, int s, bool consume) {
-  auto& b = bins<R>(c)[s];
-  const int64_t nh = (int64_t)b.host_inbox.n;
-  const int64_t n = nh + b.dev_n;
-  b.inbox_n = n;
-  if (n == 0) return;
+void prepare_inbox(Ctx& c, bool consume) {
   hipStream_t st = c.stream;
   Scratch& sc = scratch(c);
   const int nt = c.ntiles;
-  Soa<double>& raw = b.inbox_raw;
-  raw.reserve(n);
-  // host-staged particles first, then the ones drawn on the device
-  if (nh > 0) {
-    for (int q = 0; q < 6; ++q)
-      FOPIS_HIP(hipMemcpyAsync(raw.c[q].p, b.host_inbox.c[q], nh * sizeof(double), hipMemcpyHostToDevice, st));
-    b.upload_pending = true;
+  InboxArgs a{};
+  int ns = 0, nbmax = 0;
+  int64_t nmax = 0, nsum = 0, nbsum = 0;
+  for (int s = 0; s < c.S; ++s) {
+    auto& b = bins<R>(c)[s];
+    const int64_t nh = (int64_t)b.host_inbox.n, n = nh + b.dev_n;
+    b.inbox_n = n;
+    if (n == 0) continue;
+    if (n > (int64_t)0xffffffffll) throw Error(FOPIS_E_ARG, "more than 2^32 staged particles");
+    InboxArgs::Sp& e = a.sp[ns++];
+    if (nh > 0) {
+      b.inbox_raw.reserve(nh);
+      for (int q = 0; q < 6; ++q)
+        FOPIS_HIP(hipMemcpyAsync(b.inbox_raw.c[q].p, b.host_inbox.c[q], nh * sizeof(double), hipMemcpyHostToDevice, st));
+      b.upload_pending = true;
+    }
+    b.ibeg.alloc(nt + 1);
+    b.inbox.reserve(n);
+    e.h = b.inbox_raw.c[0].p;
+    e.hs = (int64_t)b.inbox_raw.size();
+    e.nh = nh;
+    e.d = b.dev_inbox.c[0].p;
+    e.ds = (int64_t)b.dev_inbox.size();
+    e.n = n;
+    e.dst = b.inbox.c[0].p;
+    e.dsts = (int64_t)b.inbox.size();
+    e.ibeg = b.ibeg.p;
+    // up to 64 blocks (a scatter block reads every block's histogram), 256 for
+    // runs of more than 2^20
+    const int most = n > ((int64_t)1 << 20) ? 256 : 64;
+    e.items = (int)((n + 256 * most - 1) / (256 * most));
+    e.nb = (int)((n + (int64_t)256 * e.items - 1) / ((int64_t)256 * e.items));
+    nbmax = std::max(nbmax, e.nb);
+    nmax = std::max(nmax, n);
+    nsum += n;
+    nbsum += e.nb;
   }
-  if (b.dev_n > 0)
-    for (int q = 0; q < 6; ++q)
-      FOPIS_HIP(hipMemcpyAsync(raw.c[q].p + nh, b.dev_inbox.c[q].p, b.dev_n * sizeof(double),
-                               hipMemcpyDeviceToDevice, st));
-  TileArgs<double> a{};
+  if (ns == 0) return;
+  sc.ibuf.alloc(std::max<size_t>(sc.ibuf.n, (size_t)(4 * nsum + 256 * nbsum)));
+  uint32_t* at = sc.ibuf.p;
+  for (int e = 0; e < ns; ++e) {
+    InboxArgs::Sp& p = a.sp[e];
+    for (int q = 0; q < 2; ++q) {
+      p.key[q] = at;
+      p.idx[q] = at + p.n;
+      at += 2 * p.n;
+    }
+    p.hist = at;
+    at += (int64_t)256 * p.nb;
+  }
   for (int q = 0; q < 3; ++q) {
     a.N[q] = c.Nc[q];
     a.T[q] = c.nt[q];
@@ -1797,29 +1989,31 @@ void prepare_inbox(Ctx& c, int s, bool consume) {
   a.xmax[0] = c.nx - 1;
   a.xmax[1] = c.ny - 1;
   a.xmax[2] = c.nz - 1;
-  sc.keys.alloc(std::max<size_t>(sc.keys.n, n));
-  sc.perm.alloc(std::max<size_t>(sc.perm.n, n));
+  a.nt = (uint32_t)nt;
   int bits = 1;
   while (((int64_t)1 << bits) < (int64_t)nt + 1) ++bits;
-  k_keys_tile<double><<<div_up(n, 256), 256, 0, st>>>(ptrs(raw), n, a, sc.keys.p, 0, (uint32_t)nt);
-  sc.sorter.sort(st, sc.keys.p, sc.perm.p, n, bits, true);
-  sc.cnt.alloc(std::max<size_t>(sc.cnt.n, nt + 1));
-  sc.first.alloc(std::max<size_t>(sc.first.n, nt + 1));
-  count_sorted_tiles(st, sc.keys.p, n, 0, nt, sc.first.p, sc.cnt.p);
-  exclusive_scan_u32(st, sc.cnt.p, nt + 1, sc.first.p, sc.tmp);
-  b.ibeg.alloc(nt + 1);
-  b.inbox.reserve(n);
-  // inbox in tile order (invalid ones sort past ibeg[nt] and are not copied)
-  k_fill_regions<double><<<div_up(n, 256), 256, 0, st>>>(ptrs(b.inbox), sc.first.p, ptrs(raw), sc.keys.p,
-                                                         sc.perm.p, n, 0, sc.first.p, (uint32_t)nt, 0, 0);
-  k_i32_from_i64<<<div_up(nt + 1, 256), 256, 0, st>>>(sc.first.p, b.ibeg.p, nt + 1);
+  const int passes = (bits + 7) / 8, width = (bits + passes - 1) / passes;
+  const dim3 grid(nbmax, ns);
+  for (int p = 0; p < passes; ++p) {
+    const int shift = p * width;
+    const uint32_t dmask = (1u << width) - 1u;
+    if (p == 0) {
+      k_inbox_count<true><<<grid, 256, 0, st>>>(a, 0, shift, dmask);
+      k_inbox_scatter<true><<<grid, 256, 0, st>>>(a, 0, shift, width);
+    } else {
+      k_inbox_count<false><<<grid, 256, 0, st>>>(a, p & 1, shift, dmask);
+      k_inbox_scatter<false><<<grid, 256, 0, st>>>(a, p & 1, shift, width);
+    }
+  }
+  k_inbox_place<<<dim3(div_up(std::max<int64_t>(nmax, (int64_t)nt + 1), 256), ns), 256, 0, st>>>(a, passes & 1);
   FOPIS_HIP(hipGetLastError());
   // the pinned staging may be refilled once the upload has been consumed by the
   // stream (the step synchronises on its status read before the next stage)
-  if (consume) {
-    b.host_inbox.n = 0;
-    b.dev_n = 0;
-  }
+  if (consume)
+    for (auto& b : bins<R>(c)) {
+      b.host_inbox.n = 0;
+      b.dev_n = 0;
+    }
 }
 
 template <class R, int MODE>
@@ -1906,7 +2100,7 @@ template <class R>
 void deposit_bin(Ctx& c, bool push) {
   hipStream_t st = c.stream;
   Phase whole(c, "particles");
-  for (int s = 0; s < c.S; ++s) prepare_inbox<R>(c, s, true);
+  prepare_inbox<R>(c, true);
   // (rho and density are written whole by the window reduction)
   FOPIS_HIP(hipMemsetAsync(c.status.p, 0, c.status.n * sizeof(int32_t), st));
   for (int o = 0; o < c.nobj; ++o)
@@ -2308,12 +2502,10 @@ void particles_ledger(Ctx& c, int s, int64_t* out) {
 }
 
 void particles_density_only(Ctx& c) {
-  for (int s = 0; s < c.S; ++s) {
-    if (c.fp32)
-      prepare_inbox<float>(c, s, false);
-    else
-      prepare_inbox<double>(c, s, false);
-  }
+  if (c.fp32)
+    prepare_inbox<float>(c, false);
+  else
+    prepare_inbox<double>(c, false);
   FOPIS_HIP(hipMemsetAsync(c.density.p, 0, c.density.n * sizeof(double), c.stream));
   for (int s = 0; s < c.S; ++s) {
     if (c.fp32)
