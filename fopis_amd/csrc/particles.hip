@@ -75,6 +75,19 @@ struct TileArgs {
   R* sink;  // kSink elements nobody reads (stores of lanes with nothing to keep)
 };
 
+// The species of one launch (blockIdx.y): the tiles of one fill a quarter of
+// the chip at 33^3 and two workgroups a CU at 65^3, and a launch costs as much
+// as a tile there. One launch for both species took the step at 33^3 (FP64, 20
+// ppc) from 705 to 634 us; at 129^3 and 257^3, where a species alone fills the
+// chip many times over, the times are the same.
+constexpr int kTileSet = 4;  // 4 sets of arguments fill a kernel's 4 KB
+template <class R>
+struct TileSet {
+  TileArgs<R> s[kTileSet];
+  int32_t* arr[kTileSet];
+};
+static_assert(sizeof(TileSet<double>) <= 4096, "kernel arguments are at most 4 KB");
+
 // ------------------------------------------------------------------ helpers
 
 __device__ __forceinline__ int fdiv(int a, int b) { return a >= 0 ? a / b : -((-a + b - 1) / b); }
@@ -445,7 +458,8 @@ __device__ __forceinline__ unsigned long long fix_weight(double v) {
 // needs a block-wide scan with two barriers per iteration so that no slot is
 // written before it has been read.
 template <class R, int MODE, bool DB = false>
-__global__ __launch_bounds__(kBlock) void k_tile(TileArgs<R> a) {
+__global__ __launch_bounds__(kBlock) void k_tile(TileSet<R> set) {
+  const TileArgs<R>& a = set.s[blockIdx.y];
   using SM = TileSmem<R, MODE>;
   __shared__ __attribute__((aligned(16))) char smem[SM::bytes];
   __shared__ int sh_rank[4 * kWaves];
@@ -1014,7 +1028,9 @@ __global__ __launch_bounds__(kBlock) void k_tile(TileArgs<R> a) {
 // past a tile's capacity go to the stray list. k_arrive_done then adds the
 // arrivals to the tiles' counts and clears them for the next step.
 template <class R>
-__global__ __launch_bounds__(kBlock) void k_scatter(TileArgs<R> a, int32_t* __restrict__ arr) {
+__global__ __launch_bounds__(kBlock) void k_scatter(TileSet<R> set) {
+  const TileArgs<R>& a = set.s[blockIdx.y];
+  int32_t* const arr = set.arr[blockIdx.y];
   const int s = blockIdx.x;
   const int sz = s % a.T[2], sy = (s / a.T[2]) % a.T[1], sx = s / (a.T[2] * a.T[1]);
   const int lane = threadIdx.x & 63;
@@ -1072,11 +1088,13 @@ __global__ __launch_bounds__(kBlock) void k_scatter(TileArgs<R> a, int32_t* __re
   }
 }
 
-__global__ void k_arrive_done(int32_t* __restrict__ cnt, const int32_t* __restrict__ capa, int32_t* __restrict__ arr,
-                              int nt) {
+template <class R>
+__global__ void k_arrive_done(TileSet<R> set, int nt) {
+  const TileArgs<R>& a = set.s[blockIdx.y];
+  int32_t* const arr = set.arr[blockIdx.y];
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nt) return;
-  cnt[t] = min(cnt[t] + arr[t], capa[t]);
+  a.cnt[t] = min(a.cnt[t] + arr[t], a.capa[t]);
   arr[t] = 0;
 }
 
@@ -2016,11 +2034,33 @@ void prepare_inbox(Ctx& c, bool consume) {
     }
 }
 
-template <class R, int MODE>
-void launch_tiles(Ctx& c, int s) {
-  TileArgs<R> a = tile_args<R>(c, s);
-  k_tile<R, MODE><<<c.ntiles, kBlock, 0, c.stream>>>(a);
+// Calls f(set, number of species) for the species that `take` picks, kTileSet
+// at a time; db: the species that bin into their second buffer.
+template <class R, class Take, class F>
+void each_set(Ctx& c, const std::vector<char>& db, Take take, F f) {
+  TileSet<R> set{};
+  int n = 0;
+  for (int s = 0; s < c.S; ++s) {
+    if (take(s)) {
+      auto& b = bins<R>(c)[s];
+      set.s[n] = tile_args<R>(c, s);
+      if (db[s]) set.s[n].dst = ptrs(b.reg2);
+      set.arr[n] = b.arr.p;
+      ++n;
+    }
+    if (n == kTileSet || (n > 0 && s + 1 == c.S)) {
+      f(set, n);
+      n = 0;
+    }
+  }
   FOPIS_HIP(hipGetLastError());
+}
+
+template <class R, int MODE>
+void launch_tiles(Ctx& c) {
+  each_set<R>(c, std::vector<char>(c.S, 0), [](int) { return true; }, [&](const TileSet<R>& set, int n) {
+    k_tile<R, MODE><<<dim3(c.ntiles, n), kBlock, 0, c.stream>>>(set);
+  });
 }
 
 // The binning pass of species s into its second region buffer (allocated on
@@ -2042,13 +2082,15 @@ bool reg2_ready(Ctx& c, int s) {
   return true;
 }
 
+// Push (when asked for), deposit and binning, into the second buffer or in place.
 template <class R, int MODE>
-void launch_tiles_db(Ctx& c, int s) {
-  auto& b = bins<R>(c)[s];
-  TileArgs<R> a = tile_args<R>(c, s);
-  a.dst = ptrs(b.reg2);
-  k_tile<R, MODE, true><<<c.ntiles, kBlock, 0, c.stream>>>(a);
-  FOPIS_HIP(hipGetLastError());
+void launch_bin(Ctx& c, const std::vector<char>& dbs) {
+  each_set<R>(c, dbs, [&](int s) { return dbs[s] != 0; }, [&](const TileSet<R>& set, int n) {
+    k_tile<R, MODE, true><<<dim3(c.ntiles, n), kBlock, 0, c.stream>>>(set);
+  });
+  each_set<R>(c, dbs, [&](int s) { return dbs[s] == 0; }, [&](const TileSet<R>& set, int n) {
+    k_tile<R, MODE><<<dim3(c.ntiles, n), kBlock, 0, c.stream>>>(set);
+  });
 }
 
 // Returns the species that deposited or counted past their tile windows.
@@ -2110,31 +2152,19 @@ void deposit_bin(Ctx& c, bool push) {
   for (int s = 0; s < c.S; ++s) dbs[s] = c.tile_double_buffer && reg2_ready<R>(c, s);
   {
     Phase ph(c, "tile");
-    for (int s = 0; s < c.S; ++s) {
-      if (dbs[s]) {
-        if (push)
-          launch_tiles_db<R, M_VEL | M_POS | M_DEP | M_BIN>(c, s);
-        else
-          launch_tiles_db<R, M_DEP | M_BIN>(c, s);
-      } else {
-        if (push)
-          launch_tiles<R, M_VEL | M_POS | M_DEP | M_BIN>(c, s);
-        else
-          launch_tiles<R, M_DEP | M_BIN>(c, s);
-      }
-    }
+    if (push)
+      launch_bin<R, M_VEL | M_POS | M_DEP | M_BIN>(c, dbs);
+    else
+      launch_bin<R, M_DEP | M_BIN>(c, dbs);
   }
   {
     Phase ph(c, "bin");
-    for (int s = 0; s < c.S; ++s) {
-      auto& b = bins<R>(c)[s];
-      TileArgs<R> a = tile_args<R>(c, s);
-      if (dbs[s]) a.dst = ptrs(b.reg2);
-      k_scatter<R><<<c.ntiles, kBlock, 0, st>>>(a, b.arr.p);
-      k_arrive_done<<<div_up(c.ntiles, 256), 256, 0, st>>>(b.cnt.p, b.capa.p, b.arr.p, c.ntiles);
-      if (dbs[s]) b.reg.swap(b.reg2);
-    }
-    FOPIS_HIP(hipGetLastError());
+    each_set<R>(c, dbs, [](int) { return true; }, [&](const TileSet<R>& set, int n) {
+      k_scatter<R><<<dim3(c.ntiles, n), kBlock, 0, st>>>(set);
+      k_arrive_done<R><<<dim3(div_up(c.ntiles, 256), n), 256, 0, st>>>(set, c.ntiles);
+    });
+    for (int s = 0; s < c.S; ++s)
+      if (dbs[s]) bins<R>(c)[s].reg.swap(bins<R>(c)[s].reg2);
   }
   for (int s = 0; s < c.S; ++s) {
     bins<R>(c)[s].inbox_n = 0;
@@ -2456,27 +2486,21 @@ void particles_emit(Ctx& c, int o, int s, int axis, int sign, int per_node, doub
 
 void particles_velocity(Ctx& c) {
   Phase ph(c, "velocity");
-  for (int s = 0; s < c.S; ++s) {
-    if (c.fp32)
-      launch_tiles<float, M_VEL>(c, s);
-    else
-      launch_tiles<double, M_VEL>(c, s);
-  }
+  if (c.fp32)
+    launch_tiles<float, M_VEL>(c);
+  else
+    launch_tiles<double, M_VEL>(c);
 }
 
 void particles_position(Ctx& c) {
   {
     Phase ph(c, "position");
     FOPIS_HIP(hipMemsetAsync(c.status.p, 0, c.status.n * sizeof(int32_t), c.stream));
-    for (int s = 0; s < c.S; ++s) {
-      if (c.fp32) {
-        launch_tiles<float, M_POS>(c, s);
-        c.sp32[s].has_invalid = true;
-      } else {
-        launch_tiles<double, M_POS>(c, s);
-        c.sp64[s].has_invalid = true;
-      }
-    }
+    if (c.fp32)
+      launch_tiles<float, M_POS>(c);
+    else
+      launch_tiles<double, M_POS>(c);
+    for (int s = 0; s < c.S; ++s) (c.fp32 ? c.sp32[s].has_invalid : c.sp64[s].has_invalid) = true;
   }
   std::vector<int32_t> stat(kStat * c.S);
   FOPIS_HIP(hipMemcpyAsync(stat.data(), c.status.p, stat.size() * sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
@@ -2507,12 +2531,10 @@ void particles_density_only(Ctx& c) {
   else
     prepare_inbox<double>(c, false);
   FOPIS_HIP(hipMemsetAsync(c.density.p, 0, c.density.n * sizeof(double), c.stream));
-  for (int s = 0; s < c.S; ++s) {
-    if (c.fp32)
-      launch_tiles<float, M_DENS>(c, s);
-    else
-      launch_tiles<double, M_DENS>(c, s);
-  }
+  if (c.fp32)
+    launch_tiles<float, M_DENS>(c);
+  else
+    launch_tiles<double, M_DENS>(c);
   for (int s = 0; s < c.S; ++s) {
     if (c.fp32)
       c.sp32[s].inbox_n = 0;
