@@ -129,6 +129,24 @@ struct SoaPtr {
   R* c[6];
 };
 
+// A fixed piece of pinned host memory that kernels write.
+struct PinBuf {
+  void* p = nullptr;
+  PinBuf() = default;
+  PinBuf(const PinBuf&) = delete;
+  PinBuf& operator=(const PinBuf&) = delete;
+  ~PinBuf() {
+    if (p) (void)hipHostFree(p);
+  }
+  void alloc(size_t bytes) {
+    if (p) return;
+    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
+      p = nullptr;
+      throw Error(FOPIS_E_NOMEM, "pinned host allocation failed");
+    }
+  }
+};
+
 // Growable pinned host staging of particles added on the host (six FP64
 // components), so that their upload is an asynchronous DMA.
 struct PinSoa {
@@ -310,7 +328,8 @@ struct Ctx {
   DBuf<double> psi;            // conductor response of the last step: phi after minus phi before the charge
   int psi_step = -1;           // step that formed psi (-1: none)
   bool carry = true;           // warm starts from psi (FOPIS_CARRY=0: the previous phi for both solves)
-  DBuf<int32_t> mg_state;     // [4] solve flag and cycle count on the device
+  DBuf<int32_t> mg_state;     // [8] solve flags and counts on the device
+  PinBuf mg_words;            // what the host reads of them
   DBuf<double> mg_part;       // per-block residual partials and the norms of the solve (fixed address)
   // captured once: [0] one V-cycle + FP64 update + norm check, [1] two
   // V-cycles (the second continuing from the first's correction) + update + check

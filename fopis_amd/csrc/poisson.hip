@@ -110,17 +110,13 @@ __global__ __launch_bounds__(256) void k_resid0(const double* __restrict__ phi, 
   }
 }
 
-// Solve state on the device: st[0] done flag, st[1] cycles applied, st[3]
-// stays 0 (the done flag of launches that always run), st[4] the current
-// pair's skip flag, st[5] FP64 updates applied, st[6] pair residual passes
-// run; dst[0..2] = ||r||^2, ||b||^2, relative residual of the
-// last check, dst[3] the relative residual the solve started from.
-__global__ void k_solve_begin(int* st) {
-  st[0] = 0;
-  st[1] = 0;
-  st[5] = 0;
-  st[6] = 0;
-}
+// Solve state on the device: st[0] done flag, st[1] cycles applied, st[2] 0
+// once the true residual has confirmed the end, st[3] stays 0 (the done flag of
+// launches that always run), st[4] the current pair's skip flag, st[5] FP64
+// updates applied, st[6] pair residual passes run, st[7] the opposite of st[0]
+// (the done flag of launches that run once the cycles are done); dst[0..2] =
+// ||r||^2, ||b||^2, relative residual of the last check, dst[3] the relative
+// residual the solve started from. The first check of a solve sets them.
 
 // After a V-cycle's correction e: phi += e and the FP64 residual
 // r = b - A phi is updated as r -= A e (exact up to FP64 rounding, so no
@@ -209,15 +205,8 @@ __global__ __launch_bounds__(256) void k_pair_check(const double* part, int nb, 
   }
 }
 
-// Final sum of the residual partials (one block, fixed tree: deterministic),
-// cycle count and the stopping test of the solve loop. keep_bb: ||b||^2 is
-// the one already in dst[1] (the partials carry r^2 only). count_cycle V-cycles
-// were applied, less one when *skipped (a pair whose second cycle was skipped).
-__global__ __launch_bounds__(256) void k_norm(const double* part, int nb, double* dst, int* st, double tol,
-                                              int max_cycles, int count_cycle, int keep_bb,
-                                              const int* skipped = nullptr) {
-  if (st[0]) return;
-  __shared__ double s1[256], s2[256];
+// Sums of the residual partials over a block (fixed tree: deterministic), in s1[0] and s2[0].
+__device__ __forceinline__ void sum_partials(const double* part, int nb, double* s1, double* s2) {
   double a = 0.0, b = 0.0;
   for (int i = threadIdx.x; i < nb; i += 256) {
     a += part[2 * i];
@@ -233,48 +222,76 @@ __global__ __launch_bounds__(256) void k_norm(const double* part, int nb, double
     }
     __syncthreads();
   }
+}
+
+// Cycle count and the stopping test of the solve loop. FIRST: of the residual
+// the solve starts from, which also sets the solve's state. The others keep
+// the ||b||^2 in dst[1] (their partials carry r^2 only); count_cycle V-cycles
+// were applied, less one when *skipped (a pair whose second cycle was skipped).
+template <bool FIRST>
+__global__ __launch_bounds__(256) void k_norm(const double* part, int nb, double* dst, int* st, double tol,
+                                              int max_cycles, int count_cycle, const int* skipped) {
+  if (!FIRST && st[0]) return;
+  __shared__ double s1[256], s2[256];
+  sum_partials(part, nb, s1, s2);
   if (threadIdx.x == 0) {
-    const double rr = s1[0], bb = keep_bb ? dst[1] : s2[0];
-    const int cyc = st[1] + count_cycle - (skipped ? skipped[0] : 0);
-    if (count_cycle > 0) st[5] += 1;  // an FP64 update preceded this check
+    const double rr = s1[0], bb = FIRST ? s2[0] : dst[1];
+    const int cyc = FIRST ? 0 : st[1] + count_cycle - (skipped ? skipped[0] : 0);
     const double rel = bb > 0.0 ? sqrt(rr / bb) : sqrt(rr);
     dst[0] = rr;
     dst[1] = bb;
     dst[2] = rel;
+    if (FIRST) dst[3] = rel;
+    const int end = (rel <= tol || (bb == 0.0 && rr < 1e-300) || cyc >= max_cycles) ? 1 : 0;
+    st[0] = end;
     st[1] = cyc;
-    st[0] = (rel <= tol || (bb == 0.0 && rr < 1e-300) || cyc >= max_cycles) ? 1 : 0;
+    if (FIRST) st[2] = 1;
+    st[5] = FIRST ? 0 : st[5] + 1;  // an FP64 update preceded this check
+    if (FIRST) st[6] = 0;
+    st[7] = 1 - end;
   }
 }
 
-// The true residual's norms at the end of a solve (flag untouched).
-__global__ __launch_bounds__(256) void k_norm_final(const double* part, int nb, double* dst) {
+// What the host reads after a round of cycles (pinned memory it and the device share).
+struct SolveWords {
+  int32_t done, confirmed, cycles, updates, pair_passes;
+  double relres, relres0;
+};
+
+// Once the cycles are done: the true residual's norms, and whether they confirm
+// the end. The words go to the host directly; with two
+// copies, a second wait and a launch per face a solve took 47 to 70 us more
+// (33^3: step 634 us, now 587; 17^3 alone: 379 us, now 310).
+__global__ __launch_bounds__(256) void k_norm_final(const double* part, int nb, double* dst, int* st, double tol,
+                                                    int max_cycles, SolveWords* out) {
   __shared__ double s1[256], s2[256];
-  double a = 0.0, b = 0.0;
-  for (int i = threadIdx.x; i < nb; i += 256) {
-    a += part[2 * i];
-    b += part[2 * i + 1];
-  }
-  s1[threadIdx.x] = a;
-  s2[threadIdx.x] = b;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) {
-      s1[threadIdx.x] += s1[threadIdx.x + o];
-      s2[threadIdx.x] += s2[threadIdx.x + o];
-    }
-    __syncthreads();
-  }
+  const int done = st[0];
+  if (done) sum_partials(part, nb, s1, s2);
   if (threadIdx.x == 0) {
-    dst[0] = s1[0];
-    dst[1] = s2[0];
-    dst[2] = s2[0] > 0.0 ? sqrt(s1[0] / s2[0]) : sqrt(s1[0]);
+    int good = 0;
+    if (done) {
+      const double rr = s1[0], bb = s2[0];
+      const double rel = bb > 0.0 ? sqrt(rr / bb) : sqrt(rr);
+      dst[0] = rr;
+      dst[1] = bb;
+      dst[2] = rel;
+      good = (rel <= tol || (bb == 0.0 && rr < 1e-300) || st[1] >= max_cycles) ? 1 : 0;
+    }
+    st[2] = 1 - good;
+    out->done = done;
+    out->confirmed = good;
+    out->cycles = st[1];
+    out->updates = st[5];
+    out->pair_passes = st[6];
+    out->relres = dst[2];
+    out->relres0 = dst[3];
   }
 }
 
-__global__ void k_reopen(int* st) { st[0] = 0; }
-
-// The relative residual the solve starts from, kept beside the running norms.
-__global__ void k_keep_start(double* dst) { dst[3] = dst[2]; }
+__global__ void k_reopen(int* st) {
+  st[0] = 0;
+  st[7] = 1;
+}
 
 // Kernels over a level's interior give each thread the same column position
 // in kRows consecutive rows (b), issue every load of those rows before the
@@ -1252,37 +1269,35 @@ __global__ __launch_bounds__(kTailThreads) void k_coarse_tail(TailArgs<P> A) {
   for (int q = threadIdx.x; q < L0.count; q += kTailThreads) A.ge[A.gidx[q]] = s[L0.oe + tab[L0.list + q]];
 }
 
-// Face conditions on phi (Field.cpp:10-96): D -> 0, N -> copy the neighbour.
-__global__ void k_face(double* phi, int cx, int cy, int cz, int axis, int side, int neumann) {
-  const int u = blockIdx.x * blockDim.x + threadIdx.x;
-  const int v = blockIdx.y;
-  int nu, nv;
-  if (axis == 0) {
-    nu = cz - 2;
-    nv = cy - 2;
-  } else if (axis == 1) {
-    nu = cz - 2;
-    nv = cx - 2;
-  } else {
-    nu = cy - 2;
-    nv = cx - 2;
+// Face conditions on phi (Field.cpp:10-96): D -> 0, N -> copy the neighbour,
+// in the reference's order (x low and up, y, z), where a later face takes what
+// an earlier one left on a shared edge. A thread finds its
+// node's final value instead: from the last face down, D gives 0 and N steps
+// inwards, to a node that no face writes. So the six (blockIdx.z) take one
+// launch, not six in order. unconfirmed: nothing is done while the solve goes on.
+struct FaceKinds {
+  char k[6];
+};
+__global__ void k_faces(double* phi, int cx, int cy, int cz, FaceKinds bc, const int* unconfirmed) {
+  if (*unconfirmed) return;
+  const int f = blockIdx.z, axis = f >> 1;
+  const int n[3] = {cx, cy, cz};
+  const int ua = axis == 2 ? 1 : 2, va = axis == 0 ? 1 : 0;
+  const int u = blockIdx.x * blockDim.x + threadIdx.x, v = blockIdx.y;
+  if (u >= n[ua] - 2 || v >= n[va] - 2) return;
+  int at[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) at[q] = q == axis ? ((f & 1) ? n[q] - 2 : 1) : (q == ua ? u + 1 : v + 1);
+  const int64_t t = ((int64_t)at[0] * cy + at[1]) * cz + at[2];
+  bool zero = false;
+#pragma unroll
+  for (int q = 2; q >= 0; --q) {
+    const bool low = at[q] == 1;
+    if (!low && at[q] != n[q] - 2) continue;
+    zero = zero || bc.k[2 * q + (low ? 0 : 1)] != 'N';
+    if (!zero) at[q] += low ? 1 : -1;
   }
-  if (u >= nu || v >= nv) return;
-  const int nmax = axis == 0 ? cx : (axis == 1 ? cy : cz);
-  const int bi = side == 0 ? 1 : nmax - 2, ni = side == 0 ? 2 : nmax - 3;
-  int64_t t, s;
-  const int64_t sI = (int64_t)cy * cz, sJ = cz;
-  if (axis == 0) {
-    t = bi * sI + (v + 1) * sJ + (u + 1);
-    s = ni * sI + (v + 1) * sJ + (u + 1);
-  } else if (axis == 1) {
-    t = (v + 1) * sI + bi * sJ + (u + 1);
-    s = (v + 1) * sI + ni * sJ + (u + 1);
-  } else {
-    t = (v + 1) * sI + (u + 1) * sJ + bi;
-    s = (v + 1) * sI + (u + 1) * sJ + ni;
-  }
-  phi[t] = neumann ? phi[s] : 0.0;
+  phi[t] = zero ? 0.0 : phi[((int64_t)at[0] * cy + at[1]) * cz + at[2]];
 }
 
 Lv lv_of(const MgLevel& m) { return Lv{m.n[0], m.n[1], m.n[2], m.sx, m.sy}; }
@@ -1587,7 +1602,6 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
   // level-0 FP64 residual kept by the cycle updates (the level's own array when P is double)
   double* r64 = std::is_same<P, double>::value ? reinterpret_cast<double*>(r0) : c.mg_r64.p + off;
   const int* never = st + 3;  // stays 0: the final residual always runs
-  k_solve_begin<<<1, 1, 0, c.stream>>>(st);
   // the level-0 passes, on the colour-split arrays when the level has them
   bool rb = false;
   if constexpr (std::is_same<P, float>::value) rb = c.mg_rb;
@@ -1601,9 +1615,8 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
     k_resid0<P><<<nb, 256, 0, c.stream>>>(phi, rho, rc, store ? r0 : (P*)nullptr, L0, part, flag,
                                           store ? r64 : (double*)nullptr);
   };
-  resid0(true, done);
-  k_norm<<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, max_cycles, 0, 0);
-  k_keep_start<<<1, 1, 0, c.stream>>>(dst);
+  resid0(true, never);
+  k_norm<true><<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, max_cycles, 0, nullptr);
   // Queue as many cycles as the previous two solves needed, then more. With
   // pairs, two V-cycles share one FP64 update and norm check: the second
   // runs on the same right-hand side, continuing from the first's correction
@@ -1620,8 +1633,11 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
   const bool pairs = c.mg_pairs && c.mg_tail > 0 && (int)c.mg.size() > 1;
   int npair = pairs ? pred / 2 : 0;
   int batch = pred - 2 * npair;
-  int32_t hs[7];
-  double hd[4];
+  SolveWords* const words = reinterpret_cast<SolveWords*>(c.mg_words.p);
+  FaceKinds faces;
+  for (int f = 0; f < 6; ++f) faces.k[f] = c.d.boundary[f];
+  // (u runs along z, or y on the z faces; v along y or x)
+  const dim3 face_grid(div_up(std::max(c.cy, c.cz) - 2, 64), std::max(c.cx, c.cy) - 2, 6);
   int* skip = st + 4;
   // One cycle (or pair): the V-cycle(s), the FP64 update and the norm
   // check. Their ~30 (~60) launches are captured once into a graph of kernel
@@ -1650,7 +1666,7 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
     } else {
       k_update<P><<<nb, 256, 0, c.stream>>>(phi, e, r64, r0, L0, part, done);
     }
-    k_norm<<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, max_cycles, nv, 1, nv == 2 ? skip : nullptr);
+    k_norm<false><<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, max_cycles, nv, nv == 2 ? skip : nullptr);
   };
   if (c.mg_use_graph && (!c.mg_graph[0] || c.mg_graph_esz != sizeof(P) || c.mg_graph_tol != tol ||
                          c.mg_graph_cap != max_cycles)) {
@@ -1692,47 +1708,27 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
       npair = 0;
       batch = 2;
     }
-    FOPIS_HIP(hipMemcpyAsync(hs, st, sizeof(hs), hipMemcpyDeviceToHost, c.stream));
+    // once done, the true residual b - A phi confirms the end and the face
+    // conditions follow, all queued before the one wait of the round
+    resid0(false, st + 7);
+    k_norm_final<<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, max_cycles, words);
+    k_faces<<<face_grid, 64, 0, c.stream>>>(c.phi.p, c.cx, c.cy, c.cz, faces, st + 2);
+    FOPIS_HIP(hipGetLastError());
     FOPIS_HIP(hipStreamSynchronize(c.stream));
-    if (!hs[0]) continue;
-    // confirm on the true residual b - A phi before stopping
-    resid0(false, never);
-    k_norm_final<<<1, 256, 0, c.stream>>>(part, nb, dst);
-    FOPIS_HIP(hipMemcpyAsync(hd, dst, sizeof(hd), hipMemcpyDeviceToHost, c.stream));
-    FOPIS_HIP(hipStreamSynchronize(c.stream));
-    const bool zero_rhs = hd[1] == 0.0 && hd[0] < 1e-300;
-    if (hd[2] <= tol || zero_rhs || hs[1] >= max_cycles) break;
+    if (!words->done) continue;
+    if (words->confirmed) break;
     // the recursively updated residual has drifted from the true one: the
     // further cycles start from the true residual
     resid0(true, never);
     k_reopen<<<1, 1, 0, c.stream>>>(st);
   }
-  const int cycles = hs[1];
-  c.mg_updates_last = hs[5];
-  c.mg_pair_passes_last = hs[6];
+  const int cycles = words->cycles;
+  c.mg_updates_last = words->updates;
+  c.mg_pair_passes_last = words->pair_passes;
   c.mg_hist[1] = c.mg_hist[0];
   c.mg_hist[0] = cycles;
-  // face conditions in the reference's order: x low/up, y, z
-  for (int axis = 0; axis < 3; ++axis)
-    for (int side = 0; side < 2; ++side) {
-      const char bcc = c.d.boundary[2 * axis + side];
-      if (bcc == 'P') continue;
-      int nu, nv;
-      if (axis == 0) {
-        nu = c.cz - 2;
-        nv = c.cy - 2;
-      } else if (axis == 1) {
-        nu = c.cz - 2;
-        nv = c.cx - 2;
-      } else {
-        nu = c.cy - 2;
-        nv = c.cx - 2;
-      }
-      k_face<<<dim3(div_up(nu, 64), nv), 64, 0, c.stream>>>(c.phi.p, c.cx, c.cy, c.cz, axis, side, bcc == 'N');
-    }
-  FOPIS_HIP(hipGetLastError());
-  *relres_out = hd[2];
-  c.relres0_last = hd[3];
+  *relres_out = words->relres;
+  c.relres0_last = words->relres0;
   return cycles;
 }
 
@@ -1818,6 +1814,7 @@ void poisson_init(Ctx& c) {
     FOPIS_HIP(hipMemsetAsync(c.erb.p, 0, 2 * c.rb_cs * sizeof(float), c.stream));
     FOPIS_HIP(hipMemsetAsync(c.rrb.p, 0, 2 * c.rb_cs * sizeof(float), c.stream));
   }
+  c.mg_words.alloc(sizeof(SolveWords));
   c.mg_state.alloc(8);
   FOPIS_HIP(hipMemsetAsync(c.mg_state.p, 0, 8 * sizeof(int32_t), c.stream));
   c.mg_part.alloc(2 * kResidBlocks + 4);
