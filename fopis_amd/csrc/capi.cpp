@@ -369,8 +369,7 @@ int fopis_energy(fopis_ctx* ctx, double* out) {
   NEED_CTX
   return guarded([&] {
     if (!out) throw Error(FOPIS_E_ARG, "null output");
-    out[0] = particles_energy(ctx->c);
-    out[1] = fields_energy(ctx->c);
+    energy(ctx->c, out);
   });
 }
 

@@ -143,46 +143,6 @@ __global__ void k_edge(const double* __restrict__ phi, double* __restrict__ out,
   out[g] = (phi[p] - phi[p + d]) * (1.0 / 1.0);
 }
 
-// Sum of squared edge fields over Field::getEfieldEnergy's index ranges.
-__global__ __launch_bounds__(256) void k_efield_energy(const double* __restrict__ phi, int cx, int cy, int cz,
-                                                       double* part) {
-  __shared__ double s[256];
-  const int64_t nn = (int64_t)cx * cy * cz, sI = (int64_t)cy * cz, sJ = cz;
-  double acc = 0.0;
-  for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < nn; g += (int64_t)gridDim.x * 256) {
-    const int k = (int)(g % cz), j = (int)((g / cz) % cy), i = (int)(g / sI);
-    if (i < 1 || i > cx - 2 || j < 1 || j > cy - 2 || k < 1 || k > cz - 2) continue;
-    const double p = phi[g];
-    if (i < cx - 2) {
-      const double e = (p - phi[g + sI]);
-      acc += e * e;
-    }
-    if (j < cy - 2) {
-      const double e = (p - phi[g + sJ]);
-      acc += e * e;
-    }
-    if (k < cz - 2) {
-      const double e = (p - phi[g + 1]);
-      acc += e * e;
-    }
-  }
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = s[0];
-}
-
-__global__ void k_serial_sum(const double* part, int n, double* out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < n; ++i) s += part[i];
-    *out = s;
-  }
-}
-
 Faces faces(const Ctx& c) {
   Faces f;
   for (int q = 0; q < 6; ++q) f.b[q] = c.d.boundary[q] != 'P';
@@ -287,21 +247,6 @@ void fields_set(Ctx& c, int which, int s, const double* in) {
   if (which >= FOPIS_EX && which <= FOPIS_EZ) throw Error(FOPIS_E_ARG, "edge fields are derived from phi");
   const size_t n = field_len(c, which);
   copy_in(field_ptr(c, which, s), in, n * sizeof(double), c.stream);
-}
-
-void fields_energy_queue(Ctx& c, double* part, double* sum) {
-  k_efield_energy<<<kEnergyBlocks, 256, 0, c.stream>>>(c.phi.p, c.cx, c.cy, c.cz, part);
-  k_serial_sum<<<1, 1, 0, c.stream>>>(part, kEnergyBlocks, sum);
-  FOPIS_HIP(hipGetLastError());
-}
-
-double fields_energy(Ctx& c) {
-  c.red.alloc(std::max<size_t>(c.red.n, kEnergyBlocks + 1));
-  fields_energy_queue(c, c.red.p, c.red.p + kEnergyBlocks);
-  double e = 0.0;
-  FOPIS_HIP(hipMemcpyAsync(&e, c.red.p + kEnergyBlocks, sizeof(double), hipMemcpyDeviceToHost, c.stream));
-  FOPIS_HIP(hipStreamSynchronize(c.stream));
-  return 0.5 * c.d.eps0 * e;
 }
 
 }  // namespace fopis

@@ -330,6 +330,7 @@ struct Ctx {
   bool carry = true;           // warm starts from psi (FOPIS_CARRY=0: the previous phi for both solves)
   DBuf<int32_t> mg_state;     // [8] solve flags and counts on the device
   PinBuf mg_words;            // what the host reads of them
+  PinBuf energy_words;        // the energy sums, on the host
   DBuf<double> mg_part;       // per-block residual partials and the norms of the solve (fixed address)
   // captured once: [0] one V-cycle + FP64 update + norm check, [1] two
   // V-cycles (the second continuing from the first's correction) + update + check
@@ -395,13 +396,10 @@ void particles_density_only(Ctx& c);
 void particles_deposit_bin(Ctx& c, bool push);
 void particles_sort_by_cell(Ctx& c);
 void particles_cell_keys(Ctx& c, int s, int64_t cap, int32_t* keys, int64_t* n);
-double particles_energy(Ctx& c);
 // Energy reductions: kEnergyBlocks partials per quantity, summed in a fixed order.
 constexpr int kEnergyBlocks = 1024;
-// Queues sum v^2 of every species into sums[s] (part: S * kEnergyBlocks doubles).
-void particles_energy_queue(Ctx& c, double* part, double* sums);
-// 1/2 sum_s m_s size_s v2[s].
-double particles_energy_from(const Ctx& c, const double* v2);
+// Kinetic energy of all species and field energy.
+void energy(Ctx& c, double* out);
 // Device address of this device's scratch array (set up once per device, with it current).
 void noalloc_setup(Ctx& c);
 // fopis_energy computed with the partials in that array (allocates nothing).
@@ -415,9 +413,6 @@ void fields_efield(Ctx& c);
 void fields_reduce_windows(Ctx& c, bool do_rho, bool do_dens, uint32_t far_mask = ~0u);
 void fields_get(Ctx& c, int which, int s, double* out);
 void fields_set(Ctx& c, int which, int s, const double* in);
-double fields_energy(Ctx& c);
-// Queues the sum of squared edge fields into *sum (part: kEnergyBlocks doubles).
-void fields_energy_queue(Ctx& c, double* part, double* sum);
 
 void poisson_init(Ctx& c);
 void poisson_free(Ctx& c);

@@ -1418,33 +1418,110 @@ __global__ void k_cell_keys(SoaPtr<R> f, int64_t n, int ny1, int nz1, int32_t* k
   keys[i] = (ci * ny1 + cj) * nz1 + ck;
 }
 
-// sum of v^2 over n particles into per-block partials
-// Sum of vx^2 + vy^2 + vz^2 (FP64) over the live particles of the tile
-// regions, read in place: a fixed grid of workgroups strides over the tiles
-// and each writes one partial. A particle that a standalone position update
-// absorbed keeps its slot with x = NaN until the next re-bin;
-// Grid::getParticleEnergy skips it (GridParticleTreatment.cpp:104-118).
+// Energies: row s of the grid sums vx^2 + vy^2 + vz^2 (FP64) over the live
+// particles of species s in their tile regions, the last row the squared edge
+// fields over Field::getEfieldEnergy's index ranges; each workgroup writes one
+// partial and k_energy_sum adds those, in fixed orders. A tile is shared by
+// `split` workgroups where the tiles alone would not fill the row, and a thread
+// has four particles' loads in flight (the reads bound it: 129^3 with 64 ppc,
+// FP64: 2 x 784 us with one particle in flight and x always read, 1089 us both now).
+// A particle that a standalone position update absorbed keeps its slot with
+// x = NaN until the next re-bin; Grid::getParticleEnergy skips it
+// (GridParticleTreatment.cpp:104-118): x is read only where there may be one.
 template <class R>
-__global__ __launch_bounds__(kBlock) void k_v2_tiles(SoaPtr<R> f, const int64_t* start, const int32_t* cnt,
-                                                     int ntiles, double* part) {
-  __shared__ double s[kBlock];
+struct EnergyArgs {
+  struct Sp {
+    const R *x, *vx, *vy, *vz;  // x: null where every slot is live
+    const int64_t* start;
+    const int32_t* cnt;
+  } sp[FOPIS_MAX_SPECIES];
+  int ns, ntiles, split;
+  const double* phi;
+  int cx, cy, cz;
+};
+
+template <class R>
+__device__ __forceinline__ double sum_v2(const EnergyArgs<R>& a, int row) {
+  const typename EnergyArgs<R>::Sp& f = a.sp[row];
   double acc = 0.0;
-  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const int64_t b0 = start[t];
-    const int n = cnt[t];
-    for (int i = threadIdx.x; i < n; i += kBlock) {
-      if (isnan(f.c[0][b0 + i])) continue;
-      const double vx = f.c[3][b0 + i], vy = f.c[4][b0 + i], vz = f.c[5][b0 + i];
-      acc += vx * vx + vy * vy + vz * vz;
+  auto tile = [&](auto check, int t, int q) {
+    const int64_t b0 = f.start[t];
+    const int n = f.cnt[t], step = a.split * kBlock;
+    for (int i = q * kBlock + threadIdx.x; i < n; i += 4 * step) {
+      R v[4][3], x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t j = b0 + min(i + u * step, n - 1);
+        v[u][0] = f.vx[j];
+        v[u][1] = f.vy[j];
+        v[u][2] = f.vz[j];
+        x[u] = decltype(check)::value ? f.x[j] : (R)0;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const double vx = v[u][0], vy = v[u][1], vz = v[u][2];
+        if (i + u * step < n && !isnan(x[u])) acc += vx * vx + vy * vy + vz * vz;
+      }
     }
+  };
+  const int items = a.ntiles * a.split;
+  for (int w = blockIdx.x; w < items; w += gridDim.x) {
+    if (f.x)
+      tile(std::true_type{}, w / a.split, w % a.split);
+    else
+      tile(std::false_type{}, w / a.split, w % a.split);
   }
-  s[threadIdx.x] = acc;
+  return acc;
+}
+
+template <class R>
+__device__ __forceinline__ double sum_field(const EnergyArgs<R>& a) {
+  const double* __restrict__ phi = a.phi;
+  const int cx = a.cx, cy = a.cy, cz = a.cz;
+  const int64_t nn = (int64_t)cx * cy * cz, sI = (int64_t)cy * cz, sJ = cz;
+  double acc = 0.0;
+  for (int64_t g = (int64_t)blockIdx.x * kBlock + threadIdx.x; g < nn; g += (int64_t)gridDim.x * kBlock) {
+    const int k = (int)(g % cz), j = (int)((g / cz) % cy), i = (int)(g / sI);
+    if (i < 1 || i > cx - 2 || j < 1 || j > cy - 2 || k < 1 || k > cz - 2) continue;
+    const double p = phi[g];
+    const double ex = i < cx - 2 ? p - phi[g + sI] : 0.0;
+    const double ey = j < cy - 2 ? p - phi[g + sJ] : 0.0;
+    const double ez = k < cz - 2 ? p - phi[g + 1] : 0.0;
+    acc += ex * ex;
+    acc += ey * ey;
+    acc += ez * ez;
+  }
+  return acc;
+}
+
+__device__ __forceinline__ double block_sum(double v, double* s) {
+  s[threadIdx.x] = v;
   __syncthreads();
   for (int o = kBlock / 2; o > 0; o >>= 1) {
     if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = s[0];
+  return s[0];
+}
+
+template <class R>
+__global__ __launch_bounds__(kBlock) void k_energy(EnergyArgs<R> a, double* part) {
+  __shared__ double s[kBlock];
+  const double acc = (int)blockIdx.y < a.ns ? sum_v2(a, blockIdx.y) : sum_field(a);
+  const double sum = block_sum(acc, s);
+  if (threadIdx.x == 0) part[(size_t)blockIdx.y * kEnergyBlocks + blockIdx.x] = sum;
+}
+
+// One workgroup per row (53 us per row with one thread); the sums go to pinned
+// host memory.
+__global__ __launch_bounds__(kBlock) void k_energy_sum(const double* part, double* out) {
+  __shared__ double s[kBlock];
+  double acc = 0.0;
+#pragma unroll
+  for (int q = 0; q < kEnergyBlocks / kBlock; ++q)
+    acc += part[(size_t)blockIdx.x * kEnergyBlocks + q * kBlock + threadIdx.x];
+  const double sum = block_sum(acc, s);
+  if (threadIdx.x == 0) out[blockIdx.x] = sum;
 }
 
 // Per-tile sums of x, y, z, vx, vy, vz and vx^2, vy^2, vz^2 (FP64) over the
@@ -1486,14 +1563,6 @@ __global__ __launch_bounds__(kBlock) void k_count_valid(const R* x, const int64_
   for (int i = threadIdx.x; i < n; i += kBlock) k += isnan(x[b0 + i]) ? 0 : 1;
   for (int o = 32; o > 0; o >>= 1) k += __shfl_xor(k, o);
   if ((threadIdx.x & 63) == 0 && k) atomicAdd(out, (unsigned long long)k);
-}
-
-__global__ void k_sum_serial(const double* part, int n, double* out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < n; ++i) s += part[i];
-    *out = s;
-  }
 }
 
 // ------------------------------------------------------- device generator
@@ -2199,6 +2268,7 @@ void particles_init(Ctx& c) {
   c.status.alloc(kStat * FOPIS_MAX_SPECIES);
   FOPIS_HIP(hipMemsetAsync(c.status.p, 0, c.status.n * sizeof(int32_t), c.stream));
   noalloc_setup(c);
+  c.energy_words.alloc((FOPIS_MAX_SPECIES + 1) * sizeof(double));
   for (int s = 0; s < c.S; ++s) {
     if (c.fp32)
       bin_flat<float>(c, s, c.sp32[s].reg, 0, false);
@@ -2589,51 +2659,46 @@ void particles_cell_keys(Ctx& c, int s, int64_t cap, int32_t* keys, int64_t* n) 
     keys_impl<double>(c, s, cap, keys, n);
 }
 
-// Queues, for every species s, sum v^2 over its live particles into
-// sums[s]: part holds kEnergyBlocks partials per species (fixed-order sums,
-// so the result is the same from run to run).
+// sum v^2 of every species and the squared edge fields, with the partials in
+// `part` ((S + 1) * kEnergyBlocks doubles; fixed-order sums, so the result is
+// the same from run to run): 1/2 sum_s m_s size_s sum v^2 and the field's energy.
 template <class R>
-static void queue_v2(Ctx& c, double* part, double* sums) {
+static void energy_impl(Ctx& c, double* part, double* out) {
+  EnergyArgs<R> a{};
+  a.ns = c.S;
+  a.ntiles = c.ntiles;
+  a.split = std::max(1, kEnergyBlocks / c.ntiles);
   for (int s = 0; s < c.S; ++s) {
     auto& b = bins<R>(c)[s];
-    double* ps = part + (size_t)s * kEnergyBlocks;
-    if (b.cnt.p && c.ntiles > 0) {
-      k_v2_tiles<R><<<kEnergyBlocks, kBlock, 0, c.stream>>>(ptrs(b.reg), b.start.p, b.cnt.p, c.ntiles, ps);
-      k_sum_serial<<<1, 1, 0, c.stream>>>(ps, kEnergyBlocks, sums + s);
-    } else {
-      k_sum_serial<<<1, 1, 0, c.stream>>>(ps, 0, sums + s);
-    }
+    a.sp[s] = {b.has_invalid ? b.reg.c[0].p : nullptr, b.reg.c[3].p, b.reg.c[4].p, b.reg.c[5].p, b.start.p, b.cnt.p};
   }
+  a.phi = c.phi.p;
+  a.cx = c.cx;
+  a.cy = c.cy;
+  a.cz = c.cz;
+  double* h = static_cast<double*>(c.energy_words.p);
+  k_energy<R><<<dim3(kEnergyBlocks, c.S + 1), kBlock, 0, c.stream>>>(a, part);
+  k_energy_sum<<<c.S + 1, kBlock, 0, c.stream>>>(part, h);
   FOPIS_HIP(hipGetLastError());
-}
-
-// 1/2 sum_s m_s size_s sum v^2 from the per-species sums copied to the host.
-static double kinetic(const Ctx& c, const double* v2) {
-  double res = 0.0;
+  FOPIS_HIP(hipStreamSynchronize(c.stream));
+  out[0] = 0.0;
   for (int s = 0; s < c.S; ++s) {
     const fopis_species_desc& sd = c.d.species[s];
-    res += 0.5 * sd.mass * v2[s] * sd.size;
+    out[0] += 0.5 * sd.mass * h[s] * sd.size;
   }
-  return res;
+  out[1] = 0.5 * c.d.eps0 * h[c.S];
 }
 
-void particles_energy_queue(Ctx& c, double* part, double* sums) {
+static void energy_with(Ctx& c, double* part, double* out) {
   if (c.fp32)
-    queue_v2<float>(c, part, sums);
+    energy_impl<float>(c, part, out);
   else
-    queue_v2<double>(c, part, sums);
+    energy_impl<double>(c, part, out);
 }
 
-double particles_energy_from(const Ctx& c, const double* v2) { return kinetic(c, v2); }
-
-double particles_energy(Ctx& c) {
-  const size_t np = (size_t)c.S * kEnergyBlocks;
-  c.red.alloc(std::max<size_t>(c.red.n, np + c.S));
-  particles_energy_queue(c, c.red.p, c.red.p + np);
-  std::vector<double> v2(c.S);
-  FOPIS_HIP(hipMemcpyAsync(v2.data(), c.red.p + np, c.S * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-  FOPIS_HIP(hipStreamSynchronize(c.stream));
-  return kinetic(c, v2.data());
+void energy(Ctx& c, double* out) {
+  c.red.alloc(std::max<size_t>(c.red.n, (size_t)(c.S + 1) * kEnergyBlocks));
+  energy_with(c, c.red.p, out);
 }
 
 template <class R>
@@ -2678,11 +2743,11 @@ void particles_moments(Ctx& c, int s, double* out) {
 //
 // fopis_energy_noalloc keeps its partial sums in this file-scope array instead
 // of library-allocated memory: kEnergyBlocks partials per species and for the
-// field, then the S + 1 sums. Every call overwrites all of them (nothing has to
+// field (the sums go to the context's pinned words). Every call overwrites all of them (nothing has to
 // start at zero). Each device holds its own copy for the life of the process;
 // host code reaches it only through the address hipGetSymbolAddress returns
 // for the current device, never through the array's name.
-constexpr size_t kNoAllocDoubles = (size_t)(FOPIS_MAX_SPECIES + 1) * kEnergyBlocks + FOPIS_MAX_SPECIES + 1;
+constexpr size_t kNoAllocDoubles = (size_t)(FOPIS_MAX_SPECIES + 1) * kEnergyBlocks;
 static __device__ __align__(256) double noalloc_scratch[kNoAllocDoubles];
 
 namespace {
@@ -2708,20 +2773,11 @@ void noalloc_setup(Ctx& c) {
 
 void energy_noalloc(Ctx& c, double* out) {
   if (!c.noalloc) throw Error(FOPIS_E_STATE, "scratch array not set up for this context");
-  const size_t need = (size_t)(c.S + 1) * kEnergyBlocks + c.S + 1;
+  const size_t need = (size_t)(c.S + 1) * kEnergyBlocks;
   if (c.S < 0 || c.S > FOPIS_MAX_SPECIES || need > kNoAllocDoubles)
     throw Error(FOPIS_E_ARG, "energy partials of " + std::to_string(c.S) + " species exceed the scratch array (" +
                                  std::to_string(FOPIS_MAX_SPECIES) + " species at most)");
-  double* part = c.noalloc;
-  double* fpart = part + (size_t)c.S * kEnergyBlocks;
-  double* sums = fpart + kEnergyBlocks;
-  particles_energy_queue(c, part, sums);
-  fields_energy_queue(c, fpart, sums + c.S);
-  double h[FOPIS_MAX_SPECIES + 1];
-  FOPIS_HIP(hipMemcpyAsync(h, sums, (size_t)(c.S + 1) * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-  FOPIS_HIP(hipStreamSynchronize(c.stream));
-  out[0] = particles_energy_from(c, h);
-  out[1] = 0.5 * c.d.eps0 * h[c.S];
+  energy_with(c, c.noalloc, out);
 }
 
 }  // namespace fopis

@@ -205,7 +205,7 @@ int fopis_energy(fopis_ctx* ctx, double* out);
  * reference. For callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc). The
  * partial sums live in a fixed array of the library, one per device, of
- * (FOPIS_MAX_SPECIES + 1) * 1024 + FOPIS_MAX_SPECIES + 1 doubles (74 KB),
+ * (FOPIS_MAX_SPECIES + 1) * 1024 doubles (74 KB),
  * held until the process ends; a context with more species than that is
  * refused. The result equals fopis_energy's bit for bit (same kernels, same
  * summation order). Every call on a device shares that device's array:
