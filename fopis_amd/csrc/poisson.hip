@@ -1584,6 +1584,9 @@ P* vcycle(Ctx& c, int l, const int* done, const P* from = nullptr) {
   return E_<P>(m);
 }
 
+// A whole solve is captured up to this many expected cycles (about 600 kernel nodes).
+constexpr int kWholeMost = 32;
+
 template <class P>
 int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const double* rho0) {
   MgLevel& m0 = c.mg[0];
@@ -1615,8 +1618,10 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
     k_resid0<P><<<nb, 256, 0, c.stream>>>(phi, rho, rc, store ? r0 : (P*)nullptr, L0, part, flag,
                                           store ? r64 : (double*)nullptr);
   };
-  resid0(true, never);
-  k_norm<true><<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, max_cycles, 0, nullptr);
+  auto begin = [&] {
+    resid0(true, never);
+    k_norm<true><<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, max_cycles, 0, nullptr);
+  };
   // Queue as many cycles as the previous two solves needed, then more. With
   // pairs, two V-cycles share one FP64 update and norm check: the second
   // runs on the same right-hand side, continuing from the first's correction
@@ -1640,10 +1645,12 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
   const dim3 face_grid(div_up(std::max(c.cy, c.cz) - 2, 64), std::max(c.cx, c.cy) - 2, 6);
   int* skip = st + 4;
   // One cycle (or pair): the V-cycle(s), the FP64 update and the norm
-  // check. Their ~30 (~60) launches are captured once into a graph of kernel
+  // check. Their ~15 (~30) launches are captured once into a graph of kernel
   // nodes (every pointer and size in them is fixed for the context; the
   // tolerance and the cycle cap are arguments of the norm kernel, so the
-  // graphs are rebuilt when they change) and replayed.
+  // graphs are rebuilt when they change) and replayed. From the second solve
+  // in a row that expects the same cycles on, the whole solve is one graph:
+  // the chip idles about 10 us between two graphs.
   auto cycle = [&](int nv) {
     const P* e = vcycle<P>(c, 0, done);
     if (nv == 2) {
@@ -1668,29 +1675,48 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
     }
     k_norm<false><<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, max_cycles, nv, nv == 2 ? skip : nullptr);
   };
-  if (c.mg_use_graph && (!c.mg_graph[0] || c.mg_graph_esz != sizeof(P) || c.mg_graph_tol != tol ||
-                         c.mg_graph_cap != max_cycles)) {
-    for (int k = 0; k < 2; ++k) {
-      if (c.mg_graph[k]) {
-        FOPIS_HIP(hipGraphExecDestroy(c.mg_graph[k]));
-        c.mg_graph[k] = nullptr;
-      }
-      hipGraph_t g = nullptr;
-      FOPIS_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
-      cycle(k + 1);
-      const hipError_t ec = hipStreamEndCapture(c.stream, &g);
-      if (ec != hipSuccess || !g)
-        throw Error(FOPIS_E_DEVICE, std::string("V-cycle capture: ") + hipGetErrorString(ec));
-      const hipError_t ei = hipGraphInstantiate(&c.mg_graph[k], g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      if (ei != hipSuccess) {
-        c.mg_graph[k] = nullptr;
-        throw Error(FOPIS_E_DEVICE, std::string("V-cycle graph: ") + hipGetErrorString(ei));
-      }
+  // once done, the true residual b - A phi confirms the end and the face
+  // conditions follow, all queued before the one wait of the round
+  auto finish = [&] {
+    resid0(false, st + 7);
+    k_norm_final<<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, max_cycles, words);
+    k_faces<<<face_grid, 64, 0, c.stream>>>(c.phi.p, c.cx, c.cy, c.cz, faces, st + 2);
+  };
+  auto capture = [&](hipGraphExec_t& exec, auto body) {
+    if (exec) {
+      FOPIS_HIP(hipGraphExecDestroy(exec));
+      exec = nullptr;
     }
-    c.mg_graph_esz = sizeof(P);
+    hipGraph_t g = nullptr;
+    FOPIS_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
+    body();
+    const hipError_t ec = hipStreamEndCapture(c.stream, &g);
+    if (ec != hipSuccess || !g)
+      throw Error(FOPIS_E_DEVICE, std::string("V-cycle capture: ") + hipGetErrorString(ec));
+    const hipError_t ei = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    if (ei != hipSuccess) {
+      exec = nullptr;
+      throw Error(FOPIS_E_DEVICE, std::string("V-cycle graph: ") + hipGetErrorString(ei));
+    }
+  };
+  if (c.mg_use_graph && (!c.mg_graph[0] || c.mg_graph_tol != tol || c.mg_graph_cap != max_cycles)) {
+    for (int k = 0; k < 2; ++k) capture(c.mg_graph[k], [&] { cycle(k + 1); });
     c.mg_graph_tol = tol;
     c.mg_graph_cap = max_cycles;
+    c.mg_whole_pred = 0;
+  }
+  bool whole = c.mg_use_graph && rho0 == c.rho.p && pred == c.mg_pred_last && pred <= kWholeMost;
+  c.mg_pred_last = pred;
+  if (whole && c.mg_whole_pred != pred) {
+    c.mg_whole_pred = 0;
+    capture(c.mg_whole, [&] {
+      begin();
+      for (int q = 0; q < npair; ++q) cycle(2);
+      for (int q = 0; q < batch; ++q) cycle(1);
+      finish();
+    });
+    c.mg_whole_pred = pred;
   }
   auto launch = [&](int nv) {
     if (c.mg_use_graph)
@@ -1698,9 +1724,16 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
     else
       cycle(nv);
   };
+  if (!whole) begin();
   for (;;) {
-    for (int q = 0; q < npair; ++q) launch(2);
-    for (int q = 0; q < batch; ++q) launch(1);
+    if (whole) {
+      FOPIS_HIP(hipGraphLaunch(c.mg_whole, c.stream));
+      whole = false;
+    } else {
+      for (int q = 0; q < npair; ++q) launch(2);
+      for (int q = 0; q < batch; ++q) launch(1);
+      finish();
+    }
     if (pairs) {  // later rounds: one pair (up to two cycles) at a time
       npair = 1;
       batch = 0;
@@ -1708,11 +1741,6 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
       npair = 0;
       batch = 2;
     }
-    // once done, the true residual b - A phi confirms the end and the face
-    // conditions follow, all queued before the one wait of the round
-    resid0(false, st + 7);
-    k_norm_final<<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, max_cycles, words);
-    k_faces<<<face_grid, 64, 0, c.stream>>>(c.phi.p, c.cx, c.cy, c.cz, faces, st + 2);
     FOPIS_HIP(hipGetLastError());
     FOPIS_HIP(hipStreamSynchronize(c.stream));
     if (!words->done) continue;
@@ -1838,9 +1866,9 @@ void poisson_init(Ctx& c) {
 }
 
 void poisson_free(Ctx& c) {
-  for (auto& g : c.mg_graph) {
-    if (g) (void)hipGraphExecDestroy(g);
-    g = nullptr;
+  for (hipGraphExec_t* g : {&c.mg_graph[0], &c.mg_graph[1], &c.mg_whole}) {
+    if (*g) (void)hipGraphExecDestroy(*g);
+    *g = nullptr;
   }
 }
 
