@@ -368,7 +368,7 @@ struct Ctx {
   size_t id3(int i, int j, int k) const { return ((size_t)i * cy + j) * cz + k; }
 };
 
-// ---- copies between the caller's pageable arrays and the device (hostcopy.cpp) ----
+// ---- copies between the caller's pageable arrays and the device (hostcopy.hip) ----
 struct HostSeg {
   void* host;
   void* dev;

@@ -27,10 +27,12 @@ def _roundtrip(dims, rounds, seed, out):
 @pytest.mark.parametrize(
     "dims",
     [
-        (128, 64, 127),  # one plane short of 8 MiB: plain
-        (128, 64, 128),  # 8 MiB, whole chunks
+        (64, 64, 127),  # short of 4 MiB: plain both ways
+        (64, 64, 128),  # 4 MiB: chunked on the way out
         (64, 64, 257),  # 8 MiB and 32 KiB: a short last chunk
-        (131, 129, 133),  # odd, more chunks than slots of its threads
+        (128, 128, 192),  # 24 MiB: chunked both ways, whole chunks
+        (131, 129, 193),  # odd
+        (257, 259, 261),  # more chunks than slots
     ],
 )
 @pytest.mark.parametrize("threads", [1, 2])
@@ -42,3 +44,23 @@ def test_field_roundtrip(dims, threads):
     for t in th:
         t.join()
     assert out == [True] * (3 * threads)
+
+
+@pytest.mark.parametrize("n", [700_001, 1_000_002])
+def test_particle_roundtrip(n):
+    """Six components in one copy, each at another address modulo 16 when n is odd."""
+    from fopis_amd import lib as F
+
+    ctx = F.Context(F.make_desc(17, 17, 17, [(-1.0, 1.0, 1.0)], 1.0))
+    try:
+        rng = np.random.default_rng(2)
+        p = {k: rng.uniform(0.0, 16.0, n) for k in ("x", "y", "z")}
+        p.update({k: rng.standard_normal(n) for k in ("vx", "vy", "vz")})
+        ctx.set_particles(0, p)
+        got = ctx.get_particles(0)
+    finally:
+        ctx.close()
+    tile = lambda d: sum((np.minimum(d[k].astype(np.int64), 15) // 8) * f for k, f in (("x", 4), ("y", 2), ("z", 1)))
+    order = np.argsort(tile(p), kind="stable")
+    for k in p:
+        assert np.array_equal(got[k], p[k][order])
