@@ -4,7 +4,7 @@
 // into a fresh array and 17 GB/s into a touched one, one thread moving the
 // bytes between the runtime's staging and the caller's pages (and taking the
 // page faults). Here a few threads each keep two pinned chunks in flight on the
-// stream and move them: 43 GB/s into a fresh array (3.2 ms instead of 13.4), 42
+// stream and move them: 43 GB/s into a fresh array (3.2 ms instead of 13.4), 38
 // GB/s to the device, where the link is the bound. The chunks cross the link by
 // a kernel: hipMemcpyAsync took 3.7 ms in some processes and 12.0 ms in others
 // or at other times of one (11.6 GB/s, whichever engine it was given).
@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <system_error>
 #include <thread>
@@ -25,11 +26,12 @@ namespace fopis {
 namespace {
 
 constexpr size_t kChunk = (size_t)2 << 20;
-// From here on the threads are faster than a plain copy (into a fresh array
-// 4.6 MB: 0.42 ms for 0.48, 12 MB 0.60 for 1.37; to the device 18 MB: 0.64 for
-// 0.52, 35 MB 0.96 for 1.21): they cost 0.2 ms to start.
-constexpr size_t kLeastOut = (size_t)4 << 20, kLeastIn = (size_t)24 << 20;
-constexpr size_t kLeastChunk = (size_t)512 << 10;
+// From here on the threads are faster than a plain copy (2.4 MB out: 0.28 ms for
+// 0.55 into fresh arrays, 0.11 for 0.14 into touched ones; 7.8 MB 0.50 for 0.98
+// and 0.29 for 0.44; in, 18 MB: 0.59 for 0.52, 35 MB 1.10 for 1.21). A small
+// copy takes fewer of them.
+constexpr size_t kLeastOut = (size_t)2 << 20, kLeastIn = (size_t)24 << 20;
+constexpr size_t kLeastChunk = (size_t)128 << 10, kPerThread = (size_t)1280 << 10;
 constexpr int kMostThreads = 8;
 
 // A chunk's place in its slot: where it has its device address modulo 16, so
@@ -38,9 +40,8 @@ constexpr size_t kSlot = kChunk + 64;
 inline char* in_slot(char* slot, const char* dev) { return slot + (reinterpret_cast<uintptr_t>(dev) & 15); }
 
 // The pinned chunks: one block of 32 MB per process, made by the first large
-// copy (a copy with a block of its own took 12 ms), used by one copy at a time
-// (another goes the plain way meanwhile), kept while a context lives and given
-// back with the last one.
+// copy, used by one copy at a time (another goes the plain way meanwhile), kept
+// while a context lives and given back with the last one.
 std::mutex g_mu;
 char* g_pin = nullptr;
 int g_contexts = 0;
@@ -51,7 +52,7 @@ struct Lease {
   Lease() {
     std::lock_guard<std::mutex> lk(g_mu);
     if (g_busy || g_contexts == 0) return;
-    if (!g_pin && hipHostMalloc(reinterpret_cast<void**>(&g_pin), (size_t)kMostThreads * 2 * kSlot,
+    if (!g_pin && hipHostMalloc(reinterpret_cast<void**>(&g_pin), (size_t)kMostThreads * 2 * kSlot + 64,
                                 hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
       g_pin = nullptr;
       (void)hipGetLastError();
@@ -75,9 +76,15 @@ struct Lease {
 
 // `bytes` bytes between device memory and a pinned slot, both at the same
 // address modulo 16: the ends byte by byte, the rest in 16-byte pieces, a
-// wavefront's 1 KB apart.
+// wavefront's 1 KB apart. 64 workgroups: 128 took 3.4 ms out and 4.6 in for 139
+// MB, 64 3.2 and 3.7.
+// A launch first tells the host that the chunks before its own have landed.
 constexpr int kMoveBlocks = 64;
-__global__ __launch_bounds__(256) void k_move(char* __restrict__ to, const char* __restrict__ from, uint32_t bytes) {
+__global__ __launch_bounds__(256) void k_move(char* __restrict__ to, const char* __restrict__ from, uint32_t bytes,
+                                              uint32_t* landed, uint32_t chunk) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *reinterpret_cast<volatile uint32_t*>(landed) = chunk;
+  }
   const uint32_t head = min((uint32_t)(-reinterpret_cast<uintptr_t>(from) & 15u), bytes);
   const uint32_t n16 = (bytes - head) / 16, tail = head + 16 * n16;
   const uint4* f = reinterpret_cast<const uint4*>(from + head);
@@ -96,7 +103,10 @@ __global__ __launch_bounds__(256) void k_move(char* __restrict__ to, const char*
     const uint32_t e = threadIdx.x < 16 ? threadIdx.x : tail + threadIdx.x - 16;
     if (threadIdx.x < 16 ? e < head : e < bytes) to[e] = from[e];
   }
+  __threadfence_system();  // the next launch announces this chunk
 }
+
+__global__ void k_landed(uint32_t* landed, uint32_t chunks) { *reinterpret_cast<volatile uint32_t*>(landed) = chunks; }
 
 struct Chunk {
   char* host;
@@ -104,48 +114,77 @@ struct Chunk {
   size_t bytes;
 };
 
-// One worker: up to two chunks in flight, in the order they are claimed.
-void work(const std::vector<Chunk>& chunks, std::atomic<size_t>& next, std::atomic<int>& err, char* pin, bool to_host,
-          hipStream_t st, int dev) {
-  hipEvent_t ev[2] = {nullptr, nullptr};
-  size_t idx[2] = {0, 0};
-  bool busy[2] = {false, false};
-  auto ok = [&](hipError_t e) {
-    if (e != hipSuccess) {
-      int none = (int)hipSuccess;
-      err.compare_exchange_strong(none, (int)e);
-    }
-    return e == hipSuccess;
-  };
-  bool good = ok(hipSetDevice(dev));
-  for (auto& e : ev) good = good && ok(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  int s = 0;
-  // slot s: finish what it holds, then the next chunk; ends when both are empty
-  while (good) {
-    char* slot = pin + (size_t)s * kSlot;
-    if (busy[s]) {
-      const Chunk& c = chunks[idx[s]];
-      good = ok(hipEventSynchronize(ev[s]));
-      if (good && to_host) std::memcpy(c.host, in_slot(slot, c.dev), c.bytes);
-      busy[s] = false;
-    }
-    const size_t i = good && err.load() == (int)hipSuccess ? next.fetch_add(1) : chunks.size();
-    if (i < chunks.size()) {
+// One copy. The calling thread launches the chunks in order and moves bytes
+// like the other threads, which make no runtime calls (a thread's first ones
+// cost it 0.1 ms; 2.4 MB out took 0.42 ms with them into fresh arrays, 0.28
+// without). Chunk i uses slot i % nslots.
+struct Copy {
+  std::vector<Chunk> chunks;
+  std::unique_ptr<std::atomic<uint8_t>[]> moved;  // by a thread, between the caller's array and the slot
+  std::atomic<size_t> next{0};
+  std::atomic<bool> stop{false};
+  char* pin = nullptr;
+  uint32_t* landed = nullptr;  // chunks whose kernels have ended
+  size_t nslots = 0, launched = 0;
+  bool to_host = false;
+  hipStream_t st = nullptr;
+  hipError_t err = hipSuccess;
+
+  char* slot(size_t i) const { return in_slot(pin + (i % nslots) * kSlot, chunks[i].dev); }
+  size_t ended() const { return __atomic_load_n(landed, __ATOMIC_ACQUIRE); }
+
+  // launches every chunk that may go (the calling thread)
+  void pump() {
+    const size_t n = chunks.size();
+    while (launched < n && !stop.load()) {
+      const size_t i = launched;
+      if (to_host ? i >= nslots && !moved[i - nslots].load(std::memory_order_acquire)
+                  : !moved[i].load(std::memory_order_acquire))
+        return;
       const Chunk& c = chunks[i];
-      idx[s] = i;
-      char* at = in_slot(slot, c.dev);
-      if (!to_host) std::memcpy(at, c.host, c.bytes);
-      k_move<<<kMoveBlocks, 256, 0, st>>>(to_host ? at : c.dev, to_host ? c.dev : at, (uint32_t)c.bytes);
-      good = ok(hipGetLastError()) && ok(hipEventRecord(ev[s], st));
-      busy[s] = true;
-    } else if (!busy[s ^ 1]) {
-      break;
+      k_move<<<kMoveBlocks, 256, 0, st>>>(to_host ? slot(i) : c.dev, to_host ? c.dev : slot(i), (uint32_t)c.bytes,
+                                          landed, (uint32_t)i);
+      if (++launched == n) k_landed<<<1, 1, 0, st>>>(landed, (uint32_t)n);
+      fail(hipGetLastError());
     }
-    s ^= 1;
   }
-  for (auto& e : ev)
-    if (e) (void)hipEventDestroy(e);
-}
+  void fail(hipError_t e) {
+    if (e == hipSuccess) return;
+    if (err == hipSuccess) err = e;
+    stop.store(true);
+  }
+  // waits until ready() (or stop); the calling thread keeps launching meanwhile
+  template <class F>
+  void wait(bool caller, F ready) {
+    for (unsigned k = 1; !ready() && !stop.load(std::memory_order_relaxed); ++k) {
+      if (caller) pump();
+      if (caller && (k & 0xffff) == 0) {
+        const hipError_t e = hipStreamQuery(st);
+        if (e != hipErrorNotReady) fail(e);
+      }
+      if ((k & 0xff) == 0) std::this_thread::yield();
+    }
+  }
+  void work(bool caller, bool moves) {
+    const size_t n = chunks.size();
+    if (caller) pump();
+    for (size_t i; moves && (i = next.fetch_add(1)) < n;) {
+      const Chunk& c = chunks[i];
+      if (to_host) {
+        wait(caller, [&] { return ended() > i; });
+        if (stop.load()) return;
+        std::memcpy(c.host, slot(i), c.bytes);
+      } else {
+        wait(caller, [&] { return i < nslots || ended() > i - nslots; });
+        if (stop.load()) return;
+        std::memcpy(slot(i), c.host, c.bytes);
+      }
+      moved[i].store(1, std::memory_order_release);
+      if (caller) pump();
+    }
+    if (caller) wait(true, [&] { return launched == n; });
+  }
+};
 
 }  // namespace
 
@@ -174,35 +213,38 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
   };
   if (total < (to_host ? kLeastOut : kLeastIn)) return plain();
   const int cpus = std::max(1, (int)std::thread::hardware_concurrency() / 2);
-  // a thread takes two chunks or more where there are enough
-  const size_t chunk = std::min(kChunk, std::max(kLeastChunk, (total / (2 * kMostThreads) + 4095) / 4096 * 4096));
-  const int nt = (int)std::min<size_t>({(size_t)kMostThreads, (size_t)cpus, total / chunk});
+  const int nt = (int)std::min<size_t>({(size_t)kMostThreads, (size_t)cpus, std::max<size_t>(2, total / kPerThread)});
+  const size_t chunk = std::min(kChunk, std::max(kLeastChunk, (total / (3 * (size_t)nt) + 4095) / 4096 * 4096));
   if (nt < 2) return plain();
   Lease pin;
   if (!pin.p) return plain();
-  std::vector<Chunk> chunks;
+  Copy c;
   for (int q = 0; q < nseg; ++q)
     for (size_t at = 0; at < seg[q].bytes; at += chunk)
-      chunks.push_back(Chunk{static_cast<char*>(seg[q].host) + at, static_cast<char*>(seg[q].dev) + at,
-                             std::min(chunk, seg[q].bytes - at)});
-  int dev = 0;
-  FOPIS_HIP(hipGetDevice(&dev));
-  std::atomic<size_t> next{0};
-  std::atomic<int> err{(int)hipSuccess};
+      c.chunks.push_back(Chunk{static_cast<char*>(seg[q].host) + at, static_cast<char*>(seg[q].dev) + at,
+                               std::min(chunk, seg[q].bytes - at)});
+  c.moved.reset(new std::atomic<uint8_t>[c.chunks.size()]);
+  for (size_t i = 0; i < c.chunks.size(); ++i) c.moved[i].store(0);
+  c.pin = pin.p;
+  c.landed = reinterpret_cast<uint32_t*>(pin.p + (size_t)kMostThreads * 2 * kSlot);
+  *c.landed = 0;
+  c.nslots = (size_t)nt * 2;
+  c.to_host = to_host;
+  c.st = st;
   std::vector<std::thread> th;
   th.reserve(nt);
+  if (to_host) c.pump();  // the first chunks are on their way while the threads start
   try {
-    for (int t = 1; t < nt; ++t)
-      th.emplace_back(work, std::cref(chunks), std::ref(next), std::ref(err), pin.p + (size_t)t * 2 * kSlot, to_host, st,
-                      dev);
+    for (int t = to_host ? 1 : 0; t < nt; ++t) th.emplace_back([&c] { c.work(false, true); });
   } catch (const std::system_error&) {
     // fewer threads than asked for: those that started, and this one, take every chunk
   }
-  work(chunks, next, err, pin.p, to_host, st, dev);
+  // (on the way in the caller only launches: no chunk waits while it moves one)
+  c.work(true, to_host || th.empty());
   for (auto& t : th) t.join();
   // (on an error too: nothing may be in flight when the next copy takes the block)
   const hipError_t e = hipStreamSynchronize(st);
-  FOPIS_HIP((hipError_t)err.load());
+  FOPIS_HIP(c.err);
   FOPIS_HIP(e);
 }
 

@@ -27,8 +27,8 @@ def _roundtrip(dims, rounds, seed, out):
 @pytest.mark.parametrize(
     "dims",
     [
-        (64, 64, 127),  # short of 4 MiB: plain both ways
-        (64, 64, 128),  # 4 MiB: chunked on the way out
+        (64, 64, 63),  # short of 2 MiB: plain both ways
+        (64, 64, 64),  # 2 MiB: chunked on the way out
         (64, 64, 257),  # 8 MiB and 32 KiB: a short last chunk
         (128, 128, 192),  # 24 MiB: chunked both ways, whole chunks
         (131, 129, 193),  # odd
