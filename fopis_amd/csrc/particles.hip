@@ -457,9 +457,10 @@ __device__ __forceinline__ unsigned long long fix_weight(double v) {
 // end; otherwise particles are compacted in place (a.dst == a.reg), which
 // needs a block-wide scan with two barriers per iteration so that no slot is
 // written before it has been read.
-template <class R, int MODE, bool DB = false>
-__global__ __launch_bounds__(kBlock) void k_tile(TileSet<R> set) {
+template <class R, int MODE, bool DB = false, int NB = kBlock>
+__global__ __launch_bounds__(NB) void k_tile(TileSet<R> set) {
   const TileArgs<R>& a = set.s[blockIdx.y];
+  static_assert(NB == kBlock || DB, "the in-place ranks are those of kBlock threads");
   using SM = TileSmem<R, MODE>;
   __shared__ __attribute__((aligned(16))) char smem[SM::bytes];
   __shared__ int sh_rank[4 * kWaves];
@@ -500,7 +501,7 @@ __global__ __launch_bounds__(kBlock) void k_tile(TileSet<R> set) {
 
   if constexpr (SM::kE) {
     constexpr int ne = kEW * kEW * kEW;
-    for (int q = threadIdx.x; q < ne; q += kBlock) {
+    for (int q = threadIdx.x; q < ne; q += NB) {
       const int aa = q / (kEW * kEW), bb = (q / kEW) % kEW, cc = q % kEW;
       const int gi = o0 + 1 + aa, gj = o1 + 1 + bb, gk = o2 + 1 + cc;
       R vx = 0, vy = 0, vz = 0;
@@ -517,10 +518,10 @@ __global__ __launch_bounds__(kBlock) void k_tile(TileSet<R> set) {
     }
   }
   if constexpr (SM::kR) {
-    for (int q = threadIdx.x; q < kRW * kRW * kRW; q += kBlock) sR[q] = 0ull;
+    for (int q = threadIdx.x; q < kRW * kRW * kRW; q += NB) sR[q] = 0ull;
   }
   if constexpr (SM::kD) {
-    for (int q = threadIdx.x; q < kDW * kDW * kDW; q += kBlock) sD[q] = 0;
+    for (int q = threadIdx.x; q < kDW * kDW * kDW; q += NB) sD[q] = 0;
   }
   if constexpr ((MODE & M_BIN) != 0) {
     if (threadIdx.x < 2) s_res[threadIdx.x] = 0;
@@ -554,10 +555,10 @@ __global__ __launch_bounds__(kBlock) void k_tile(TileSet<R> set) {
   const int ocap = ((MODE & M_BIN) != 0) ? a.ocapa[t] : 0;
   const int64_t ost = ((MODE & M_BIN) != 0) ? a.ostart[t] : 0;
   const int rcap = a.capa[t];
-  const int64_t sink_at = ((int64_t)t * kBlock + threadIdx.x) & (kSink - 1);
+  const int64_t sink_at = ((int64_t)t * NB + threadIdx.x) & (kSink - 1);
   const uint64_t odir_b = reinterpret_cast<uint64_t>(a.odir), snk_b = reinterpret_cast<uint64_t>(a.sink);
 
-  // PPT particles per thread and iteration (FP32: two chunks of kBlock, whose
+  // PPT particles per thread and iteration (FP32: two chunks of NB, whose
   // loads are in flight together; one block scan ranks both), the next
   // iteration's particles loaded while the current ones are processed
   constexpr int PPT = sizeof(R) == 4 ? 2 : 1;
@@ -592,7 +593,7 @@ __global__ __launch_bounds__(kBlock) void k_tile(TileSet<R> set) {
   };
   R nxt[PPT][6];
 #pragma unroll
-  for (int u = 0; u < PPT; ++u) fetch(u * kBlock + threadIdx.x, nxt[u]);
+  for (int u = 0; u < PPT; ++u) fetch(u * NB + threadIdx.x, nxt[u]);
 
   // one particle through velocity, position, cell, density, capture and
   // deposit; returns whether it is still valid (and in dt the tile it bins
@@ -848,20 +849,20 @@ __global__ __launch_bounds__(kBlock) void k_tile(TileSet<R> set) {
   // the face tiles: all of them run at once at a launch's start, and their
   // wavefronts queued on the one counter.)
   int nlost = 0;
-  for (int c0 = 0; c0 < ntot; c0 += PPT * kBlock) {
+  for (int c0 = 0; c0 < ntot; c0 += PPT * NB) {
     R p[PPT][6];
 #pragma unroll
     for (int u = 0; u < PPT; ++u)
 #pragma unroll
       for (int c = 0; c < 6; ++c) p[u][c] = nxt[u][c];
 #pragma unroll
-    for (int u = 0; u < PPT; ++u) fetch(c0 + (PPT + u) * kBlock + threadIdx.x, nxt[u]);
+    for (int u = 0; u < PPT; ++u) fetch(c0 + (PPT + u) * NB + threadIdx.x, nxt[u]);
     bool valid[PPT], lost[PPT];
     int dt[PPT][3];
 #pragma unroll
     for (int u = 0; u < PPT; ++u) {
       lost[u] = false;
-      valid[u] = work(p[u], c0 + u * kBlock + threadIdx.x, dt[u], lost[u]);
+      valid[u] = work(p[u], c0 + u * NB + threadIdx.x, dt[u], lost[u]);
     }
     if constexpr ((MODE & M_POS) != 0) {
       // particles absorbed at a domain face, counted per wavefront
@@ -988,7 +989,7 @@ __global__ __launch_bounds__(kBlock) void k_tile(TileSet<R> set) {
     } else if constexpr ((MODE & (M_VEL | M_POS)) != 0) {
 #pragma unroll
       for (int u = 0; u < PPT; ++u) {
-        const int idx = c0 + u * kBlock + threadIdx.x;
+        const int idx = c0 + u * NB + threadIdx.x;
         if (idx < ntot && idx < nreg) {
           if (!valid[u]) p[u][0] = (R)NAN;  // invalid until the next re-bin drops it
           // only what the pass changes: 72 bytes of traffic per FP64 particle
@@ -1016,11 +1017,11 @@ __global__ __launch_bounds__(kBlock) void k_tile(TileSet<R> set) {
   if constexpr (SM::kR) {
     double* P = a.rho_part + (size_t)t * (kRW * kRW * kRW);
     const double scale = a.q / (sizeof(R) == 4 ? (double)kFix32 : kFix);  // exact: powers of two
-    for (int q = threadIdx.x; q < kRW * kRW * kRW; q += kBlock) P[q] = (double)(long long)sR[q] * scale;
+    for (int q = threadIdx.x; q < kRW * kRW * kRW; q += NB) P[q] = (double)(long long)sR[q] * scale;
   }
   if constexpr (SM::kD) {
     int32_t* P = a.dens_part + (size_t)t * (kDW * kDW * kDW);
-    for (int q = threadIdx.x; q < kDW * kDW * kDW; q += kBlock) P[q] = sD[q];
+    for (int q = threadIdx.x; q < kDW * kDW * kDW; q += NB) P[q] = sD[q];
   }
 }
 
@@ -2155,11 +2156,20 @@ bool reg2_ready(Ctx& c, int s) {
   return true;
 }
 
+constexpr int kWide = 1024;
+constexpr int64_t kWideMost = 256;  // workgroups, one per CU
+
 // Push (when asked for), deposit and binning, into the second buffer or in place.
 template <class R, int MODE>
 void launch_bin(Ctx& c, const std::vector<char>& dbs) {
   each_set<R>(c, dbs, [&](int s) { return dbs[s] != 0; }, [&](const TileSet<R>& set, int n) {
-    k_tile<R, MODE, true><<<dim3(c.ntiles, n), kBlock, 0, c.stream>>>(set);
+    // A launch of at most one workgroup a CU is a chain of each tile's
+    // particles, NB at a time: 1024 threads then (33^3, 20 ppc, FP64, 64 tiles
+    // and two species: 72 us with 256 threads, 45 with 1024).
+    if ((int64_t)c.ntiles * n <= kWideMost)
+      k_tile<R, MODE, true, kWide><<<dim3(c.ntiles, n), kWide, 0, c.stream>>>(set);
+    else
+      k_tile<R, MODE, true><<<dim3(c.ntiles, n), kBlock, 0, c.stream>>>(set);
   });
   each_set<R>(c, dbs, [&](int s) { return dbs[s] == 0; }, [&](const TileSet<R>& set, int n) {
     k_tile<R, MODE><<<dim3(c.ntiles, n), kBlock, 0, c.stream>>>(set);
