@@ -403,9 +403,9 @@ def main():
     }
     tr = pmc_traffic(args.workload) if not args.precision else None
     if tr:
-        # HBM bytes of one k_tile launch (one species) from the committed rocprofv3 FETCH_SIZE/WRITE_SIZE summary
-        line["roofline"]["traffic"] = tr.get("bytes_per_launch")
-        line["roofline"]["algorithmic_bytes_per_launch"] = bpp * n_avg / h.S
+        # HBM bytes of one k_tile launch (all species; the committed rocprofv3 FETCH_SIZE/WRITE_SIZE summary is of one)
+        line["roofline"]["traffic"] = tr["bytes_per_launch"] * h.S if tr.get("bytes_per_launch") else None
+        line["roofline"]["algorithmic_bytes_per_launch"] = bpp * n_avg
     # the first solve of one more step, for the CPU Poisson baseline: its
     # right-hand side (the deposited charge, before the conductor correction)
     # and its warm start (the previous step's phi)
