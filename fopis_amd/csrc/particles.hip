@@ -2180,8 +2180,7 @@ void launch_bin(Ctx& c, const std::vector<char>& dbs) {
 template <class R>
 uint32_t after_bin(Ctx& c) {
   std::vector<int32_t> stat(kStat * c.S);
-  FOPIS_HIP(hipMemcpyAsync(stat.data(), c.status.p, kStat * c.S * sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
-  FOPIS_HIP(hipStreamSynchronize(c.stream));
+  copy_out(stat.data(), c.status.p, kStat * c.S * sizeof(int32_t), c.stream);
   for (auto& b : bins<R>(c)) b.upload_pending = false;
   for (int s = 0; s < c.S; ++s) {
     if (stat[kStat * s + 1] > 0)
@@ -2401,8 +2400,7 @@ static int64_t count_impl(Ctx& c, int s) {
     n = (int64_t)k;
   } else {
     std::vector<int32_t> cnt(c.ntiles);
-    FOPIS_HIP(hipMemcpyAsync(cnt.data(), b.cnt.p, c.ntiles * sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
-    FOPIS_HIP(hipStreamSynchronize(c.stream));
+    copy_out(cnt.data(), b.cnt.p, c.ntiles * sizeof(int32_t), c.stream);
     for (int v : cnt) n += v;
   }
   return n + (int64_t)b.host_inbox.n + staged_inside(c, b);
@@ -2587,8 +2585,7 @@ void particles_position(Ctx& c) {
     for (int s = 0; s < c.S; ++s) (c.fp32 ? c.sp32[s].has_invalid : c.sp64[s].has_invalid) = true;
   }
   std::vector<int32_t> stat(kStat * c.S);
-  FOPIS_HIP(hipMemcpyAsync(stat.data(), c.status.p, stat.size() * sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
-  FOPIS_HIP(hipStreamSynchronize(c.stream));
+  copy_out(stat.data(), c.status.p, stat.size() * sizeof(int32_t), c.stream);
   for (int s = 0; s < c.S; ++s) {
     if (c.fp32)
       c.sp32[s].absorbed += stat[kStat * s + 4];

@@ -27,6 +27,9 @@ def _roundtrip(dims, rounds, seed, out):
 @pytest.mark.parametrize(
     "dims",
     [
+        (6, 6, 7),  # small: one chunk
+        (16, 16, 32),  # 64 KiB: the largest of those
+        (16, 16, 33),  # plain
         (64, 64, 63),  # short of 2 MiB: plain both ways
         (64, 64, 64),  # 2 MiB: chunked on the way out
         (64, 64, 257),  # 8 MiB and 32 KiB: a short last chunk
@@ -46,7 +49,7 @@ def test_field_roundtrip(dims, threads):
     assert out == [True] * (3 * threads)
 
 
-@pytest.mark.parametrize("n", [700_001, 1_000_002])
+@pytest.mark.parametrize("n", [1, 1_365, 1_366, 700_001, 1_000_002])
 def test_particle_roundtrip(n):
     """Six components in one copy, each at another address modulo 16 when n is odd."""
     from fopis_amd import lib as F
