@@ -79,6 +79,7 @@ struct DBuf {
     if (count == 0) return;
     if (hipMalloc(&p, count * sizeof(T)) != hipSuccess) {
       p = nullptr;
+      (void)hipGetLastError();  // reported here: the next check of a launch is not to find it
       throw Error(FOPIS_E_NOMEM, "device allocation of " + std::to_string(count * sizeof(T)) + " bytes failed");
     }
     n = count;
@@ -142,6 +143,7 @@ struct PinBuf {
     if (p) return;
     if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
       p = nullptr;
+      (void)hipGetLastError();
       throw Error(FOPIS_E_NOMEM, "pinned host allocation failed");
     }
   }
@@ -179,8 +181,10 @@ struct PinSoa {
       if (st) FOPIS_HIP(hipStreamSynchronize(st));
       for (auto& p : c) {
         double* np = nullptr;
-        if (hipHostMalloc(reinterpret_cast<void**>(&np), nc * sizeof(double), hipHostMallocDefault) != hipSuccess)
+        if (hipHostMalloc(reinterpret_cast<void**>(&np), nc * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+          (void)hipGetLastError();
           throw Error(FOPIS_E_NOMEM, "pinned host allocation failed");
+        }
         if (n) std::memcpy(np, p, n * sizeof(double));
         if (p) (void)hipHostFree(p);
         p = np;

@@ -123,6 +123,21 @@ __global__ __launch_bounds__(256) void k_move(char* __restrict__ to, const char*
 
 __global__ void k_landed(uint32_t* landed, uint32_t chunks) { *reinterpret_cast<volatile uint32_t*>(landed) = chunks; }
 
+// The launches' own status: hipGetLastError would also give what an earlier
+// call of this thread left there, its program's or this library's.
+hipError_t launch_move(char* to, const char* from, size_t bytes, uint32_t* landed, size_t chunk, size_t blocks,
+                       hipStream_t st) {
+  uint32_t n = (uint32_t)bytes, k = (uint32_t)chunk;
+  void* a[] = {&to, &from, &n, &landed, &k};
+  return hipLaunchKernel(reinterpret_cast<const void*>(&k_move), dim3((unsigned)blocks), dim3(256), a, 0, st);
+}
+
+hipError_t launch_landed(uint32_t* landed, size_t chunks, hipStream_t st) {
+  uint32_t k = (uint32_t)chunks;
+  void* a[] = {&landed, &k};
+  return hipLaunchKernel(reinterpret_cast<const void*>(&k_landed), dim3(1), dim3(1), a, 0, st);
+}
+
 struct Chunk {
   char* host;
   char* dev;
@@ -157,10 +172,8 @@ struct Copy {
                   : !moved[i].load(std::memory_order_acquire))
         return;
       const Chunk& c = chunks[i];
-      k_move<<<kMoveBlocks, 256, 0, st>>>(to_host ? slot(i) : c.dev, to_host ? c.dev : slot(i), (uint32_t)c.bytes,
-                                          landed, (uint32_t)i);
-      if (++launched == n) k_landed<<<1, 1, 0, st>>>(landed, (uint32_t)n);
-      fail(hipGetLastError());
+      fail(launch_move(to_host ? slot(i) : c.dev, to_host ? c.dev : slot(i), c.bytes, landed, i, kMoveBlocks, st));
+      if (++launched == n) fail(launch_landed(landed, n, st));
     }
   }
   void fail(hipError_t e) {
@@ -176,6 +189,7 @@ struct Copy {
       if (caller && (k & 0xffff) == 0) {
         const hipError_t e = hipStreamQuery(st);
         if (e != hipErrorNotReady) fail(e);
+        if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();  // no error of a later launch
       }
       if ((k & 0xff) == 0) std::this_thread::yield();
     }
@@ -236,10 +250,9 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
       at[q] = in_slot(pin.p + off, dev);
       off += (seg[q].bytes + 31) / 16 * 16;
       if (seg[q].bytes > 0)
-        k_move<<<(unsigned)std::min<size_t>(kMoveBlocks, seg[q].bytes / 4096 + 1), 256, 0, st>>>(
-            at[q], dev, (uint32_t)seg[q].bytes, pin.word(), 0);
+        FOPIS_HIP(launch_move(at[q], dev, seg[q].bytes, pin.word(), 0,
+                              std::min<size_t>(kMoveBlocks, seg[q].bytes / 4096 + 1), st));
     }
-    FOPIS_HIP(hipGetLastError());
     FOPIS_HIP(hipStreamSynchronize(st));
     for (int q = 0; q < nseg; ++q) std::memcpy(seg[q].host, at[q], seg[q].bytes);
     return;

@@ -1,0 +1,83 @@
+"""Error paths of the library's host code, on the CPU in front of a HIP
+runtime without a device (fake_hip/fake_hip.cpp, preloaded into a process of
+its own per case): failed allocations and launches, a stream that reports an
+error, and what a call leaves behind for the next one."""
+
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes as C
+import numpy as np
+from fopis_amd import guess as G
+from fopis_amd import lib as F
+
+ARG, DEVICE, NOMEM = -1, -3, -4
+fake = C.CDLL(None)
+fake.fake_log.restype = C.c_char_p
+
+
+def log(clear=True):
+    lines = fake.fake_log().decode().splitlines()
+    if clear:
+        fake.fake_log_clear()
+    return lines
+
+
+def context(*dims, **kw):
+    return F.Context(F.make_desc(*dims, [(-1.0, 1.0, 1.0)], 1.0, **kw))
+
+
+def refused(f, *a, **kw):
+    try:
+        f(*a, **kw)
+    except F.FopisError as e:
+        return e.code
+    return 0
+"""
+
+
+@pytest.fixture(scope="session")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-w",
+                    os.path.join(HERE, "fake_hip", "fake_hip.cpp"), "-o", so, "-lpthread"], check=True)
+
+    def run(body, env=None):
+        before = os.environ.get("LD_PRELOAD")
+        e = dict(os.environ, LD_PRELOAD=f"{so} {before}" if before else so, PYTHONPATH=ROOT, **(env or {}))
+        r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body)], env=e, cwd=ROOT, capture_output=True,
+                           text=True, timeout=60)
+        assert r.returncode == 0, f"exit {r.returncode}\n{r.stdout}\n{r.stderr}"
+
+    return run
+
+
+def test_reported_failure_is_not_reported_again(fake):
+    """A call that reported a failed allocation, or a program's own failed
+    launch: copies afterwards, small and large, return their bytes. (They
+    returned the earlier error as theirs.)"""
+    fake("""
+    for dims in ((9, 9, 9), (65, 65, 65)):
+        ctx = context(*dims)
+        rho = np.random.default_rng(1).standard_normal(ctx.field_shape(F.RHO))
+        ctx.set_field(F.RHO, rho)
+        fake.fake_fail_malloc(0)
+        assert refused(ctx.get_field, F.EX) == NOMEM
+        assert np.array_equal(ctx.get_field(F.RHO), rho)
+        fake.hipMemcpy(None, None, 8, 0)  # an error the program has not asked for yet
+        assert np.array_equal(ctx.get_field(F.RHO), rho)
+        fake.fake_delay(20)  # longer than the copy asks the stream in between
+        assert np.array_equal(ctx.get_field(F.RHO), rho)
+        fake.fake_delay(0)
+        assert fake.hipGetLastError() in (0, 1)  # the program's, or overwritten by the stream's "not ready"
+        ctx.set_field(F.RHO, rho)
+        ctx.close()
+    """)
