@@ -531,6 +531,12 @@ struct WreduceArgs {
   WreduceLayer l[kWMaxLayers];
   int n;
 };
+// The layers of one backward pass whose partials wait for k_wgrad_reduce; it
+// lives and dies with the pass, so a pass that fails leaves none behind.
+struct WgradQueue {
+  WreduceArgs a{};
+  int blocks = 0;
+};
 constexpr int kWredBlocks = (kWTile + 63) / 64;  // per tile
 
 __global__ __launch_bounds__(256) void k_wgrad_reduce(WreduceArgs A) {
@@ -980,8 +986,6 @@ struct GuessNet {
   DBuf<uint16_t> T0, T1, T2;
   bool train_alloc = false;
   std::vector<DBuf<float>> wpart;  // weight- and bias-gradient partial sums, one buffer per layer
-  WreduceArgs wred{};              // the layers whose partials wait for k_wgrad_reduce
-  int wred_blocks = 0;
   DBuf<double> dpart, scal, loss_acc;
   DBuf<uint8_t> cellmask;  // training-data objects
   DBuf<double> rwarm;      // eps0 (b - A phi) of the warm start at the interior nodes (modes 2 and 3)
@@ -1134,8 +1138,9 @@ void launch_wgrad_t(hipStream_t st, WgradArgs& a, int nchunk) {
 
 // Weight and bias gradient of one layer: the partials now, dw and db when
 // wgrad_flush runs. `slot` names the layer's partial buffer.
-void wgrad(Ctx& c, GuessNet& g, int slot, const int* d, int cin, int cout, bool up, const uint16_t* x,
+void wgrad(Ctx& c, GuessNet& g, WgradQueue& wq, int slot, const int* d, int cin, int cout, bool up, const uint16_t* x,
            const uint16_t* gy, float* dw, float* db) {
+  if (wq.a.n >= kWMaxLayers) throw Error(FOPIS_E_STATE, "more layers than a weight-gradient reduction takes");
   WgradArgs a{};
   a.x = x;
   a.g = gy;
@@ -1172,14 +1177,12 @@ void wgrad(Ctx& c, GuessNet& g, int slot, const int* d, int cin, int cout, bool 
     go(std::true_type{});
   else
     go(std::false_type{});
-  g.wred.l[g.wred.n++] = WreduceLayer{a.part, dw, db, nchunk, cin, cout, a.nco, g.wred_blocks};
-  g.wred_blocks += npairs * kWredBlocks;
+  wq.a.l[wq.a.n++] = WreduceLayer{a.part, dw, db, nchunk, cin, cout, a.nco, wq.blocks};
+  wq.blocks += npairs * kWredBlocks;
 }
 
-void wgrad_flush(Ctx& c, GuessNet& g) {
-  if (g.wred.n > 0) k_wgrad_reduce<<<g.wred_blocks, 256, 0, c.stream>>>(g.wred);
-  g.wred.n = 0;
-  g.wred_blocks = 0;
+void wgrad_flush(Ctx& c, const WgradQueue& wq) {
+  if (wq.a.n > 0) k_wgrad_reduce<<<wq.blocks, 256, 0, c.stream>>>(wq.a);
 }
 
 void alloc_train(GuessNet& g) {
@@ -1266,9 +1269,10 @@ void forward(Ctx& c, GuessNet& g, int epi, bool phi_add = false) {
 // Backward pass from g.gOUT; fills g.grad.
 void backward(Ctx& c, GuessNet& g) {
   hipStream_t st = c.stream;
+  WgradQueue wq;
   auto wg = [&](int li, const uint16_t* x, const uint16_t* gy) {
     GuessLayer& l = g.L[li];
-    wgrad(c, g, li, g.lv[l.lvl], l.cin, l.cout, l.up != 0, x, gy, g.grad.p + l.woff, g.grad.p + l.boff);
+    wgrad(c, g, wq, li, g.lv[l.lvl], l.cin, l.cout, l.up != 0, x, gy, g.grad.p + l.woff, g.grad.p + l.boff);
   };
   // data gradient of layer li at its output grid into dx ([out voxels][cin]),
   // through the ReLU of the layer's input y where that is a layer's output
@@ -1323,7 +1327,7 @@ void backward(Ctx& c, GuessNet& g) {
   wg(E0B, g.A0.p, g.gS0.p);
   dg(E0B, g.gS0.p, g.gA0.p, g.A0.p);
   wg(E0A, g.X0.p, g.gA0.p);
-  wgrad_flush(c, g);
+  wgrad_flush(c, wq);
 }
 
 GuessNet& net(Ctx& c) {
@@ -1837,8 +1841,9 @@ void nn_conv3d_backward(int n0, int n1, int n2, int cin, int cout, int up, const
   Ctx cc;
   cc.stream = ts.s;
   const int dims[3] = {n0, n1, n2};
-  wgrad(cc, tmp, 0, dims, cin, cout, up != 0, dx.p, dg.p, dgw.p, dgb.p);
-  wgrad_flush(cc, tmp);
+  WgradQueue wq;
+  wgrad(cc, tmp, wq, 0, dims, cin, cout, up != 0, dx.p, dg.p, dgw.p, dgb.p);
+  wgrad_flush(cc, wq);
   cc.stream = nullptr;
   if (dx_out) {
     const int nqd = 27 * cout / 8, nqpd = (nqd + 3) / 4 * 4;

@@ -81,3 +81,37 @@ def test_reported_failure_is_not_reported_again(fake):
         ctx.set_field(F.RHO, rho)
         ctx.close()
     """)
+
+
+def test_failed_gradient_leaves_nothing_queued(fake):
+    """An allocation that fails in the middle of a backward pass: the next pass
+    reduces its own 15 layers, as on a fresh network. (The layers queued by the
+    failed pass stayed, and were written past the end of their list.)"""
+    fake("""
+    def net():
+        ctx = context(17, 17, 17)
+        g = G.Guess(ctx)
+        g.dataset_alloc(1)
+        n = G.net_grid(17, 17, 17)
+        g.dataset_set(0, np.zeros(n, np.uint16), np.zeros(n, np.uint8), np.zeros(n, np.uint16))
+        return ctx, g
+
+    ctx, g = net()
+    log()
+    g.grad(0)
+    clean = log()
+    allocs = sum(s.startswith("malloc") for s in clean)
+    launches = [s for s in clean if s.startswith("launch")]
+    reduces = [s for s in launches if "k_wgrad_reduce" in s]
+    assert len(reduces) == 1
+    failed = 0
+    for k in range(allocs - 15, allocs):  # the partial sums of each layer
+        ctx, g = net()
+        fake.fake_fail_malloc(k)
+        assert refused(g.grad, 0) == NOMEM
+        failed += 1
+        log()
+        g.grad(0)
+        assert [s for s in log() if s.startswith("launch")] == launches
+    assert failed == 15
+    """)
