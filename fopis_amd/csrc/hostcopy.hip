@@ -151,7 +151,7 @@ struct Chunk {
 struct Copy {
   std::vector<Chunk> chunks;
   std::unique_ptr<std::atomic<uint8_t>[]> moved;  // by a thread, between the caller's array and the slot
-  std::atomic<size_t> next{0};
+  std::atomic<size_t> next{0}, nmoved{0};
   std::atomic<bool> stop{false};
   char* pin = nullptr;
   uint32_t* landed = nullptr;  // chunks whose kernels have ended
@@ -209,9 +209,11 @@ struct Copy {
         std::memcpy(slot(i), c.host, c.bytes);
       }
       moved[i].store(1, std::memory_order_release);
+      nmoved.fetch_add(1);
       if (caller) pump();
     }
-    if (caller) wait(true, [&] { return launched == n; });
+    // only the calling thread asks the stream for errors: it goes on until no thread waits for a chunk
+    if (caller) wait(true, [&] { return launched == n && nmoved.load() == n; });
   }
 };
 

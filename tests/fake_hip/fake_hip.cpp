@@ -24,6 +24,7 @@ std::map<const void*, void*> symbols;
 std::string log_text;
 int fail_malloc = -1, fail_launch = -1, device = 0, cycles = 5, delay_ms = 0;
 bool broken = false;
+int break_after = -1;
 thread_local hipError_t last = hipSuccess;
 
 struct Config {
@@ -85,6 +86,7 @@ void work() {
 }
 
 void submit(const Op& o) {
+  if (break_after >= 0 && break_after-- == 0) broken = true;
   if (broken) return;
   if (!delay_ms) return o.run();
   std::lock_guard<std::mutex> lk(qmu);
@@ -107,6 +109,7 @@ extern "C" {
 void fake_fail_malloc(int k) { fail_malloc = k; }  // the k-th device allocation from now fails (0: the next)
 void fake_fail_launch(int k) { fail_launch = k; }
 void fake_break_stream(int on) { broken = on != 0; }  // nothing launched runs, waits and queries return an error
+void fake_break_stream_after(int k) { break_after = k; }  // once k more have run
 void fake_delay(int ms) { delay_ms = ms; }
 void fake_cycles(int n) { cycles = n; }
 void fake_set_device(int d) { device = d; }

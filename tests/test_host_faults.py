@@ -115,3 +115,26 @@ def test_failed_gradient_leaves_nothing_queued(fake):
         assert [s for s in log() if s.startswith("launch")] == launches
     assert failed == 15
     """)
+
+
+@pytest.mark.parametrize("out", [True, False])
+def test_copy_ends_when_its_stream_fails(fake, out):
+    """A stream that fails at any chunk of a copy by several threads: the copy
+    returns the error, and the next one works. (The threads still waiting for
+    a chunk were not told once the calling one had moved its own.)"""
+    fake(f"""
+    ctx = context(65, 65, 700)
+    rho = np.random.default_rng(1).standard_normal(ctx.field_shape(F.RHO))
+    ctx.set_field(F.RHO, rho)
+    assert np.array_equal(ctx.get_field(F.RHO), rho)
+    for k in range(30):
+        for again in range(3):
+            log()
+            fake.fake_break_stream_after(k)
+            code = refused(ctx.get_field, F.RHO) if {out} else refused(ctx.set_field, F.RHO, rho)
+            fake.fake_break_stream_after(-1)
+            fake.fake_break_stream(0)
+            n = sum("k_move" in s or "k_landed" in s for s in log())
+            assert code == (DEVICE if k < n else 0), (k, n, code)
+            assert np.array_equal(ctx.get_field(F.RHO), rho)
+    """)
