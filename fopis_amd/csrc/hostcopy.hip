@@ -13,9 +13,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -247,15 +247,19 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
     if (!pin.p) return plain();
     char* at[kSmallSegs];
     size_t off = 0;
+    hipError_t launched = hipSuccess;
     for (int q = 0; q < nseg; ++q) {
       const char* dev = static_cast<const char*>(seg[q].dev);
       at[q] = in_slot(pin.p + off, dev);
       off += (seg[q].bytes + 31) / 16 * 16;
-      if (seg[q].bytes > 0)
-        FOPIS_HIP(launch_move(at[q], dev, seg[q].bytes, pin.word(), 0,
-                              std::min<size_t>(kMoveBlocks, seg[q].bytes / 4096 + 1), st));
+      if (seg[q].bytes > 0 && launched == hipSuccess)
+        launched = launch_move(at[q], dev, seg[q].bytes, pin.word(), 0,
+                               std::min<size_t>(kMoveBlocks, seg[q].bytes / 4096 + 1), st);
     }
-    FOPIS_HIP(hipStreamSynchronize(st));
+    // (on an error too: nothing may be in flight when the next copy takes the block)
+    const hipError_t ended = hipStreamSynchronize(st);
+    FOPIS_HIP(launched);
+    FOPIS_HIP(ended);
     for (int q = 0; q < nseg; ++q) std::memcpy(seg[q].host, at[q], seg[q].bytes);
     return;
   }
@@ -284,8 +288,8 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
   if (to_host) c.pump();  // the first chunks are on their way while the threads start
   try {
     for (int t = to_host ? 1 : 0; t < nt; ++t) th.emplace_back([&c] { c.work(false, true); });
-  } catch (const std::system_error&) {
-    // fewer threads than asked for: those that started, and this one, take every chunk
+  } catch (const std::exception&) {
+    // no thread or no memory for one: those that started, and this one, take every chunk
   }
   // (on the way in the caller only launches: no chunk waits while it moves one)
   c.work(true, to_host || th.empty());

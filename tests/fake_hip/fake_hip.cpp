@@ -3,6 +3,7 @@
 // must not provoke: device memory is host memory, launches are logged and do
 // nothing, except that host copies' kernels move their bytes and a solve's
 // last kernel reports its cycles. fake_* (C linkage) steer it.
+#include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
 
 #include <chrono>
@@ -10,8 +11,10 @@
 #include <cstdlib>
 #include <cstring>
 #include <deque>
+#include <exception>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -22,7 +25,7 @@ std::mutex mu;
 std::map<const void*, std::string> kernels;
 std::map<const void*, void*> symbols;
 std::string log_text;
-int fail_malloc = -1, fail_launch = -1, device = 0, cycles = 5, delay_ms = 0;
+int fail_malloc = -1, fail_launch = -1, fail_thread = -1, device = 0, cycles = 5, delay_ms = 0;
 bool broken = false;
 int break_after = -1;
 thread_local hipError_t last = hipSuccess;
@@ -108,6 +111,11 @@ extern "C" {
 
 void fake_fail_malloc(int k) { fail_malloc = k; }  // the k-th device allocation from now fails (0: the next)
 void fake_fail_launch(int k) { fail_launch = k; }
+void fake_fail_thread(int k) { fail_thread = k; }  // starting the k-th thread from now throws std::bad_alloc
+int fake_pending() {
+  std::lock_guard<std::mutex> lk(qmu);
+  return (int)queue.size();
+}
 void fake_break_stream(int on) { broken = on != 0; }  // nothing launched runs, waits and queries return an error
 void fake_break_stream_after(int k) { break_after = k; }  // once k more have run
 void fake_delay(int ms) { delay_ms = ms; }
@@ -118,6 +126,30 @@ void fake_log_clear() {
   log_text.clear();
 }
 const char* fake_log() { return log_text.c_str(); }
+
+// The library's copy of several arrays, called directly.
+struct Seg {
+  void *host, *dev;
+  size_t bytes;
+};
+int fake_copy(void (*host_copy)(const Seg*, int, bool, hipStream_t), const Seg* s, int n, int out) {
+  try {
+    host_copy(s, n, out != 0, nullptr);
+    return 0;
+  } catch (const std::exception&) {
+    return 1;
+  }
+}
+
+// std::thread's start
+void start_thread(void* self, void* state, void (*depend)()) __asm__(
+    "_ZNSt6thread15_M_start_threadESt10unique_ptrINS_6_StateESt14default_deleteIS1_EEPFvvE");
+void start_thread(void* self, void* state, void (*depend)()) {
+  static const auto real = reinterpret_cast<void (*)(void*, void*, void (*)())>(
+      dlsym(RTLD_NEXT, "_ZNSt6thread15_M_start_threadESt10unique_ptrINS_6_StateESt14default_deleteIS1_EEPFvvE"));
+  if (fail_thread >= 0 && fail_thread-- == 0) throw std::bad_alloc();
+  real(self, state, depend);
+}
 
 void** __hipRegisterFatBinary(const void*) {
   static void* h = nullptr;

@@ -48,7 +48,7 @@ def refused(f, *a, **kw):
 def fake(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-w",
-                    os.path.join(HERE, "fake_hip", "fake_hip.cpp"), "-o", so, "-lpthread"], check=True)
+                    os.path.join(HERE, "fake_hip", "fake_hip.cpp"), "-o", so, "-lpthread", "-ldl"], check=True)
 
     def run(body, env=None):
         before = os.environ.get("LD_PRELOAD")
@@ -137,4 +137,43 @@ def test_copy_ends_when_its_stream_fails(fake, out):
             n = sum("k_move" in s or "k_landed" in s for s in log())
             assert code == (DEVICE if k < n else 0), (k, n, code)
             assert np.array_equal(ctx.get_field(F.RHO), rho)
+    """)
+
+
+@pytest.mark.parametrize("out", [True, False])
+def test_copy_with_fewer_threads(fake, out):
+    """Any of a copy's threads cannot be started for want of memory: the others
+    move its chunks. (The process ended.)"""
+    fake(f"""
+    ctx = context(65, 65, 700)
+    rho = np.random.default_rng(1).standard_normal(ctx.field_shape(F.RHO))
+    for k in range(8):
+        ctx.set_field(F.RHO, 0 * rho)
+        if {out}:
+            ctx.set_field(F.RHO, rho)
+        fake.fake_fail_thread(k)
+        if not {out}:
+            ctx.set_field(F.RHO, rho)
+        assert np.array_equal(ctx.get_field(F.RHO), rho)
+        fake.fake_fail_thread(-1)
+    """)
+
+
+def test_failed_launch_leaves_no_copy_in_flight(fake):
+    """A small copy of six arrays whose k-th launch fails: it returns the error
+    when the ones before have ended, so that nothing writes the pinned block
+    after another copy has taken it."""
+    fake("""
+    ctx = context(9, 9, 9)
+    f = C.cast(getattr(ctx.L, "_ZN5fopis9host_copyEPKNS_7HostSegEibP12ihipStream_t"), C.c_void_p)
+    dev = np.random.default_rng(2).standard_normal((6, 50))
+    host = np.zeros_like(dev)
+    seg = np.array([(h.ctypes.data, d.ctypes.data, d.nbytes) for h, d in zip(host, dev)], np.uint64)
+    fake.fake_delay(20)
+    for k in range(8):
+        fake.fake_fail_launch(k)
+        failed = fake.fake_copy(f, seg.ctypes.data_as(C.c_void_p), 6, 1)
+        fake.fake_fail_launch(-1)
+        assert failed == (k < 6) and fake.fake_pending() == 0
+    assert np.array_equal(host, dev)
     """)
