@@ -233,7 +233,10 @@ void host_copy_release() {
 // Copies every segment and returns when the copies are done.
 void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
   size_t total = 0;
-  for (int q = 0; q < nseg; ++q) total += seg[q].bytes;
+  for (int q = 0; q < nseg; ++q) {
+    if (seg[q].bytes > 0 && (!seg[q].host || !seg[q].dev)) FOPIS_HIP(hipErrorInvalidValue);  // as a plain copy says
+    total += seg[q].bytes;
+  }
   auto plain = [&] {
     for (int q = 0; q < nseg; ++q) {
       if (seg[q].bytes == 0) continue;

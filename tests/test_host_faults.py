@@ -177,3 +177,20 @@ def test_failed_launch_leaves_no_copy_in_flight(fake):
         assert failed == (k < 6) and fake.fake_pending() == 0
     assert np.array_equal(host, dev)
     """)
+
+
+@pytest.mark.parametrize("bytes_", [8, 4096, 1 << 20, 8 << 20, 32 << 20])
+@pytest.mark.parametrize("out", [0, 1])
+def test_null_array_is_refused(fake, bytes_, out):
+    """An array that is not there, alone or behind another one, is an error of
+    the call at every size, as a plain copy's. (Pinned copies wrote to it.)"""
+    fake(f"""
+    ctx = context(9, 9, 9)
+    f = C.cast(getattr(ctx.L, "_ZN5fopis9host_copyEPKNS_7HostSegEibP12ihipStream_t"), C.c_void_p)
+    a, b = np.ones({bytes_}, np.uint8), np.zeros({bytes_}, np.uint8)
+    for rows in ([(0, a)], [(b.ctypes.data, a), (0, a)]):
+        seg = np.array([(h, d.ctypes.data, d.nbytes) for h, d in rows], np.uint64)
+        assert fake.fake_copy(f, seg.ctypes.data_as(C.c_void_p), len(rows), {out}) == 1
+    seg = np.array([(b.ctypes.data, a.ctypes.data, a.nbytes), (0, 0, 0)], np.uint64)  # an empty one may be null
+    assert fake.fake_copy(f, seg.ctypes.data_as(C.c_void_p), 2, {out}) == 0
+    """)
