@@ -43,31 +43,47 @@ constexpr int kSmallSegs = 8;
 constexpr size_t kSlot = kChunk + 64;
 inline char* in_slot(char* slot, const char* dev) { return slot + (reinterpret_cast<uintptr_t>(dev) & 15); }
 
-// The pinned memory: one block of 32 MB and one for small copies per process,
-// each made by the first copy that wants it, used by one copy at a time
-// (another goes the plain way meanwhile), kept while a context lives and given
-// back with the last one. The word behind the chunks is Copy::landed.
+// The pinned memory: one block for large copies and one for small ones per
+// process, each made by the first copy that wants it, used by one copy at a
+// time (another goes the plain way meanwhile), kept while a context lives and
+// given back with the last one. The word behind the chunks is Copy::landed.
+// The large one starts with kFirst bytes, for two threads and copies out of
+// kLeastFirst and more, and becomes 32 MB once the copies have asked for kWorth
+// bytes: pinning and touching 32 MB takes 0.6 to 1.6 ms (1 MB 0.04), which a
+// program that reads one field and closes its context would not get back. Plain
+// 2.6 MB take 160 us, 4.6 MB 285, 7.8 MB 470, 18 MB 1100; through 1 MB 160, 240,
+// 370, 770; through 32 MB 115, 190, 270, 520: some 15 us a MB less than through
+// 1 MB, so 48 MB of copies save about what the large block costs.
+constexpr size_t kFirst = ((size_t)1 << 20) + 64, kLeastFirst = (size_t)4 << 20, kWorth = (size_t)48 << 20;
 struct Block {
-  size_t bytes;
+  size_t first, full, least;  // least: bytes of a copy that the first size serves
   char* p = nullptr;
   bool busy = false;
+  size_t bytes = 0, asked = 0;
 };
 std::mutex g_mu;
-Block g_large{(size_t)kMostThreads * 2 * kSlot + 64};
-Block g_small{kSmall + kSmallSegs * 32 + 64};
+Block g_large{kFirst, (size_t)kMostThreads * 2 * kSlot + 64, kLeastFirst};
+Block g_small{kSmall + kSmallSegs * 32 + 64, kSmall + kSmallSegs * 32 + 64, 0};
 int g_contexts = 0;
 
 struct Lease {
   Block& b;
   char* p = nullptr;
-  explicit Lease(Block& block) : b(block) {
+  Lease(Block& block, size_t total) : b(block) {
     std::lock_guard<std::mutex> lk(g_mu);
     if (b.busy || g_contexts == 0) return;
-    if (!b.p && hipHostMalloc(reinterpret_cast<void**>(&b.p), b.bytes, hipHostMallocPortable | hipHostMallocCoherent) !=
-                    hipSuccess) {
-      b.p = nullptr;
-      (void)hipGetLastError();
-      return;
+    b.asked = std::min(kWorth, b.asked + std::min(kWorth, total));
+    const size_t want = b.asked == kWorth ? b.full : b.first;
+    if (b.bytes < b.full && want < b.full && total < b.least) return;
+    if (b.bytes < want) {
+      drop(b);
+      if (hipHostMalloc(reinterpret_cast<void**>(&b.p), want, hipHostMallocPortable | hipHostMallocCoherent) !=
+          hipSuccess) {
+        b.p = nullptr;
+        (void)hipGetLastError();
+        return;
+      }
+      b.bytes = want;
     }
     b.busy = true;
     p = b.p;
@@ -78,13 +94,19 @@ struct Lease {
     b.busy = false;
     give_back();
   }
-  uint32_t* word() const { return reinterpret_cast<uint32_t*>(p + (b.bytes - 64) / 16 * 16); }
+  size_t room() const { return (b.bytes - 64) / 16 * 16; }
+  uint32_t* word() const { return reinterpret_cast<uint32_t*>(p + room()); }
+  static void drop(Block& q) {
+    if (q.p) (void)hipHostFree(q.p);
+    q.p = nullptr;
+    q.bytes = 0;
+  }
   static void give_back() {  // with g_mu held
     if (g_contexts > 0) return;
     for (Block* q : {&g_large, &g_small})
-      if (q->p && !q->busy) {
-        (void)hipHostFree(q->p);
-        q->p = nullptr;
+      if (!q->busy) {
+        drop(*q);
+        q->asked = 0;
       }
   }
 };
@@ -155,12 +177,12 @@ struct Copy {
   std::atomic<bool> stop{false};
   char* pin = nullptr;
   uint32_t* landed = nullptr;  // chunks whose kernels have ended
-  size_t nslots = 0, launched = 0;
+  size_t nslots = 0, slot_bytes = 0, launched = 0;
   bool to_host = false;
   hipStream_t st = nullptr;
   hipError_t err = hipSuccess;
 
-  char* slot(size_t i) const { return in_slot(pin + (i % nslots) * kSlot, chunks[i].dev); }
+  char* slot(size_t i) const { return in_slot(pin + (i % nslots) * slot_bytes, chunks[i].dev); }
   size_t ended() const { return __atomic_load_n(landed, __ATOMIC_ACQUIRE); }
 
   // launches every chunk that may go (the calling thread)
@@ -246,7 +268,7 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
     FOPIS_HIP(hipStreamSynchronize(st));
   };
   if (to_host && total > 0 && total <= kSmall && nseg <= kSmallSegs) {
-    Lease pin(g_small);
+    Lease pin(g_small, 0);
     if (!pin.p) return plain();
     char* at[kSmallSegs];
     size_t off = 0;
@@ -268,11 +290,17 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
   }
   if (total < (to_host ? kLeastOut : kLeastIn)) return plain();
   const int cpus = std::max(1, (int)std::thread::hardware_concurrency() / 2);
-  const int nt = (int)std::min<size_t>({(size_t)kMostThreads, (size_t)cpus, std::max<size_t>(2, total / kPerThread)});
-  const size_t chunk = std::min(kChunk, std::max(kLeastChunk, (total / (3 * (size_t)nt) + 4095) / 4096 * 4096));
-  if (nt < 2) return plain();
-  Lease pin(g_large);
+  if (cpus < 2) return plain();
+  Lease pin(g_large, total);
   if (!pin.p) return plain();
+  // (the threads wait for this copy alone, not through what the stream still has to do)
+  FOPIS_HIP(hipStreamSynchronize(st));
+  const int nt = pin.b.bytes < pin.b.full ? 2
+                                          : (int)std::min<size_t>({(size_t)kMostThreads, (size_t)cpus,
+                                                                   std::max<size_t>(2, total / kPerThread)});
+  const size_t slot = std::min(kSlot, pin.room() / (2 * (size_t)nt) / 64 * 64);
+  const size_t chunk = std::min((slot - 64) / 4096 * 4096,
+                                std::max(kLeastChunk, (total / (3 * (size_t)nt) + 4095) / 4096 * 4096));
   Copy c;
   for (int q = 0; q < nseg; ++q)
     for (size_t at = 0; at < seg[q].bytes; at += chunk)
@@ -284,6 +312,7 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
   c.landed = pin.word();
   *c.landed = 0;
   c.nslots = (size_t)nt * 2;
+  c.slot_bytes = slot;
   c.to_host = to_host;
   c.st = st;
   std::vector<std::thread> th;

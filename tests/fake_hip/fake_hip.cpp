@@ -54,6 +54,7 @@ struct Op {
   uint32_t bytes = 0;
   uint32_t* landed = nullptr;
   uint32_t chunk = 0;
+  bool last_busy = false;
   char* words = nullptr;  // a solve's: done, confirmed, cycles, updates, pair passes, two residuals
   void run() const {
     if (landed) __atomic_store_n(landed, chunk, __ATOMIC_RELEASE);
@@ -72,7 +73,7 @@ struct Op {
 auto& queue = *new std::deque<Op>;
 auto& cv = *new std::condition_variable;
 auto& qmu = *new std::mutex;
-bool worker = false;
+bool worker = false, busy = false;
 
 void work() {
   std::unique_lock<std::mutex> lk(qmu);
@@ -82,6 +83,7 @@ void work() {
     lk.unlock();
     std::this_thread::sleep_for(std::chrono::milliseconds(delay_ms));
     o.run();
+    if (o.last_busy) busy = false;
     lk.lock();
     queue.pop_front();
     cv.notify_all();
@@ -119,6 +121,12 @@ int fake_pending() {
 void fake_break_stream(int on) { broken = on != 0; }  // nothing launched runs, waits and queries return an error
 void fake_break_stream_after(int k) { break_after = k; }  // once k more have run
 void fake_delay(int ms) { delay_ms = ms; }
+void fake_busy() {  // work of the stream that is not a copy's
+  busy = true;
+  Op o;
+  o.last_busy = true;
+  submit(o);
+}
 void fake_cycles(int n) { cycles = n; }
 void fake_set_device(int d) { device = d; }
 void fake_log_clear() {
@@ -147,6 +155,7 @@ void start_thread(void* self, void* state, void (*depend)()) __asm__(
 void start_thread(void* self, void* state, void (*depend)()) {
   static const auto real = reinterpret_cast<void (*)(void*, void*, void (*)())>(
       dlsym(RTLD_NEXT, "_ZNSt6thread15_M_start_threadESt10unique_ptrINS_6_StateESt14default_deleteIS1_EEPFvvE"));
+  note("thread " + std::string(busy ? "busy" : "idle"));
   if (fail_thread >= 0 && fail_thread-- == 0) throw std::bad_alloc();
   real(self, state, depend);
 }

@@ -67,3 +67,20 @@ def test_particle_roundtrip(n):
     order = np.argsort(tile(p), kind="stable")
     for k in p:
         assert np.array_equal(got[k], p[k][order])
+
+
+def test_field_roundtrip_through_the_large_block():
+    """The sizes of one to eight threads after copies large enough for the
+    whole pinned block, and again once the last context gave it back."""
+    for _ in range(2):
+        out = []
+        _roundtrip((257, 259, 261), 1, 1, out)
+        from fopis_amd import lib as F
+
+        keep = F.Context(F.make_desc(9, 9, 9, [(-1.0, 1.0, 1.0)], 1.0))
+        try:
+            for dims in ((257, 259, 261), (64, 64, 65), (67, 65, 131), (113, 117, 119), (129, 131, 133)):
+                _roundtrip(dims, 3, 5, out)
+        finally:
+            keep.close()
+        assert out == [True] * 16

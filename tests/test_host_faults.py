@@ -65,7 +65,7 @@ def test_reported_failure_is_not_reported_again(fake):
     launch: copies afterwards, small and large, return their bytes. (They
     returned the earlier error as theirs.)"""
     fake("""
-    for dims in ((9, 9, 9), (65, 65, 65)):
+    for dims in ((9, 9, 9), (81, 81, 81)):
         ctx = context(*dims)
         rho = np.random.default_rng(1).standard_normal(ctx.field_shape(F.RHO))
         ctx.set_field(F.RHO, rho)
@@ -101,7 +101,8 @@ def test_failed_gradient_leaves_nothing_queued(fake):
     g.grad(0)
     clean = log()
     allocs = sum(s.startswith("malloc") for s in clean)
-    launches = [s for s in clean if s.startswith("launch")]
+    own = lambda lines: [s for s in lines if s.startswith("launch") and "k_move" not in s and "k_landed" not in s]
+    launches = own(clean)
     reduces = [s for s in launches if "k_wgrad_reduce" in s]
     assert len(reduces) == 1
     failed = 0
@@ -112,7 +113,7 @@ def test_failed_gradient_leaves_nothing_queued(fake):
         failed += 1
         log()
         g.grad(0)
-        assert [s for s in log() if s.startswith("launch")] == launches
+        assert own(log()) == launches
     assert failed == 15
     """)
 
@@ -193,4 +194,44 @@ def test_null_array_is_refused(fake, bytes_, out):
         assert fake.fake_copy(f, seg.ctypes.data_as(C.c_void_p), len(rows), {out}) == 1
     seg = np.array([(b.ctypes.data, a.ctypes.data, a.nbytes), (0, 0, 0)], np.uint64)  # an empty one may be null
     assert fake.fake_copy(f, seg.ctypes.data_as(C.c_void_p), 2, {out}) == 0
+    """)
+
+
+def test_pinned_block_follows_use(fake):
+    """One read of a field pins little; 48 MB of reads pin the large block,
+    once; the last context gives it back. Every way returns the bytes."""
+    fake("""
+    for dims in ((65, 65, 65), (81, 81, 81), (65, 65, 65)):
+        ctx = context(*dims)
+        rho = np.random.default_rng(1).standard_normal(ctx.field_shape(F.RHO))
+        ctx.set_field(F.RHO, rho)
+        log()
+        for k in range(30):
+            assert np.array_equal(ctx.get_field(F.RHO), rho)
+            pins = [int(s.split()[1]) for s in log() if s.startswith("pin")]
+            if k == 48 * 2**20 // rho.nbytes:
+                assert len(pins) == 1 and pins[0] > 2**25
+            else:
+                assert sum(pins) <= (2**20 + 64 if k == 0 and rho.nbytes > 2**22 else 0)
+        ctx.close()
+    for dims in ((30, 257, 255), (97, 97, 97), (257, 129, 65), (257, 129, 225)):
+        ctx = context(*dims)
+        rho = np.random.default_rng(1).standard_normal(ctx.field_shape(F.RHO))
+        ctx.set_field(F.RHO, rho)
+        assert np.array_equal(ctx.get_field(F.RHO), rho)
+        ctx.close()
+    """)
+
+
+def test_threads_start_on_an_idle_stream(fake):
+    """A copy's threads start when the stream has done what came before."""
+    fake("""
+    ctx = context(81, 81, 81)
+    fake.fake_delay(5)
+    for k in range(20):
+        log()
+        fake.fake_busy()
+        ctx.get_field(F.RHO)
+        threads = [s for s in log() if s.startswith("thread")][k == 0:]  # the first one is the fake stream's
+        assert threads and set(threads) == {"thread idle"}
     """)
