@@ -252,6 +252,20 @@ void host_copy_release() {
   Lease::give_back();
 }
 
+// An array that the runtime knows (pinned by the caller, say) is copied
+// directly by a plain copy, faster than through the blocks here: 54 KB out in 9
+// us for 18, 2.6 MB in 54 for 115, 139 MB in 2.4 ms for 3.1.
+bool known(const HostSeg* seg, int nseg) {
+  for (int q = 0; q < nseg; ++q) {
+    hipPointerAttribute_t a{};
+    if (seg[q].bytes == 0) continue;
+    const hipError_t e = hipPointerGetAttributes(&a, seg[q].host);
+    if (e == hipSuccess && a.type != hipMemoryTypeUnregistered) return true;
+    if (e != hipSuccess && hipPeekAtLastError() == e) (void)hipGetLastError();
+  }
+  return false;
+}
+
 // Copies every segment and returns when the copies are done.
 void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
   size_t total = 0;
@@ -268,6 +282,7 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
     FOPIS_HIP(hipStreamSynchronize(st));
   };
   if (to_host && total > 0 && total <= kSmall && nseg <= kSmallSegs) {
+    if (known(seg, nseg)) return plain();
     Lease pin(g_small, 0);
     if (!pin.p) return plain();
     char* at[kSmallSegs];
@@ -290,7 +305,7 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
   }
   if (total < (to_host ? kLeastOut : kLeastIn)) return plain();
   const int cpus = std::max(1, (int)std::thread::hardware_concurrency() / 2);
-  if (cpus < 2) return plain();
+  if (cpus < 2 || known(seg, nseg)) return plain();
   Lease pin(g_large, total);
   if (!pin.p) return plain();
   // (the threads wait for this copy alone, not through what the stream still has to do)

@@ -24,6 +24,7 @@ namespace {
 std::mutex mu;
 std::map<const void*, std::string> kernels;
 std::map<const void*, void*> symbols;
+std::map<char*, size_t> pinned;
 std::string log_text;
 int fail_malloc = -1, fail_launch = -1, fail_thread = -1, device = 0, cycles = 5, delay_ms = 0;
 bool broken = false;
@@ -227,9 +228,23 @@ hipError_t hipFree(void* p) {
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
   note("pin " + std::to_string(n));
   *p = std::calloc(1, n);
+  std::lock_guard<std::mutex> lk(mu);
+  pinned[static_cast<char*>(*p)] = n;
+  return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+  *a = {};
+  std::lock_guard<std::mutex> lk(mu);
+  auto it = pinned.upper_bound(static_cast<char*>(const_cast<void*>(p)));
+  const bool in = it != pinned.begin() && p < (--it)->first + it->second;
+  a->type = in ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
   return hipSuccess;
 }
 hipError_t hipHostFree(void* p) {
+  {
+    std::lock_guard<std::mutex> lk(mu);
+    pinned.erase(static_cast<char*>(p));
+  }
   std::free(p);
   return hipSuccess;
 }

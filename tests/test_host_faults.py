@@ -235,3 +235,22 @@ def test_threads_start_on_an_idle_stream(fake):
         threads = [s for s in log() if s.startswith("thread")][k == 0:]  # the first one is the fake stream's
         assert threads and set(threads) == {"thread idle"}
     """)
+
+
+def test_pinned_array_is_copied_directly(fake):
+    """An array that the caller has pinned goes by one plain copy at every size.
+    (It went through the library's own pinned memory, which takes longer.)"""
+    fake("""
+    ctx = context(9, 9, 9)
+    f = C.cast(getattr(ctx.L, "_ZN5fopis9host_copyEPKNS_7HostSegEibP12ihipStream_t"), C.c_void_p)
+    p = C.c_void_p()
+    fake.hipHostMalloc.argtypes = [C.c_void_p, C.c_size_t, C.c_uint]
+    fake.hipHostMalloc(C.byref(p), 64 << 20, 0)
+    for n in (8, 4096, 3 << 20, 8 << 20, 60 << 20):
+        for out in (0, 1):
+            a = np.ones(n, np.uint8)
+            seg = np.array([(p.value + 64, a.ctypes.data, n)], np.uint64)
+            log()
+            assert fake.fake_copy(f, seg.ctypes.data_as(C.c_void_p), 1, out) == 0
+            assert log() == [f"memcpy {n}"]
+    """)
