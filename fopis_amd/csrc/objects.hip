@@ -771,18 +771,25 @@ __global__ __launch_bounds__(256) void k_bj_update(double* W, int np, int kt, co
   }
 }
 
-// C = B^-1 without exchanging rows; false where that would have happened (C is then undefined).
+// C = B^-1 without exchanging rows; false where that would have happened, or
+// without memory for a third matrix (C is then undefined, B as it was).
 static bool invert_in_order(Ctx& c, const double* B, double* C, int n) {
   hipStream_t st = c.stream;
   const int nt = div_up(n, kBJ), np = nt * kBJ;
   DBuf<double> W, F, V;
   DBuf<BjSteps> steps;
   DBuf<int> bad;
-  W.alloc((size_t)np * np);
-  F.alloc((size_t)kBJ * np);
-  V.alloc((size_t)kBJ * np);
-  steps.alloc(2);
-  bad.alloc(1);
+  if ((int64_t)np * np >= (int64_t)1 << 32) return false;  // more threads than a launch can hold
+  try {
+    W.alloc((size_t)np * np);
+    F.alloc((size_t)kBJ * np);
+    V.alloc((size_t)kBJ * np);
+    steps.alloc(2);
+    bad.alloc(1);
+  } catch (const Error& e) {
+    if (e.code != FOPIS_E_NOMEM) throw;
+    return false;
+  }
   FOPIS_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), st));
   k_bj_load<<<div_up((int64_t)np * np, 256), 256, 0, st>>>(B, n, W.p, np);
   k_bj_diag<<<1, 256, 0, st>>>(W.p, np, 0, steps.p, bad.p);
@@ -829,8 +836,8 @@ void objects_build_cmatrix(Ctx& c, int o) {
     finish_cmatrix(c, ob);
     return;
   }
-  // C = B^-1 by Gauss-Jordan with partial pivoting: B from the per-node solves
-  // (Neumann faces, nodes on a face), or one whose columns do not peak on the diagonal
+  // C = B^-1 by Gauss-Jordan with partial pivoting, in place: B from the per-node solves (Neumann faces, nodes on a
+  // face), one whose columns do not peak on the diagonal, or no room for the blocks
   k_identity<<<div_up((int64_t)n * n, 256), 256, 0, st>>>(ob.C.p, n);
   DBuf<double> f;
   f.alloc(n + 2);

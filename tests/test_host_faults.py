@@ -254,3 +254,30 @@ def test_pinned_array_is_copied_directly(fake):
             assert fake.fake_copy(f, seg.ctypes.data_as(C.c_void_p), 1, out) == 0
             assert log() == [f"memcpy {n}"]
     """)
+
+
+def test_cmatrix_without_room_for_the_blocked_inversion(fake):
+    """Any allocation of the blocked inversion fails: the elimination in place
+    inverts, as it did where only it was there. (The call failed.)"""
+    fake("""
+    def build(k):
+        ctx = context(17, 17, 17)
+        mask = np.zeros((18, 18, 18), np.uint8)
+        mask[8, 8, 8] = 1
+        ctx.set_object(0, mask, np.array([(i, j, 8) for i in range(6, 11) for j in range(6, 11)], np.int32))
+        log()
+        fake.fake_fail_malloc(k)
+        code = refused(ctx.build_cmatrix, 0)
+        fake.fake_fail_malloc(-1)
+        ctx.close()
+        return code, log()
+
+    code, clean = build(-1)
+    assert code == 0 and not any("k_gj_elim" in s for s in clean)
+    n = sum(s.startswith("malloc") for s in clean)
+    for k in range(n - 5, n):  # W, F, V, the steps, the flag
+        code, lines = build(k)
+        assert code == 0 and any("k_gj_elim" in s for s in lines), (k, code)
+        assert not any("k_bj" in s for s in lines)
+    assert build(0)[0] == NOMEM
+    """)
