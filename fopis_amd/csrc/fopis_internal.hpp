@@ -339,8 +339,13 @@ struct Ctx {
   // captured once: [0] one V-cycle + FP64 update + norm check, [1] two
   // V-cycles (the second continuing from the first's correction) + update + check
   hipGraphExec_t mg_graph[2] = {nullptr, nullptr};
-  hipGraphExec_t mg_whole = nullptr;  // a whole solve of mg_whole_pred expected cycles (0: none)
-  int mg_whole_pred = 0, mg_pred_last = 0;
+  size_t mg_graph_nodes[2] = {0, 0};
+  // a whole solve by its expected cycles: its graph once it has been expected often enough
+  struct Whole {
+    hipGraphExec_t exec = nullptr;
+    int seen = 0;
+  };
+  std::vector<Whole> mg_whole;
   double mg_graph_tol = 0.0;  // tolerance and cycle cap captured in their norm kernels
   int mg_graph_cap = 0;
   bool mg_pairs = true;  // a solve's predicted cycles run two per FP64 update

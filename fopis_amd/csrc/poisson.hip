@@ -1584,8 +1584,22 @@ P* vcycle(Ctx& c, int l, const int* done, const P* from = nullptr) {
   return E_<P>(m);
 }
 
-// A whole solve is captured up to this many expected cycles (about 600 kernel nodes).
-constexpr int kWholeMost = 32;
+// A whole solve of some number of expected cycles is captured once that number
+// has been expected kWholeAfter times, if its graph has at most kWholeNodes
+// nodes. The chip then does not idle between the graphs of single cycles and
+// pairs: a solve takes 157 us instead of 178 at 17^3, 230 for 240 at 33^3, 669
+// for 681 at 129^3. Capturing takes 130 us at 17^3, 180 at 33^3, 300 at 129^3, so
+// it pays after 7 to 30 solves. At 101^3, where the coarsest level stays outside
+// the tail and a cycle has over 200 nodes, the one graph is slower, 4.02 ms for
+// 3.87.
+constexpr int kWholeAfter = 32, kWholeMost = 32;
+constexpr size_t kWholeNodes = 600;
+
+void drop_whole(Ctx& c) {
+  for (auto& w : c.mg_whole)
+    if (w.exec) (void)hipGraphExecDestroy(w.exec);
+  c.mg_whole.assign(kWholeMost + 1, Ctx::Whole());
+}
 
 template <class P>
 int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const double* rho0) {
@@ -1648,9 +1662,8 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
   // check. Their ~15 (~30) launches are captured once into a graph of kernel
   // nodes (every pointer and size in them is fixed for the context; the
   // tolerance and the cycle cap are arguments of the norm kernel, so the
-  // graphs are rebuilt when they change) and replayed. From the second solve
-  // in a row that expects the same cycles on, the whole solve is one graph:
-  // the chip idles about 10 us between two graphs.
+  // graphs are rebuilt when they change) and replayed. A number of cycles that
+  // is expected often gets a graph of the whole solve.
   auto cycle = [&](int nv) {
     const P* e = vcycle<P>(c, 0, done);
     if (nv == 2) {
@@ -1682,7 +1695,7 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
     k_norm_final<<<1, 256, 0, c.stream>>>(part, nb, dst, st, tol, max_cycles, words);
     k_faces<<<face_grid, 64, 0, c.stream>>>(c.phi.p, c.cx, c.cy, c.cz, faces, st + 2);
   };
-  auto capture = [&](hipGraphExec_t& exec, auto body) {
+  auto capture = [&](hipGraphExec_t& exec, size_t* nodes, auto body) {
     if (exec) {
       FOPIS_HIP(hipGraphExecDestroy(exec));
       exec = nullptr;
@@ -1693,6 +1706,7 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
     const hipError_t ec = hipStreamEndCapture(c.stream, &g);
     if (ec != hipSuccess || !g)
       throw Error(FOPIS_E_DEVICE, std::string("V-cycle capture: ") + hipGetErrorString(ec));
+    if (nodes) FOPIS_HIP(hipGraphGetNodes(g, nullptr, nodes));
     const hipError_t ei = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     if (ei != hipSuccess) {
@@ -1701,22 +1715,23 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
     }
   };
   if (c.mg_use_graph && (!c.mg_graph[0] || c.mg_graph_tol != tol || c.mg_graph_cap != max_cycles)) {
-    for (int k = 0; k < 2; ++k) capture(c.mg_graph[k], [&] { cycle(k + 1); });
+    for (int k = 0; k < 2; ++k) capture(c.mg_graph[k], &c.mg_graph_nodes[k], [&] { cycle(k + 1); });
     c.mg_graph_tol = tol;
     c.mg_graph_cap = max_cycles;
-    c.mg_whole_pred = 0;
+    drop_whole(c);
   }
-  bool whole = c.mg_use_graph && rho0 == c.rho.p && pred == c.mg_pred_last && pred <= kWholeMost;
-  c.mg_pred_last = pred;
-  if (whole && c.mg_whole_pred != pred) {
-    c.mg_whole_pred = 0;
-    capture(c.mg_whole, [&] {
-      begin();
-      for (int q = 0; q < npair; ++q) cycle(2);
-      for (int q = 0; q < batch; ++q) cycle(1);
-      finish();
-    });
-    c.mg_whole_pred = pred;
+  hipGraphExec_t whole = nullptr;
+  if (c.mg_use_graph && rho0 == c.rho.p && pred <= kWholeMost &&
+      npair * c.mg_graph_nodes[1] + batch * c.mg_graph_nodes[0] <= kWholeNodes) {
+    Ctx::Whole& w = c.mg_whole[pred];
+    if (!w.exec && ++w.seen > kWholeAfter)
+      capture(w.exec, nullptr, [&] {
+        begin();
+        for (int q = 0; q < npair; ++q) cycle(2);
+        for (int q = 0; q < batch; ++q) cycle(1);
+        finish();
+      });
+    whole = w.exec;
   }
   auto launch = [&](int nv) {
     if (c.mg_use_graph)
@@ -1727,8 +1742,8 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
   if (!whole) begin();
   for (;;) {
     if (whole) {
-      FOPIS_HIP(hipGraphLaunch(c.mg_whole, c.stream));
-      whole = false;
+      FOPIS_HIP(hipGraphLaunch(whole, c.stream));
+      whole = nullptr;
     } else {
       for (int q = 0; q < npair; ++q) launch(2);
       for (int q = 0; q < batch; ++q) launch(1);
@@ -1866,10 +1881,11 @@ void poisson_init(Ctx& c) {
 }
 
 void poisson_free(Ctx& c) {
-  for (hipGraphExec_t* g : {&c.mg_graph[0], &c.mg_graph[1], &c.mg_whole}) {
-    if (*g) (void)hipGraphExecDestroy(*g);
-    *g = nullptr;
+  for (auto& g : c.mg_graph) {
+    if (g) (void)hipGraphExecDestroy(g);
+    g = nullptr;
   }
+  drop_whole(c);
 }
 
 int poisson_solve(Ctx& c, double tol, int max_cycles, double* relres, const double* rhs_override) {

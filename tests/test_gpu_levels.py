@@ -48,3 +48,31 @@ def test_levels_match_single_sweeps(monkeypatch, dims, precision):
     assert np.isfinite(phi).all()
     assert got == want
     assert np.array_equal(phi, ref)
+
+
+@pytest.mark.parametrize("dims", [(17, 17, 17), (33, 49, 25), (65, 65, 65)])
+def test_whole_solve_graph_matches_launches(monkeypatch, dims):
+    """Enough solves of alternating charges that a whole solve becomes one
+    graph, replayed between other work, against the solves launch by launch."""
+    rng = np.random.default_rng(4)
+    rhos = None
+    out = []
+    for graph in ("1", "0"):
+        monkeypatch.setenv("FOPIS_MG_GRAPH", graph)
+        ctx = F.Context(F.make_desc(*dims, [(-1.0, 1.0, 1.0)], 1.0, mg_precision=F.FP32))
+        try:
+            if rhos is None:
+                rhos = [rng.standard_normal(ctx.field_shape(F.RHO)) for _ in range(3)]
+            zero = np.zeros(ctx.field_shape(F.PHI))
+            got = []
+            for k in range(60):
+                ctx.set_field(F.RHO, rhos[k % 3])
+                ctx.set_field(F.PHI, zero)
+                got.append((ctx.solve_poisson(), ctx.get_field(F.PHI)))
+                if k % 7 == 0:
+                    ctx.update_efield()
+            out.append(got)
+        finally:
+            ctx.close()
+    for (a, phi), (b, ref) in zip(*out):
+        assert a == b and np.array_equal(phi, ref)
