@@ -4,7 +4,10 @@
 
 #include <cmath>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <string>
+#include <utility>
 
 #include "fopis_internal.hpp"
 
@@ -45,6 +48,19 @@ void timers_collect(Ctx& c) {
     }
     t.pending.clear();
   }
+}
+
+void grant_lds(const void* kernel, size_t bytes) {
+  if (bytes <= 65536) return;
+  static std::mutex mu;
+  static std::map<std::pair<const void*, int>, size_t> granted;
+  int dev = 0;
+  FOPIS_HIP(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lk(mu);
+  size_t& most = granted[{kernel, dev}];
+  if (bytes <= most) return;
+  FOPIS_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+  most = bytes;
 }
 
 static void check_desc(const fopis_desc& d) {

@@ -390,6 +390,10 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st);
 void copy_out(void* host, const void* dev, size_t bytes, hipStream_t st);
 void copy_in(void* dev, const void* host, size_t bytes, hipStream_t st);
 
+// Lets a kernel have `bytes` of dynamic LDS on the current device (64 KB need no
+// grant); never less than an earlier call gave it. Any thread may call it.
+void grant_lds(const void* kernel, size_t bytes);
+
 // ---- entry points implemented in the .hip units ----
 void particles_init(Ctx& c);
 void particles_set(Ctx& c, int s, int64_t n, const double* const* host6);

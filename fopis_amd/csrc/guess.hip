@@ -1039,20 +1039,10 @@ void pack_all(Ctx& c, GuessNet& g) {
   }
 }
 
-// Raises an instance's dynamic LDS limit once.
-template <class K>
-void grant_lds(K* kernel, size_t bytes, size_t& granted) {
-  if (bytes <= granted) return;
-  FOPIS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)bytes));
-  granted = bytes;
-}
-
 template <int CIN, int NT, int EPI>
 void launch_conv_t(hipStream_t st, ConvArgs& a) {
   constexpr size_t lds = conv_lds_bytes(CIN);
-  static size_t granted = 65536;
-  grant_lds(&k_conv<CIN, NT, EPI>, lds, granted);
+  grant_lds(reinterpret_cast<const void*>(&k_conv<CIN, NT, EPI>), lds);
   a.nbrick = div_up(a.n0, kBI) * div_up(a.n1, kBJ) * div_up(a.n2, kBK);
   // a few workgroups per compute unit, as many as its LDS holds, so that one
   // brick's loads and stores overlap another's products
@@ -1130,8 +1120,7 @@ int wgrad_chunks(const WgradArgs& a) {
 template <int PI, int PO, bool UP>
 void launch_wgrad_t(hipStream_t st, WgradArgs& a, int nchunk) {
   using W = WgradShape<PI, PO>;
-  static size_t granted = 65536;
-  grant_lds(&k_wgrad<PI, PO, UP>, W::kLds, granted);
+  grant_lds(reinterpret_cast<const void*>(&k_wgrad<PI, PO, UP>), W::kLds);
   a.nbrick = div_up(a.n0, W::BI) * div_up(a.n1, W::BJ) * div_up(a.n2, 32);
   k_wgrad<PI, PO, UP><<<dim3(nchunk, div_up(a.nci, PI) * div_up(a.nco, PO)), 256, W::kLds, st>>>(a);
 }

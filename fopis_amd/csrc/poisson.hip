@@ -1779,17 +1779,14 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
 template <typename P>
 void plan_levels(Ctx& c) {
   plan_tail(c, sizeof(P));
-  auto grant = [](const void* f, size_t bytes) {
-    if (bytes > 65536) FOPIS_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-  };
   if (c.mg_fused) {
-    grant(reinterpret_cast<const void*>(&k_level_down<P, false>), DownDim<P, false>::kLds);
-    grant(reinterpret_cast<const void*>(&k_level_down<P, true>), DownDim<P, true>::kLds);
-    grant(reinterpret_cast<const void*>(&k_level_up<P>), UpDim<P>::kLds);
+    grant_lds(reinterpret_cast<const void*>(&k_level_down<P, false>), DownDim<P, false>::kLds);
+    grant_lds(reinterpret_cast<const void*>(&k_level_down<P, true>), DownDim<P, true>::kLds);
+    grant_lds(reinterpret_cast<const void*>(&k_level_up<P>), UpDim<P>::kLds);
   }
   if (c.mg_tail < (int)c.mg.size()) {
-    grant(reinterpret_cast<const void*>(&k_coarse_tail<P, false>), c.mg_tail_bytes);
-    grant(reinterpret_cast<const void*>(&k_coarse_tail<P, true>), c.mg_tail_bytes);
+    grant_lds(reinterpret_cast<const void*>(&k_coarse_tail<P, false>), c.mg_tail_bytes);
+    grant_lds(reinterpret_cast<const void*>(&k_coarse_tail<P, true>), c.mg_tail_bytes);
   }
 }
 

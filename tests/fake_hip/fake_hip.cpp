@@ -25,6 +25,7 @@ std::mutex mu;
 std::map<const void*, std::string> kernels;
 std::map<const void*, void*> symbols;
 std::map<char*, size_t> pinned;
+std::map<std::pair<const void*, int>, size_t> granted;  // LDS beyond 64 KB, by kernel and device
 std::string log_text;
 int fail_malloc = -1, fail_launch = -1, fail_thread = -1, device = 0, cycles = 5, delay_ms = 0;
 bool broken = false;
@@ -185,7 +186,11 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
   *st = c.st;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3 g, dim3, void** a, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3 g, dim3, void** a, size_t lds, hipStream_t) {
+  {
+    std::lock_guard<std::mutex> lk(mu);
+    if (lds > 65536 && lds > granted[{f, device}]) return ret(hipErrorInvalidValue);
+  }
   if (fail_launch >= 0 && fail_launch-- == 0) return ret(hipErrorLaunchOutOfResources);
   if ((uint64_t)g.x * g.y * g.z >= ((uint64_t)1 << 32)) return ret(hipErrorInvalidConfiguration);
   const std::string& name = kernels[f];
@@ -288,7 +293,8 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
   return hipSuccess;
 }
 hipError_t hipFuncSetAttribute(const void* f, hipFuncAttribute, int v) {
-  note("attribute " + kernels[f] + " " + std::to_string(v) + " device " + std::to_string(device));
+  std::lock_guard<std::mutex> lk(mu);
+  granted[{f, device}] = (size_t)v;
   return hipSuccess;
 }
 hipError_t hipGetSymbolAddress(void** p, const void* s) {

@@ -312,3 +312,18 @@ def test_whole_solve_graphs_are_made_for_use(fake):
     ctx = context(101, 101, 101)
     assert made(ctx, 100) == [2] + [0] * 99
     """)
+
+
+def test_lds_grants_hold_per_device_and_context(fake):
+    """A kernel's LDS beyond 64 KB is granted on the device it runs on, and a
+    context with a smaller coarse tail takes none from an earlier one."""
+    fake("""
+    x, w = np.zeros((8, 8, 8, 64), np.uint16), np.zeros((27, 64, 64), np.float32)
+    for device in (0, 1):
+        fake.fake_set_device(device)
+        G.conv3d(x, w, np.zeros(64, np.float32))
+        G.conv3d_backward(x, w, x)
+    ctxs = [context(*n, mg_precision=F.FP64) for n in ((17, 17, 17), (13, 13, 13), (11, 11, 11))]
+    for c in ctxs:
+        c.solve_poisson()
+    """)
