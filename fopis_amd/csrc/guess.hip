@@ -382,7 +382,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs A) {
   extern __shared__ __attribute__((aligned(16))) uint16_t ws[];
   uint16_t* xs = ws;
   uint16_t* gs = ws + W::kXElems;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row = lane & 15, grp = lane >> 4;
   const int ngo = (A.nco + PO - 1) / PO;
   const int ci0 = (blockIdx.y / ngo) * PI, co0 = (blockIdx.y % ngo) * PO;  // the group's first tiles
@@ -457,6 +457,13 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs A) {
         bfr[ri][rj] = load8(gs + (r * PO * 16 + po * 16 + row) * kWRow + grp * 8);
         accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ones), bfr[ri][rj], accb, 0, 0, 0);
       }
+    // g is 0 past the grid, but the first voxel and row there meet x inside it
+    // through the lower tap, and 0 times an infinite or NaN x is not 0: those
+    // products are left out (x past the grid is 0 itself)
+    const int li = A.n0 - i0 - si * W::RI, lj = A.n1 - j0 - sj * W::RJ, lk = A.n2 - k0 - grp * 8;
+    u32x4 in;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) in[h] = (2 * h < lk ? 0xffffu : 0u) | (2 * h + 1 < lk ? 0xffff0000u : 0u);
 #pragma unroll
     for (int xi = 0; xi < W::RI + 2; ++xi)
 #pragma unroll
@@ -468,7 +475,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs A) {
         const u32x4 f1 = {__builtin_amdgcn_alignbit(d[1], d[0], 16), __builtin_amdgcn_alignbit(d[2], d[1], 16),
                           __builtin_amdgcn_alignbit(d[3], d[2], 16), __builtin_amdgcn_alignbit(d4, d[3], 16)};
         const u32x4 f2 = {d[1], d[2], d[3], d4};
-        const bf16x8 af[3] = {__builtin_bit_cast(bf16x8, d), __builtin_bit_cast(bf16x8, f1),
+        const bf16x8 af[3] = {__builtin_bit_cast(bf16x8, d & in), __builtin_bit_cast(bf16x8, f1),
                               __builtin_bit_cast(bf16x8, f2)};
 #pragma unroll
         for (int di = 0; di < 3; ++di)
@@ -476,6 +483,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs A) {
           for (int dj = 0; dj < 3; ++dj) {
             const int ri = xi - di, rj = xj - dj;
             if (ri < 0 || ri >= W::RI || rj < 0 || rj >= W::RJ) continue;
+            if ((di == 0 && ri >= li) || (dj == 0 && rj >= lj)) continue;
 #pragma unroll
             for (int dk = 0; dk < 3; ++dk) {
               const int t = (di * 3 + dj) * 3 + dk;

@@ -110,6 +110,29 @@ def test_conv_brick_edges_match_oracle(shape, cin, cout, up):
         _close_bf16(dx, rdx)
 
 
+@pytest.mark.parametrize("shape,up", [((9, 5, 33), False), ((3, 7, 40), False), ((8, 8, 64), False), ((6, 10, 18), True)])
+@pytest.mark.parametrize("cin,cout", [(8, 16), (16, 32), (32, 16), (32, 48)])
+def test_weight_gradient_keeps_infinities_to_their_taps(shape, cin, cout, up):
+    """An infinite input voxel at the grid's upper faces reaches the taps that
+    read it inside the grid, and no other."""
+    rng = np.random.default_rng(17)
+    xs = tuple(s // 2 for s in shape) if up else shape
+    W = np.zeros((27, cin, cout), np.float32)
+    gy = _bf16_input(rng, shape + (cout,))
+    gy[gy & 0x7FFF == 0] = 0x3F80  # (0 times infinity would be a NaN of its own)
+    for axes in ((0,), (1,), (2,), (0, 1), (1, 2), (0, 1, 2)):
+        x = _bf16_input(rng, xs + (cin,))
+        at = tuple(xs[a] - 1 if a in axes else xs[a] // 2 for a in range(3))
+        x[at + (cin // 2,)] = 0x7F80
+        dw, _, _ = GU.conv3d_backward(x, W, gy, up=up, want_dx=False)
+        rW, _, _ = unet.conv3d_backward(GU.from_bf16(x).astype(np.float64), W.astype(np.float64),
+                                        GU.from_bf16(gy).astype(np.float64), up)
+        ok = np.isfinite(rW)
+        assert 0 < (~ok).sum() <= 27 * cout
+        np.testing.assert_array_equal(np.isfinite(dw), ok)
+        np.testing.assert_allclose(dw[ok], rW[ok], rtol=1e-4, atol=1e-4 * np.max(np.abs(rW[ok])))
+
+
 def _desc(n):
     return F.make_desc(n, n, n, [(-1.0, 1.0, 1.0)], eps0=1.0, mg_precision=F.FP64)
 
