@@ -433,6 +433,7 @@ void poisson_free(Ctx& c);
 int poisson_solve(Ctx& c, double tol, int max_cycles, double* relres, const double* rhs_override);
 
 void objects_set(Ctx& c, int o, const uint8_t* mask, int ncmat, const int32_t* ijk, int fixed, double fixed_pot);
+bool objects_invert(Ctx& c, double* B, double* C, int n, bool peaked);
 void objects_build_cmatrix(Ctx& c, int o);
 void objects_set_cmatrix(Ctx& c, int o, const double* C);
 void objects_get_cmatrix(Ctx& c, int o, double* C);

@@ -574,8 +574,8 @@ static bool spectral_unit_responses(Ctx& c, ObjectDev& ob, double* B) {
 // columns instead of twice over per column, by 2 launches instead of 256:
 // 1538 nodes 36 -> 2.1 ms (bound by the serial steps of the diagonal tiles and
 // the tiles beside them), the whole build at 6146 nodes 1.6 s -> 50 ms. Where a
-// step would have exchanged rows (nodes given twice) *bad is set, and the
-// caller runs the pivoted elimination.
+// step would have exchanged rows, or a NaN comes up (nodes given twice leave a
+// zero pivot), *bad is set, and the caller runs the pivoted elimination.
 constexpr int kBJ = 64;
 constexpr int kBJL = 66;  // LDS row length (16-byte rows off the same banks)
 
@@ -805,6 +805,30 @@ static bool invert_in_order(Ctx& c, const double* B, double* C, int n) {
   return h == 0;
 }
 
+// C = B^-1 on the device, B's contents lost; peaked: no row exchange is
+// expected. Returns whether the blocked inversion did it; otherwise Gauss-Jordan
+// with partial pivoting, in place: B from the per-node solves (Neumann faces,
+// nodes on a face), one whose columns do not peak on the diagonal after all, or
+// no room for the blocks.
+bool objects_invert(Ctx& c, double* B, double* C, int n, bool peaked) {
+  if (peaked && invert_in_order(c, B, C, n)) return true;
+  hipStream_t st = c.stream;
+  k_identity<<<div_up((int64_t)n * n, 256), 256, 0, st>>>(C, n);
+  DBuf<double> f;
+  f.alloc(n + 2);
+  DBuf<int> piv;
+  piv.alloc(1);
+  for (int col = 0; col < n; ++col) {
+    k_gj_pivot<<<1, 1024, 0, st>>>(B, n, col, piv.p, f.p + n);
+    k_gj_swap_scale<<<div_up(n, 256), 256, 0, st>>>(B, C, n, col, piv.p, f.p + n);
+    k_gj_getcol<<<div_up(n, 256), 256, 0, st>>>(B, n, col, f.p);
+    k_gj_elim<<<dim3(div_up(n, 256), n), 256, 0, st>>>(B, C, n, col, f.p);
+  }
+  FOPIS_HIP(hipGetLastError());
+  FOPIS_HIP(hipStreamSynchronize(st));
+  return false;
+}
+
 void objects_build_cmatrix(Ctx& c, int o) {
   ObjectDev& ob = c.obj[o];
   const int n = ob.ncmat;
@@ -832,24 +856,7 @@ void objects_build_cmatrix(Ctx& c, int o) {
     // the reference leaves phi and rho cleared after the unit solves (RootGridObject.cpp:83-85)
     k_zero_d<<<div_up(nn, 256), 256, 0, st>>>(c.phi.p, nn);
   }
-  if (peaked && invert_in_order(c, B.p, ob.C.p, n)) {
-    finish_cmatrix(c, ob);
-    return;
-  }
-  // C = B^-1 by Gauss-Jordan with partial pivoting, in place: B from the per-node solves (Neumann faces, nodes on a
-  // face), one whose columns do not peak on the diagonal, or no room for the blocks
-  k_identity<<<div_up((int64_t)n * n, 256), 256, 0, st>>>(ob.C.p, n);
-  DBuf<double> f;
-  f.alloc(n + 2);
-  DBuf<int> piv;
-  piv.alloc(1);
-  for (int col = 0; col < n; ++col) {
-    k_gj_pivot<<<1, 1024, 0, st>>>(B.p, n, col, piv.p, f.p + n);
-    k_gj_swap_scale<<<div_up(n, 256), 256, 0, st>>>(B.p, ob.C.p, n, col, piv.p, f.p + n);
-    k_gj_getcol<<<div_up(n, 256), 256, 0, st>>>(B.p, n, col, f.p);
-    k_gj_elim<<<dim3(div_up(n, 256), n), 256, 0, st>>>(B.p, ob.C.p, n, col, f.p);
-  }
-  FOPIS_HIP(hipGetLastError());
+  objects_invert(c, B.p, ob.C.p, n, peaked);
   finish_cmatrix(c, ob);
 }
 

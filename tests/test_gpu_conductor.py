@@ -2,6 +2,7 @@
 (surface charge, current), the capacitance matrix built by device unit-charge
 solves, the FP64 charge redistribution, and whole steps with injection and a
 floating conductor through the C++ host facade against the oracle."""
+import ctypes
 import json
 import os
 
@@ -121,6 +122,65 @@ def test_cmatrix_tile_edges(n, dup):
         M -= f[:, None] * M[c]
         I -= f[:, None] * I[c]
     assert np.max(np.abs(I - B)) <= 1e-11 * np.max(np.abs(B))
+
+
+def _invert(ctx, B, peaked):
+    """The library's inversion on a matrix of the device's memory: C, and whether the blocks did it."""
+    vp = ctypes.c_void_p
+    f = getattr(ctx.L, "_ZN5fopis14objects_invertERNS_3CtxEPdS2_ib")
+    f.restype, f.argtypes = ctypes.c_bool, [vp, vp, vp, ctypes.c_int, ctypes.c_bool]
+    hip = ctx.L  # (the runtime the library runs on)
+    hip.hipMalloc.argtypes, hip.hipFree.argtypes = [vp, ctypes.c_size_t], [vp]
+    hip.hipMemcpy.argtypes = [vp, vp, ctypes.c_size_t, ctypes.c_int]
+    dev = [vp(), vp()]
+    out = np.empty_like(B)
+    for d in dev:
+        assert hip.hipMalloc(ctypes.byref(d), B.nbytes) == 0
+    assert hip.hipMemcpy(dev[0], B.ctypes.data, B.nbytes, 1) == 0
+    done = f(ctx.h, dev[0], dev[1], len(B), peaked)
+    assert hip.hipMemcpy(out.ctypes.data, dev[1], B.nbytes, 2) == 0
+    for d in dev:
+        hip.hipFree(d)
+    return out, done
+
+
+def _peaked(rng, n):
+    """A positive definite matrix whose columns, and those of every Schur complement, peak on the diagonal."""
+    a = rng.uniform(0.0, 1.0 / n, (n, n))
+    return np.eye(n) + 0.5 * (a + a.T)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 128, 200])
+def test_blocked_inversion_has_the_eliminations_bits(n):
+    ctx = F.Context(F.make_desc(9, 9, 9, [(-1.0, 1.0, 1.0)], 1.0))
+    B = _peaked(np.random.default_rng(n), n)
+    got, done = _invert(ctx, B, True)
+    want, other = _invert(ctx, B, False)
+    assert done and not other
+    np.testing.assert_array_equal(got, want)
+    assert np.max(np.abs(got @ B - np.eye(n))) <= 1e-13 * n  # cond(B) < 4: a few n eps
+
+
+@pytest.mark.parametrize("n,col,row", [
+    (64, 5, 40),     # inside the first diagonal tile, no tile beside it
+    (64, 62, 63),    # its last rows
+    (128, 70, 100),  # inside the second one, which k_bj_update takes through its steps
+    (128, 3, 64),    # the first row of the tile below
+    (200, 10, 199),  # the last row, in a tile filled up with the identity
+    (200, 130, 195),
+])
+def test_inversion_exchanges_rows_where_the_pivot_is_below(n, col, row):
+    """A larger entry below the diagonal, found in the pivot's tile or in a
+    panel: the pivoted elimination takes over, with the inverse of B."""
+    ctx = F.Context(F.make_desc(9, 9, 9, [(-1.0, 1.0, 1.0)], 1.0))
+    B = _peaked(np.random.default_rng(7), n)
+    B[row, col], B[col, col], B[col, row] = 2.0, 0.25, 1.0
+    got, done = _invert(ctx, B, True)
+    want, _ = _invert(ctx, B, False)
+    assert not done
+    np.testing.assert_array_equal(got, want)
+    assert np.linalg.cond(B) < 50
+    assert np.max(np.abs(got - np.linalg.inv(B))) <= 1e-11 * np.max(np.abs(want))
 
 
 @pytest.mark.parametrize("nx", [17, 41])
