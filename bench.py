@@ -245,6 +245,19 @@ def pmc_traffic(workload: str):
     return None
 
 
+# Species one k_tile launch takes (kTileSet in particles.hip).
+TILE_SPECIES = 4
+
+
+def tile_traffic(tr: dict, nspecies: int):
+    """k_tile launches per step, and the HBM bytes of one of them from the
+    committed rocprofv3 FETCH_SIZE/WRITE_SIZE summary, which says how many
+    species its launch held."""
+    launches = -(-nspecies // TILE_SPECIES)
+    b = tr.get("bytes_per_launch")
+    return launches, b * (nspecies / launches) / tr.get("species_per_launch", 1) if b else None
+
+
 def poisson_roofline(desc, ms, cycles, updates=None, pair_passes=0.0):
     """Algorithmic HBM bytes of one Poisson solve over its measured time. Per
     fine-grid unknown: a V(2,2) cycle moves 83 B with FP32 levels (166 B with
@@ -403,9 +416,8 @@ def main():
     }
     tr = pmc_traffic(args.workload) if not args.precision else None
     if tr:
-        # HBM bytes of one k_tile launch (all species; the committed rocprofv3 FETCH_SIZE/WRITE_SIZE summary is of one)
-        line["roofline"]["traffic"] = tr["bytes_per_launch"] * h.S if tr.get("bytes_per_launch") else None
-        line["roofline"]["algorithmic_bytes_per_launch"] = bpp * n_avg
+        launches, line["roofline"]["traffic"] = tile_traffic(tr, h.S)
+        line["roofline"]["algorithmic_bytes_per_launch"] = bpp * n_avg / launches
     # the first solve of one more step, for the CPU Poisson baseline: its
     # right-hand side (the deposited charge, before the conductor correction)
     # and its warm start (the previous step's phi)

@@ -38,3 +38,20 @@ def test_poisson_roofline_bytes():
     r = bench.poisson_roofline(D, 3.0, 4.0, updates=2.0, pair_passes=2.0)
     assert r["algorithmic_bytes_per_solve"] == n * (4 * 83 + 2 * 40 + 2 * 8 + 56)
     assert r["updates_per_solve"] == 2.0 and r["pair_passes_per_solve"] == 2.0
+
+
+def test_tile_traffic_scales_by_species_per_launch():
+    """A launch's bytes follow the species it holds, whatever launch the
+    committed summary measured; the summaries state a launch's own particles."""
+    for species in (1, 2):
+        tr = {"bytes_per_launch": 10.0 * species, "species_per_launch": species}
+        assert bench.tile_traffic(tr, 1) == (1, 10.0)
+        assert bench.tile_traffic(tr, 4) == (1, 40.0)
+        assert bench.tile_traffic(tr, 6) == (2, 30.0)
+    assert bench.tile_traffic({"bytes_per_launch": 10.0}, 2) == (1, 20.0)
+    assert bench.tile_traffic({}, 2) == (1, None)
+    for workload, bytes_per_particle in (("c2", 96), ("c3", 48)):
+        tr = bench.pmc_traffic(workload)
+        alg = tr["algorithmic_bytes_per_launch"]
+        assert abs(alg - bytes_per_particle * tr["particles_per_launch"]) <= bytes_per_particle
+        assert 1.0 < bench.tile_traffic(tr, tr["species_per_launch"])[1] / alg < 1.1
