@@ -90,7 +90,7 @@ struct ConvArgs {
 
 // Output bricks of kBI x kBJ x 16 voxels: the brick's input with a one-voxel
 // halo (kBI+2, kBJ+2, 18) is staged once in LDS, channel rows padded by 8
-// elements so that the 16 lanes of a fragment read hit distinct banks; each
+// elements to spread the 16 lanes of a fragment read over the banks; each
 // of the 4 waves then owns kBI*kBJ/4 rows of 16 voxels (its M tiles) and reads
 // its A fragments from LDS, B fragments (weights) from global memory through
 // the caches.
@@ -126,6 +126,17 @@ __device__ inline uint32_t pack_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
 }
 
+// Waves per SIMD that k_conv's registers leave room for: as many as hold what a
+// thread keeps without scratch memory: the next brick's units (1.9 registers
+// per input channel) and, with one tile, all weights (3.4 per channel). One more than that spills: 64 -> 64 at 16^3 14.9 -> 26.8 us with two,
+// 48 -> 48 at 32^3 23.3 -> 25.9, 32 -> 16 upsampled to 128^3 115 -> 222 with three,
+// 48 -> 32 to 64^3 34 -> 39. One fewer leaves the chip waiting: 32 -> 32 at 64^3
+// takes 37 us with one, 30 with two or three.
+constexpr int conv_waves(int cin, int nt) {
+  if (cin >= 56 || (nt == 1 && cin >= 40)) return 1;
+  return cin >= 48 || nt > 2 || (nt == 1 && cin >= 24) ? 2 : 3;
+}
+
 // NT tiles of 16 output channels per workgroup, tiles blockIdx.y * NT on.
 // The input channel count is a template argument, so that the K loop unrolls
 // and every fragment's LDS address is a lane base plus an immediate: with the
@@ -141,11 +152,14 @@ __device__ inline uint32_t pack_bf16(float a, float b) {
 // neighbouring channels, so that a lane stores (and loads the addend and the
 // gate as) four channels of one voxel, 8 bytes, instead of four times 2 bytes.
 // Bound by LDS reads (one per product with 16 output channels) and the
-// latency of a brick's stage-multiply-store chain. 16 -> 16 channels at 128^3:
-// 115 -> 58 us (2.3 TB/s, 0.5 PFLOP/s), 32 -> 16 upsampled: 222 -> 117 us,
+// latency of a brick's stage-multiply-store chain: at 128^3, 16 -> 16, a compute
+// unit's LDS is busy 60 % of the time (half of it bank conflicts), the vector
+// units 45 %, the matrix cores 25 %, and waves wait 41 % of theirs; at 16^3, 64 ->
+// 64, LDS 21 %, matrix cores 10 %, waves wait 54 %. 16 -> 16 channels at 128^3:
+// 115 -> 58 us (2.3 TB/s, 0.5 PFLOP/s), 32 -> 16 upsampled: 222 -> 113 us,
 // 64 -> 64 at 16^3: 38 -> 15 us.
 template <int CIN, int NT, int EPI>
-__global__ __launch_bounds__(256, CIN >= 56 || (NT == 1 && CIN >= 40) ? 1 : (CIN >= 48 || NT > 2 || (NT == 1 && CIN >= 24) ? 2 : 3)) void k_conv(ConvArgs A) {
+__global__ __launch_bounds__(256, conv_waves(CIN, NT)) void k_conv(ConvArgs A) {
   extern __shared__ __attribute__((aligned(16))) uint16_t xs[];
   constexpr int MT = kRowsPerWave;
   constexpr int CPT = CIN / 8, NQ = 27 * CPT, NS = (NQ + 3) / 4, LS = CIN + 8;
@@ -338,9 +352,11 @@ __global__ __launch_bounds__(256, CIN >= 56 || (NT == 1 && CIN >= 40) ? 1 : (CIN
 // (kSub) and add their sums in LDS. The bias gradient is one more product,
 // with ones. Partials of a launch's workgroups go to `part`, and
 // k_wgrad_reduce adds them in workgroup order.
-// Bound by staging: at 64^3 a workgroup has two bricks of 216 to 432 products
-// per wave. The 15 layers of a 64^3 training pair: 2.29 -> 0.20 ms (with 2-byte
-// gathers, one per voxel, tap and channel), their bias sums 1.00 ms -> none.
+// Bound by the latency of staging: at 64^3 a workgroup has two bricks of 216 to
+// 432 products per wave, waves wait 42 to 63 % of their time, the LDS is busy
+// 29 to 41 % (most of it bank conflicts), the matrix cores 7 to 14 %. The 15
+// layers of a 64^3 training pair: 2.29 -> 0.21 ms (with 2-byte gathers, one per
+// voxel, tap and channel), their bias sums 1.00 ms -> none.
 constexpr int kWTile = 27 * 256 + 16;  // floats of one channel tile's partial: the taps, then the bias gradient
 constexpr int kWRow = 40;              // LDS elements of one channel's row: 34 voxels, padded to spread the banks
 

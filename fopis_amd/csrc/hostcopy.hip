@@ -3,11 +3,12 @@
 // A pageable hipMemcpy of 139 MB (one field at 257^3 nodes) reached 10 GB/s
 // into a fresh array and 17 GB/s into a touched one, one thread moving the
 // bytes between the runtime's staging and the caller's pages (and taking the
-// page faults). Here a few threads each keep two pinned chunks in flight on the
-// stream and move them: 43 GB/s into a fresh array (3.2 ms instead of 13.4), 38
-// GB/s to the device, where the link is the bound. The chunks cross the link by
-// a kernel: hipMemcpyAsync took 3.7 ms in some processes and 12.0 ms in others
-// or at other times of one (11.6 GB/s, whichever engine it was given).
+// page faults). Here the calling thread launches the chunks and a few threads
+// move them to or from the caller's pages, two pinned slots to a thread: 43 GB/s
+// into a fresh array (3.2 ms instead of 13.4), 38 GB/s to the device, where the
+// link is the bound. The chunks cross the link by a kernel: hipMemcpyAsync took
+// 3.7 ms in some processes and 12.0 ms in others or at other times of one (11.6
+// GB/s, whichever engine it was given).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

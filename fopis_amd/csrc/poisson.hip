@@ -1179,8 +1179,8 @@ __device__ inline void tail_up(P* s, const uint16_t* tab, const TailArgs<P>& A, 
   tail_smooth<P, NT, U>(s, tab, F, A.post, A.w1, A.w6);
 }
 
-// The levels of the cubic chain 15 -> 7 -> 3 -> 1 (every grid of 2^k + 1 nodes
-// per axis ends in it), as plan_tail lays them out: with the strides known at
+// The levels of the cubic chain 15 -> 7 -> 3 -> 1 (every cubic grid of 2^k + 1
+// nodes per axis ends in it), as plan_tail lays them out: with the strides known at
 // compile time a point's neighbours are immediates of one address.
 constexpr int tail_plane(int n1, int n2) { return ((n1 + 2) * (n2 + 2) + 1) & ~1; }
 constexpr TailLv cube15_lv(int q) {
@@ -1509,9 +1509,11 @@ dim3 grid_tiles(const MgLevel& m) {
 }
 
 // The level kernels take levels of up to 2^19 unknowns, 1024 tiles, two rounds
-// of the chip: beyond, the halo they recompute (8 times the tile's points are
-// loaded, 4.8 times swept first) costs more than the launches they save (63^3:
-// 19 us in two launches, 40 us in ten; 95 x 79 x 111: 59 and 43 us).
+// of the chip: beyond, the halo they load and sweep again costs more than the
+// launches they save (per point of an 8^3 tile: k_level_down loads 9.6 of r from
+// zero and 13.4 of e and r when it continues, k_level_up 8 of e and r; the first
+// half-sweeps cover 9.6 and 5.4. 63^3: 19 us in two launches, 40 us in ten; 95 x
+// 79 x 111: 59 and 43 us).
 constexpr int64_t kLevelMost = (int64_t)1 << 19;
 bool level_fused(const Ctx& c, const MgLevel& m) {
   return c.mg_fused && (int64_t)m.n[0] * m.n[1] * m.n[2] <= kLevelMost;
