@@ -309,8 +309,6 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
   if (cpus < 2 || known(seg, nseg)) return plain();
   Lease pin(g_large, total);
   if (!pin.p) return plain();
-  // (the threads wait for this copy alone, not through what the stream still has to do)
-  FOPIS_HIP(hipStreamSynchronize(st));
   const int nt = pin.b.bytes < pin.b.full ? 2
                                           : (int)std::min<size_t>({(size_t)kMostThreads, (size_t)cpus,
                                                                    std::max<size_t>(2, total / kPerThread)});
@@ -333,9 +331,17 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
   c.st = st;
   std::vector<std::thread> th;
   th.reserve(nt);
-  if (to_host) c.pump();  // the first chunks are on their way while the threads start
+  // The threads wait for this copy alone, not through what the stream still has
+  // to do: they start on an idle stream, or when the first chunk has come out
+  // (the others follow it while they start).
+  if (to_host) {
+    c.pump();
+    c.wait(true, [&] { return c.ended() > 0; });
+  } else {
+    c.fail(hipStreamSynchronize(st));
+  }
   try {
-    for (int t = to_host ? 1 : 0; t < nt; ++t) th.emplace_back([&c] { c.work(false, true); });
+    for (int t = to_host ? 1 : 0; t < nt && !c.stop.load(); ++t) th.emplace_back([&c] { c.work(false, true); });
   } catch (const std::exception&) {
     // no thread or no memory for one: those that started, and this one, take every chunk
   }
