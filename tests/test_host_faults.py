@@ -327,3 +327,14 @@ def test_lds_grants_hold_per_device_and_context(fake):
     for c in ctxs:
         c.solve_poisson()
     """)
+
+
+def test_initial_weights_of_a_seed(fake):
+    """A new network's weights, drawn on the host, are the same for a seed from build to build."""
+    fake("""
+    import hashlib
+    for seed, want in ((1, "841a4fca852919ddf61027e7cccc90e8"), (7, "1ef2ac797bdd072dc3e99739cc079aba"),
+                       (12345678901, "bac7c9fefc400aedf4aad85c20e5dc22")):
+        p = G.Guess(context(17, 17, 17), seed=seed).get_params()[0]
+        assert hashlib.sha256(p.tobytes()).hexdigest()[:32] == want
+    """)
