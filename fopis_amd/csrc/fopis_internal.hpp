@@ -130,6 +130,9 @@ struct SoaPtr {
   R* c[6];
 };
 
+// The context's pinned words: sums of the energies, then what a solve reports.
+constexpr size_t kEnergyWords = 0, kSolveWords = 128, kWords = 256;
+
 // A fixed piece of pinned host memory that kernels write.
 struct PinBuf {
   void* p = nullptr;
@@ -333,8 +336,7 @@ struct Ctx {
   int psi_step = -1;           // step that formed psi (-1: none)
   bool carry = true;           // warm starts from psi (FOPIS_CARRY=0: the previous phi for both solves)
   DBuf<int32_t> mg_state;     // [8] solve flags and counts on the device
-  PinBuf mg_words;            // what the host reads of them
-  PinBuf energy_words;        // the energy sums, on the host
+  PinBuf host_words;          // kWords bytes that kernels write for the host: the energy sums, then a solve's words
   DBuf<double> mg_part;       // per-block residual partials and the norms of the solve (fixed address)
   // captured once: [0] one V-cycle + FP64 update + norm check, [1] two
   // V-cycles (the second continuing from the first's correction) + update + check
@@ -364,8 +366,8 @@ struct Ctx {
   std::vector<TailPlan> mg_tail_plan;  // its levels
   bool mg_tail15 = false;              // it is the cubic 15 -> 7 -> 3 -> 1 chain
   int mg_tail_elems = 0;               // LDS elements of its arrays
-  DBuf<uint16_t> mg_tail_tab;          // its point lists
-  DBuf<int32_t> mg_tail_idx;           // its first level's points in that level's array
+  DBuf<uint16_t> mg_tail_tab;          // its point lists, and behind them
+  size_t mg_tail_ntab = 0;             // (from here on, 32-bit) its first level's points in that level's array
   size_t lds_max = 65536;     // LDS bytes per workgroup on the device
   GuessNet* guess = nullptr;  // owned; released by guess_free
 

@@ -355,7 +355,7 @@ __global__ __launch_bounds__(256, conv_waves(CIN, NT)) void k_conv(ConvArgs A) {
 // Bound by the latency of staging: at 64^3 a workgroup has two bricks of 216 to
 // 432 products per wave, waves wait 42 to 63 % of their time, the LDS is busy
 // 29 to 41 % (most of it bank conflicts), the matrix cores 7 to 14 %. The 15
-// layers of a 64^3 training pair: 2.29 -> 0.21 ms (with 2-byte gathers, one per
+// layers of a 64^3 training pair: 2.29 -> 0.22 ms (with 2-byte gathers, one per
 // voxel, tap and channel), their bias sums 1.00 ms -> none.
 constexpr int kWTile = 27 * 256 + 16;  // floats of one channel tile's partial: the taps, then the bias gradient
 constexpr int kWRow = 40;              // LDS elements of one channel's row: 34 voxels, padded to spread the banks

@@ -2281,7 +2281,8 @@ void particles_init(Ctx& c) {
   c.status.alloc(kStat * FOPIS_MAX_SPECIES);
   FOPIS_HIP(hipMemsetAsync(c.status.p, 0, c.status.n * sizeof(int32_t), c.stream));
   noalloc_setup(c);
-  c.energy_words.alloc((FOPIS_MAX_SPECIES + 1) * sizeof(double));
+  static_assert((FOPIS_MAX_SPECIES + 1) * sizeof(double) <= kSolveWords, "the energy sums come before the solve's words");
+  c.host_words.alloc(kWords);
   for (int s = 0; s < c.S; ++s) {
     if (c.fp32)
       bin_flat<float>(c, s, c.sp32[s].reg, 0, false);
@@ -2687,7 +2688,7 @@ static void energy_impl(Ctx& c, double* part, double* out) {
   a.cx = c.cx;
   a.cy = c.cy;
   a.cz = c.cz;
-  double* h = static_cast<double*>(c.energy_words.p);
+  double* h = reinterpret_cast<double*>(static_cast<char*>(c.host_words.p) + kEnergyWords);
   k_energy<R><<<dim3(kEnergyBlocks, c.S + 1), kBlock, 0, c.stream>>>(a, part);
   k_energy_sum<<<c.S + 1, kBlock, 0, c.stream>>>(part, h);
   FOPIS_HIP(hipGetLastError());

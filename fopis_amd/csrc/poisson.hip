@@ -17,6 +17,7 @@
 // one single-workgroup kernel per cycle.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <cstdlib>
 #include <type_traits>
 
@@ -1435,10 +1436,11 @@ void plan_tail(Ctx& c, size_t esz) {
   }
   c.mg_tail_elems = (int)(((size_t)off * esz + 15) / 16 * 16 / esz);
   while (tab.size() % 8) tab.push_back(0);
+  c.mg_tail_ntab = tab.size();
+  tab.resize(tab.size() + 2 * gidx.size());
+  std::memcpy(tab.data() + c.mg_tail_ntab, gidx.data(), gidx.size() * sizeof(int32_t));
   c.mg_tail_tab.alloc(tab.size());
-  c.mg_tail_idx.alloc(gidx.size());
   FOPIS_HIP(hipMemcpy(c.mg_tail_tab.p, tab.data(), tab.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
-  FOPIS_HIP(hipMemcpy(c.mg_tail_idx.p, gidx.data(), gidx.size() * sizeof(int32_t), hipMemcpyHostToDevice));
 }
 
 template <class P>
@@ -1452,9 +1454,9 @@ TailArgs<P> tail_args(Ctx& c, const int* done) {
   MgLevel& m0 = c.mg[c.mg_tail];
   A.ge = E_<P>(m0);
   A.gr = R_<P>(m0);
-  A.gidx = c.mg_tail_idx.p;
+  A.gidx = reinterpret_cast<const int32_t*>(c.mg_tail_tab.p + c.mg_tail_ntab);
   A.tab = c.mg_tail_tab.p;
-  A.ntab = (int)c.mg_tail_tab.n;
+  A.ntab = (int)c.mg_tail_ntab;
   A.w1 = (P)(1.0 - c.d.mg_omega);
   A.w6 = (P)(c.d.mg_omega / 6.0);
   A.pre = c.d.mg_pre;
@@ -1654,7 +1656,8 @@ int solve_impl(Ctx& c, double tol, int max_cycles, double* relres_out, const dou
   const bool pairs = c.mg_pairs && c.mg_tail > 0 && (int)c.mg.size() > 1;
   int npair = pairs ? pred / 2 : 0;
   int batch = pred - 2 * npair;
-  SolveWords* const words = reinterpret_cast<SolveWords*>(c.mg_words.p);
+  static_assert(kSolveWords + sizeof(SolveWords) <= kWords, "the context's pinned words hold a solve's");
+  SolveWords* const words = reinterpret_cast<SolveWords*>(static_cast<char*>(c.host_words.p) + kSolveWords);
   FaceKinds faces;
   for (int f = 0; f < 6; ++f) faces.k[f] = c.d.boundary[f];
   // (u runs along z, or y on the z faces; v along y or x)
@@ -1856,7 +1859,6 @@ void poisson_init(Ctx& c) {
     FOPIS_HIP(hipMemsetAsync(c.erb.p, 0, 2 * c.rb_cs * sizeof(float), c.stream));
     FOPIS_HIP(hipMemsetAsync(c.rrb.p, 0, 2 * c.rb_cs * sizeof(float), c.stream));
   }
-  c.mg_words.alloc(sizeof(SolveWords));
   c.mg_state.alloc(8);
   FOPIS_HIP(hipMemsetAsync(c.mg_state.p, 0, 8 * sizeof(int32_t), c.stream));
   c.mg_part.alloc(2 * kResidBlocks + 4);
