@@ -186,7 +186,7 @@ int fopis_solve_poisson(fopis_ctx* ctx, int32_t* cycles, double* relres);
 /* RootGrid::updateEfield + updateReferenceEfield (RootGridField.cpp:456-582). */
 int fopis_update_efield(fopis_ctx* ctx);
 /* RootGrid::mainLoopES (RootGrid.cpp:82-143) on the device, fused: one
- * kernel per species pushes, moves, absorbs, counts, deposits and re-bins;
+ * kernel (four species a launch) pushes, moves, absorbs, counts, deposits and re-bins;
  * then rho reduction, conductor correction, Poisson and E. Particles staged
  * by fopis_add_particles join this step's deposit. */
 int fopis_main_loop_es(fopis_ctx* ctx);

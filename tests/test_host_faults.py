@@ -54,7 +54,7 @@ def fake(tmp_path_factory):
         before = os.environ.get("LD_PRELOAD")
         e = dict(os.environ, LD_PRELOAD=f"{so} {before}" if before else so, PYTHONPATH=ROOT, **(env or {}))
         r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body)], env=e, cwd=ROOT, capture_output=True,
-                           text=True, timeout=60)
+                           text=True, timeout=240)
         assert r.returncode == 0, f"exit {r.returncode}\n{r.stdout}\n{r.stderr}"
 
     return run
