@@ -48,8 +48,8 @@ inline char* in_slot(char* slot, const char* dev) { return slot + (reinterpret_c
 // process, each made by the first copy that wants it, used by one copy at a
 // time (another goes the plain way meanwhile), kept while a context lives and
 // given back with the last one. The word behind the chunks is Copy::landed.
-// The large one starts with kFirst bytes, for two threads and copies out of
-// kLeastFirst and more, and becomes 32 MB once the copies have asked for kWorth
+// The large one starts with kFirst bytes, for copies out of kLeastFirst and more
+// by two threads, and becomes 32 MB once the copies have asked for kWorth
 // bytes: pinning and touching 32 MB takes 0.6 to 1.6 ms (1 MB 0.04), which a
 // program that reads one field and closes its context would not get back. Plain
 // 2.6 MB take 160 us, 4.6 MB 285, 7.8 MB 470, 18 MB 1100; through 1 MB 160, 240,
@@ -57,25 +57,26 @@ inline char* in_slot(char* slot, const char* dev) { return slot + (reinterpret_c
 // 1 MB, so 48 MB of copies save about what the large block costs.
 constexpr size_t kFirst = ((size_t)1 << 20) + 64, kLeastFirst = (size_t)4 << 20, kWorth = (size_t)48 << 20;
 struct Block {
-  size_t first, full, least;  // least: bytes of a copy that the first size serves
+  size_t first, full;
   char* p = nullptr;
   bool busy = false;
   size_t bytes = 0, asked = 0;
 };
 std::mutex g_mu;
-Block g_large{kFirst, (size_t)kMostThreads * 2 * kSlot + 64, kLeastFirst};
-Block g_small{kSmall + kSmallSegs * 32 + 64, kSmall + kSmallSegs * 32 + 64, 0};
+Block g_large{kFirst, (size_t)kMostThreads * 2 * kSlot + 64};
+Block g_small{kSmall + kSmallSegs * 32 + 64, kSmall + kSmallSegs * 32 + 64};
 int g_contexts = 0;
 
 struct Lease {
   Block& b;
   char* p = nullptr;
-  Lease(Block& block, size_t total) : b(block) {
+  // a copy of `total` bytes, for which the first size will do or not
+  Lease(Block& block, size_t total, bool first_serves) : b(block) {
     std::lock_guard<std::mutex> lk(g_mu);
     if (b.busy || g_contexts == 0) return;
     b.asked = std::min(kWorth, b.asked + std::min(kWorth, total));
     const size_t want = b.asked == kWorth ? b.full : b.first;
-    if (b.bytes < b.full && want < b.full && total < b.least) return;
+    if (b.bytes < b.full && want < b.full && !first_serves) return;
     if (b.bytes < want) {
       drop(b);
       if (hipHostMalloc(reinterpret_cast<void**>(&b.p), want, hipHostMallocPortable | hipHostMallocCoherent) !=
@@ -284,7 +285,7 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
   };
   if (to_host && total > 0 && total <= kSmall && nseg <= kSmallSegs) {
     if (known(seg, nseg)) return plain();
-    Lease pin(g_small, 0);
+    Lease pin(g_small, 0, true);
     if (!pin.p) return plain();
     char* at[kSmallSegs];
     size_t off = 0;
@@ -307,7 +308,7 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
   if (total < (to_host ? kLeastOut : kLeastIn)) return plain();
   const int cpus = std::max(1, (int)std::thread::hardware_concurrency() / 2);
   if (cpus < 2 || known(seg, nseg)) return plain();
-  Lease pin(g_large, total);
+  Lease pin(g_large, total, to_host && total >= kLeastFirst);
   if (!pin.p) return plain();
   const int nt = pin.b.bytes < pin.b.full ? 2
                                           : (int)std::min<size_t>({(size_t)kMostThreads, (size_t)cpus,

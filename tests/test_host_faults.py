@@ -214,6 +214,15 @@ def test_pinned_block_follows_use(fake):
             else:
                 assert sum(pins) <= (2**20 + 64 if k == 0 and rho.nbytes > 2**22 else 0)
         ctx.close()
+    ctx = context(129, 129, 193)
+    rho = np.zeros(ctx.field_shape(F.RHO))
+    log()
+    for k in range(3):  # 26 MB in: plain, then through the large block
+        ctx.set_field(F.RHO, rho)
+        lines = log()
+        assert any("k_move" in s for s in lines) == (k > 0)
+        assert sum(s.startswith("pin") for s in lines) == (k == 1)
+    ctx.close()
     for dims in ((30, 257, 255), (97, 97, 97), (257, 129, 65), (257, 129, 225)):
         ctx = context(*dims)
         rho = np.random.default_rng(1).standard_normal(ctx.field_shape(F.RHO))
