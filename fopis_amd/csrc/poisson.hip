@@ -1593,10 +1593,10 @@ P* vcycle(Ctx& c, int l, const int* done, const P* from = nullptr) {
 // nodes. The chip then does not idle between the graphs of single cycles and
 // pairs: a solve takes 157 us instead of 178 at 17^3, 230 for 240 at 33^3, 669
 // for 681 at 129^3. Capturing takes 130 us at 17^3, 180 at 33^3, 300 at 129^3, so
-// it pays after 7 to 30 solves. At 101^3, where the coarsest level stays outside
+// it pays after 7 to 30 solves (0.55 ms at 257^3, after 45). At 101^3, where the coarsest level stays outside
 // the tail and a cycle has over 200 nodes, the one graph is slower, 4.02 ms for
 // 3.87.
-constexpr int kWholeAfter = 32, kWholeMost = 32;
+constexpr int kWholeAfter = 16, kWholeMost = 32;
 constexpr size_t kWholeNodes = 600;
 
 void drop_whole(Ctx& c) {
