@@ -388,6 +388,7 @@ struct HostSeg {
 // a context keeps the pinned block of large copies alive
 void host_copy_retain();
 void host_copy_release();
+int quota_cpus(const char* root);
 void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st);
 void copy_out(void* host, const void* dev, size_t bytes, hipStream_t st);
 void copy_in(void* dev, const void* host, size_t bytes, hipStream_t st);

@@ -15,8 +15,11 @@
 #include <atomic>
 #include <cstring>
 #include <exception>
+#include <fstream>
+#include <limits>
 #include <memory>
 #include <mutex>
+#include <string>
 #include <thread>
 #include <vector>
 
@@ -243,6 +246,19 @@ struct Copy {
 
 }  // namespace
 
+// The CPUs that a control group's quota amounts to, rounded down but at least
+// one, from the files under `root` (version 2, then 1); without a quota the most.
+int quota_cpus(const char* root) {
+  double quota = 0.0, period = 0.0;
+  std::ifstream v2(std::string(root) + "/cpu.max");
+  if (!(v2 >> quota >> period)) {  // ("max" is no number)
+    std::ifstream q(std::string(root) + "/cpu/cpu.cfs_quota_us"), p(std::string(root) + "/cpu/cpu.cfs_period_us");
+    if (!(q >> quota) || !(p >> period)) quota = 0.0;  // (-1 is none)
+  }
+  if (!(quota > 0.0 && period > 0.0)) return std::numeric_limits<int>::max();
+  return std::max(1, (int)std::min(quota / period, 65536.0));
+}
+
 void host_copy_retain() {
   std::lock_guard<std::mutex> lk(g_mu);
   ++g_contexts;
@@ -306,7 +322,7 @@ void host_copy(const HostSeg* seg, int nseg, bool to_host, hipStream_t st) {
     return;
   }
   if (total < (to_host ? kLeastOut : kLeastIn)) return plain();
-  const int cpus = std::max(1, (int)std::thread::hardware_concurrency() / 2);
+  static const int cpus = std::min((int)std::thread::hardware_concurrency(), quota_cpus("/sys/fs/cgroup")) / 2;
   if (cpus < 2 || known(seg, nseg)) return plain();
   Lease pin(g_large, total, to_host && total >= kLeastFirst);
   if (!pin.p) return plain();

@@ -348,3 +348,25 @@ def test_initial_weights_of_a_seed(fake):
         p = G.Guess(context(17, 17, 17), seed=seed).get_params()[0]
         assert hashlib.sha256(p.tobytes()).hexdigest()[:32] == want
     """)
+
+
+def test_copy_threads_follow_the_cpu_quota(fake, tmp_path):
+    """A control group's quota bounds a copy's threads, which spin while they
+    wait: with fewer CPUs than threads they would be throttled. (Only the
+    affinity set did.)"""
+    cases = [("max 100000", None, 2**31 - 1), ("200000 100000", None, 2), ("150000 100000", None, 1), ("50000 100000", None, 1),
+             ("1600000 100000", None, 16), (None, ("-1", "100000"), 2**31 - 1), (None, ("400000", "100000"), 4),
+             (None, None, 2**31 - 1)]
+    for k, (v2, v1, _) in enumerate(cases):
+        d = tmp_path / str(k)
+        (d / "cpu").mkdir(parents=True)
+        if v2:
+            (d / "cpu.max").write_text(v2 + "\n")
+        if v1:
+            (d / "cpu" / "cpu.cfs_quota_us").write_text(v1[0] + "\n")
+            (d / "cpu" / "cpu.cfs_period_us").write_text(v1[1] + "\n")
+    fake(f"""
+    f = getattr(F.load(), "_ZN5fopis10quota_cpusEPKc")
+    f.argtypes = [C.c_char_p]
+    assert [f(b"{tmp_path}/%d" % k) for k in range({len(cases)})] == {[c[2] for c in cases]}
+    """)
